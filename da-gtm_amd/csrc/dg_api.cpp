@@ -120,11 +120,12 @@ int alloc_kstate(dg_ctx *c) {
     if ((rc = dalloc(c, &c->FI, (size_t)K * M1)) || (rc = dalloc(c, &c->Y64, (size_t)K * ld)) ||
         (rc = dalloc(c, &c->yy, K)) || (rc = dalloc(c, &c->G, K)) || (rc = dalloc(c, &c->Gm, K)) ||
         (rc = dalloc(c, &c->RT, (size_t)K * D)) ||
-        (rc = dalloc(c, &c->partRT, (size_t)c->NC * K * D)) ||
-        (rc = dalloc(c, &c->partG, (size_t)c->NC * K)) ||
+        (rc = dalloc(c, &c->partRT, std::max((size_t)c->NC * K * D, dg_pass1_part(N)))) ||
+        (rc = dalloc(c, &c->partG, (size_t)c->NC * K + (size_t)3 * dg_pass1_wgs(N))) ||
         (rc = dalloc(c, &c->partAB, std::max((size_t)c->nchAB * ((size_t)M1 * M1 + (size_t)M1 * D),
                                              (size_t)(K + 63) / 64))))
         return rc;
+    c->partLog64 = c->partG + (size_t)c->NC * K;
     DG_HIP(c, hipMemsetAsync(c->Y64, 0, (size_t)K * ld * sizeof(double), c->stream));
     DG_HIP(c, hipMemsetAsync(c->Gm, 0, (size_t)K * sizeof(double), c->stream));
     return DG_OK;

@@ -1,324 +1,552 @@
 // FP64 E-step of DA-GTM on gfx950: two streaming passes over the K x N
 // distance matrix, which is never stored.
 //
-// Pass 1 (k_e1_f64): one workgroup per 64-point tile walks all centres in
-// 64-centre tiles.  Each thread keeps an online log-sum-exp state for 4
-// points over its 4-centre slice of every tile; the 16 slices are merged in
-// LDS at the end.  Output per point: x_max, log S2 (pass-2 normaliser),
-// log g and log h.
+// Both passes take their cross term y.t from v_mfma_f64_16x16x4_f64: the FP64
+// matrix and vector rates of this chip are the same (and the two share one
+// pipe), but a matrix instruction needs one operand pair from LDS per 2048
+// flops, where a 4 x 4 register tile of FMAs needs eight per 32.  An FP64 MFMA
+// rounds like a chain of FMAs in the order of its inner index (measured: no
+// bit differs), so every sum over d or n below is one FMA chain in ascending
+// order, whatever the tiling; the results do not depend on it.
+//
+// Pass 1 (k_e1_f64): an online log-sum-exp per point, in sixteen
+// slices: slice t holds the centres k = t (mod 16) in ascending order, its
+// running maximum moving at most once per 64 centres.  The slices are merged
+// in order at the end.  Output per point: x_max, log S2 (pass-2 normaliser),
+// log g and log h, and their sums per workgroup.
 //
 // Pass 2 (k_e2_f64): one workgroup per (64-centre tile, N chunk) recomputes
-// the same distances, forms R = exp((x - x_max)/temp - log S2) in LDS and
-// accumulates G = sum_n R and RT = sum_n R t_n in registers, writing one
-// partial per chunk; k_reduce_parts sums the chunks in a fixed order.
+// the same distances, forms R = exp((x - x_max)/temp - log S2) in registers
+// and accumulates G = sum_n R and RT = sum_n R t_n, writing one partial per
+// chunk; k_reduce_parts sums the chunks in a fixed order.
 //
 // The math restates mpicomm.c:316-414 (resp) and mpicomm.c:463-500 (qual):
 // x = d * (-beta/2), E = exp(x), P = E^(1/temp), R = P / colsum(P), with
 // exp underflow (x < -745.13) giving exactly 0 and an all-zero column
 // falling back to R = 1/K (h = K; g = K in EM mode only).
+#include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "dg_internal.h"
 
 namespace {
 
-constexpr int NT = 256;   // threads per workgroup (4 waves of 64)
-constexpr int TP = 64;    // points per tile
-constexpr int TK = 64;    // centres per tile
-constexpr int DC = 16;    // d-chunk of the cross-term loop
+typedef double d2 __attribute__((ext_vector_type(2)));
+typedef double d4 __attribute__((ext_vector_type(4)));
 
-// S[dd][r] = X[(r0 + r) * ld + d0 + dd], zero for rows >= rows.
-__device__ __forceinline__ void stage_chunk(double (*S)[TP + 1], const double *__restrict__ X,
-                                            long rows, long r0, int ld, int d0, int tid) {
-#pragma unroll
-    for (int e = tid; e < TP * DC; e += NT) {
-        const int r = e / DC, dd = e % DC;
-        const long row = r0 + r;
-        S[dd][r] = (row < rows) ? X[row * ld + d0 + dd] : 0.0;
-    }
+constexpr int NT = 256;   // threads per workgroup (4 waves of 64)
+constexpr int TP = 64;    // points: a pass-2 chunk is a whole number of these
+constexpr int DC = 16;    // d-chunk of the cross-term loop
+constexpr int DCP = DC + 2;  // its row stride in LDS: 8 rows cover the banks once
+
+// D[i][j] += sum_q A[i][q] B[q][j], 16 x 16 x 4: lane l holds A[l % 16][l / 16],
+// B[l / 16][l % 16] and, in element r, D[4 r + l / 16][l % 16].
+__device__ __forceinline__ d4 mfma64(double a, double b, d4 c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
-// acc[i][j] += sum over the chunk of Ts[.][tx + 16 i] * Ys[.][ty + 16 j]
-__device__ __forceinline__ void cross_chunk(double acc[4][4], const double (*Ts)[TP + 1],
-                                            const double (*Ys)[TK + 1], int tx, int ty) {
-#pragma unroll
-    for (int dd = 0; dd < DC; ++dd) {
-        double a[4], b[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) a[i] = Ts[dd][tx + 16 * i];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) b[j] = Ys[dd][ty + 16 * j];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc[i][j] = fma(a[i], b[j], acc[i][j]);
-    }
+// Rows in LDS keep every eight d in the order 0 4 1 5 2 6 3 7, so that a lane
+// finds its elements of two successive MFMAs (d and d + 4) in one 16-byte read.
+__device__ __forceinline__ constexpr int dpos(int d) {
+    return (d & ~7) + 2 * (d & 3) + ((d >> 2) & 1);
+}
+__device__ __forceinline__ void put_pair(double *row, int d, d2 v) {   // d even: d and d + 1
+    row[dpos(d)] = v.x;
+    row[dpos(d) + 2] = v.y;
 }
 
 // Exponent x = d * (-beta/2) with d = (-2 s + |y|^2) + |t|^2 in the
-// reference's dgemm + dger order (comm.c:590-619); -inf when exp underflows.
-__device__ __forceinline__ double exponent(double s, double yk, double tn, double nbh, bool valid) {
+// reference's dgemm + dger order (comm.c:590-619); -inf when exp underflows
+// (and for the +inf |y|^2 that stands for a centre past the end).
+__device__ __forceinline__ double exponent(double s, double yk, double tn, double nbh) {
     const double d = fma(-2.0, s, yk) + tn;
     const double x = d * nbh;
-    return (valid && x > kExpUnderflowX) ? x : -INFINITY;
+    return (x > kExpUnderflowX) ? x : -INFINITY;
 }
 
 // ---------------------------------------------------------------- pass 1
-__global__ __launch_bounds__(NT) void k_e1_f64(
-    const double *__restrict__ T, const double *__restrict__ tt, long N,
-    const double *__restrict__ Y, const double *__restrict__ yy, int K, int ld,
-    double nbh, double it, int two, int isDA, double logK,
-    double *__restrict__ pm, double *__restrict__ pl,
-    double *__restrict__ logg, double *__restrict__ logh) {
-    __shared__ double Ts[DC][TP + 1];
-    __shared__ double Ys[DC][TK + 1];
-    __shared__ double red[3][16][TP];
-
-    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-    const long n0 = (long)blockIdx.x * TP;
-
-    double tn[4], xm[4], s1[4], s2[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const long n = n0 + tx + 16 * i;
-        tn[i] = (n < N) ? tt[n] : 0.0;
-        xm[i] = -INFINITY; s1[i] = 0.0; s2[i] = 0.0;
-    }
-
-    for (int k0 = 0; k0 < K; k0 += TK) {
-        double acc[4][4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc[i][j] = 0.0;
-        for (int d0 = 0; d0 < ld; d0 += DC) {
-            __syncthreads();
-            stage_chunk(Ts, T, N, n0, ld, d0, tid);
-            stage_chunk(Ys, Y, K, k0, ld, d0, tid);
-            __syncthreads();
-            cross_chunk(acc, Ts, Ys, tx, ty);
-        }
-        double yk[4]; bool kv[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int k = k0 + ty + 16 * j;
-            kv[j] = k < K;
-            yk[j] = kv[j] ? yy[k] : 0.0;
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            double x[4], t = -INFINITY;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                x[j] = exponent(acc[i][j], yk[j], tn[i], nbh, kv[j]);
-                t = fmax(t, x[j]);
-            }
-            if (t > xm[i]) {             // new running max: rescale the sums
-                const double r = xm[i] - t;
-                s1[i] *= exp(r);
-                if (two) s2[i] *= exp(r * it);
-                xm[i] = t;
-            }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                if (x[j] != -INFINITY) {
-                    const double r = x[j] - xm[i];
-                    s1[i] += exp(r);
-                    if (two) s2[i] += exp(r * it);
-                }
-            }
+// One slice's online sums: m its running maximum, s1 and s2 the sums of
+// exp(x - m) and exp((x - m) / temp).
+struct Slice {
+    double m = -INFINITY, s1 = 0.0, s2 = 0.0;
+    // a new running maximum rescales the sums
+    __device__ __forceinline__ void raise(double top, double it, int two) {
+        if (top > m) {
+            const double r = m - top;
+            s1 *= exp(r);
+            if (two) s2 *= exp(r * it);
+            m = top;
         }
     }
+};
 
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        red[0][ty][tx + 16 * i] = xm[i];
-        red[1][ty][tx + 16 * i] = s1[i];
-        red[2][ty][tx + 16 * i] = s2[i];
+// Below this a term cannot change a sum: each slice's sums are at least 1 (its
+// maximum's own term), and e^-37 is less than half a unit in their last place.
+constexpr double kNoTerm = -37.0;
+
+// log g and log h of a point from its merged sums (mpicomm.c:382-390 for a
+// zero column), stored with the normalisers; returns its share of the sums
+struct PointOut {
+    double *pm, *pl, *logg, *logh;
+    double it, logK;
+    int two, isDA;
+    __device__ __forceinline__ void put(long n, double M, double S1, double S2, double &lg,
+                                        double &lh, double &zc) const {
+        double l2 = 0.0;
+        if (M == -INFINITY) {
+            lg = isDA ? -INFINITY : logK;
+            lh = logK;
+            zc = 1.0;
+        } else {
+            const double l1 = log(S1);
+            l2 = two ? log(S2) : l1;
+            lg = M + l1;
+            lh = M * it + l2;
+        }
+        pm[n] = M;
+        pl[n] = l2;
+        logg[n] = lg;
+        logh[n] = lh;
     }
+};
+
+// the workgroup's sums of log g, log h and zero columns to partLog
+__device__ __forceinline__ void put_logs(double lg, double lh, double zc,
+                                         double (*sm)[NT / 64], double *__restrict__ partLog) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        lg += __shfl_xor(lg, o);
+        lh += __shfl_xor(lh, o);
+        zc += __shfl_xor(zc, o);
+    }
+    const int w = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0) { sm[0][w] = lg; sm[1][w] = lh; sm[2][w] = zc; }
     __syncthreads();
-    if (tid < TP) {
-        const int p = tid;
-        const long n = n0 + p;
-        double M = -INFINITY;
-        for (int t = 0; t < 16; ++t) M = fmax(M, red[0][t][p]);
-        double S1 = 0.0, S2 = 0.0;
-        if (M != -INFINITY) {
-            for (int t = 0; t < 16; ++t) {
-                const double m = red[0][t][p];
-                if (m == -INFINITY) continue;
-                const double r = m - M;
-                S1 += red[1][t][p] * exp(r);
-                if (two) S2 += red[2][t][p] * exp(r * it);
-            }
-        }
-        if (n < N) {
-            if (M == -INFINITY) {          // zero column (mpicomm.c:382-390)
-                pm[n] = -INFINITY;
-                pl[n] = 0.0;
-                logh[n] = logK;
-                logg[n] = isDA ? -INFINITY : logK;
-            } else {
-                const double lS1 = log(S1);
-                const double lS2 = two ? log(S2) : lS1;
-                pm[n] = M;
-                pl[n] = lS2;
-                logg[n] = M + lS1;
-                logh[n] = M * it + lS2;
-            }
-        }
+    if (threadIdx.x < 3) {
+        const double *s = sm[threadIdx.x];
+        partLog[3 * (long)blockIdx.x + threadIdx.x] = (s[0] + s[1]) + (s[2] + s[3]);
     }
 }
 
-// ---------------------------------------------------------------- pass 2
-template <int DJ>
-struct E2Smem {
-    double Tb[TP][16 * DJ + 1];
-    double Rs[TK][TP + 1];
-    double Ys[DC][TK + 1];
-    double gr[16][TK];
-};
+// 64 points (16 per wave) against the centres in tiles of 128: a wave holds
+// eight 16 x 16 accumulators.  The operands pass through LDS in 16-wide d
+// chunks, double buffered, the next chunk's loads in registers while one is
+// multiplied.  Lane (j, g) holds point j and rows 4 r + g of an accumulator.
+//   S = 1: the workgroup takes every centre, row i of accumulator a of tile t
+//          being centre 128 t + 16 a + i; the lane keeps slices 4 r + g and
+//          the workgroup finishes its points.
+//   S = 4: it takes the slices 4 q .. 4 q + 3, q = blockIdx.y, accumulator a
+//          of tile t holding those of the 64 centres from 64 (8 t + a) on (row
+//          i: centre 16 (i / 4) + 4 q + i % 4 of them); the lane keeps slice
+//          4 q + g, and k_e1_merge finishes the points.
+// Bound by the FP64 pipe, which the matrix instructions, the exponentials (two
+// per element away from temperature 1, left out where no term of a wave can
+// change its sum) and the exponents share: at N = 10^6, D = 166, K = 8000,
+// temperature 2, 62 ms, of which the 2 K N D flops take 35 at the pipe's measured
+// 77.7 TFLOP/s (4 x 4 register tiles of FMAs: 132 ms, their eight LDS reads per
+// 16 FMAs cost twice the pipe's time).  N = 1640, K = 5832: 0.26 ms (3.27).
+constexpr int P1 = 64, C1 = 128, RW = C1 / 16;
 
-template <int DJ>
-__global__ __launch_bounds__(NT) void k_e2_f64(
+template <int S>
+__global__ __launch_bounds__(NT, 2) void k_e1_f64(
+    const double *__restrict__ T, const double *__restrict__ tt, long N,
+    const double *__restrict__ Y, const double *__restrict__ yy, int K, int D, int ld, double nbh,
+    PointOut po, double *__restrict__ partLog, double *__restrict__ part) {
+    constexpr int LT = P1 / 32, LY = C1 / 32;      // 16-byte loads per thread and chunk
+    constexpr int CT = C1 * S;                     // centres from one tile to the next
+    constexpr int CA = 16 * S;                     // from one accumulator to the next
+    __shared__ __attribute__((aligned(16))) double Ts[2][P1 * DCP];
+    __shared__ __attribute__((aligned(16))) double Ys[2][C1 * DCP];
+    __shared__ double ys[2][C1];
+    __shared__ double sm[3][NT / 64];
+
+    const int tid = threadIdx.x, l = tid & 63, w = tid >> 6, j = l & 15, g = l >> 4;
+    const int q4 = 4 * blockIdx.y;
+    const long n0 = (long)blockIdx.x * P1, n = n0 + 16 * w + j;
+    const int ntiles = (K + CT - 1) / CT;
+    const int nch = (D + DC - 1) / DC;                // d chunks per centre tile
+    const int last8 = (D - (nch - 1) * DC + 7) / 8;   // 8-wide steps of the last one
+    const double it = po.it;
+    const int two = po.two;
+    auto centre = [&](int t, int row) {
+        const int i = row & 15;
+        return t * CT + (row >> 4) * CA + (S == 1 ? i : 16 * (i >> 2) + q4 + (i & 3));
+    };
+
+    // staging: eight threads per row of a chunk, 16 bytes each; rows past the
+    // end repeat the last one (|y|^2 = +inf there, and no point is stored)
+    const int sr = tid >> 3, sp = tid & 7;
+    d2 rt[LT], ry[LY];
+    double ryy = INFINITY;
+    auto load = [&](int t, int q) {                    // tile t, d chunk q
+#pragma unroll
+        for (int i = 0; i < LT; ++i)
+            rt[i] = *(const d2 *)(T + min(n0 + sr + 32 * i, N - 1) * ld + q * DC + 2 * sp);
+#pragma unroll
+        for (int i = 0; i < LY; ++i)
+            ry[i] = *(const d2 *)(Y + (long)min(centre(t, sr + 32 * i), K - 1) * ld + q * DC + 2 * sp);
+        if (q == 0 && tid < C1) {
+            const int k = centre(t, tid);
+            ryy = (k < K) ? yy[k] : INFINITY;
+        }
+    };
+    auto store = [&](int b, int t, int q) {
+#pragma unroll
+        for (int i = 0; i < LT; ++i) put_pair(&Ts[b][(sr + 32 * i) * DCP], 2 * sp, rt[i]);
+#pragma unroll
+        for (int i = 0; i < LY; ++i) put_pair(&Ys[b][(sr + 32 * i) * DCP], 2 * sp, ry[i]);
+        if (q == 0 && tid < C1) ys[t & 1][tid] = ryy;
+    };
+
+    const double tn = (n < N) ? tt[n] : 0.0;
+    Slice sl[S == 1 ? 4 : 1];
+    d4 acc[RW];
+    // slice s takes in the four centres it has of 64: exponents x of rows
+    // row0 + step i
+    auto take = [&](Slice &s, double (&x)[4], const double *yt, int row0, int step) {
+        double top = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            x[i] = exponent(x[i], yt[row0 + step * i + g], tn, nbh);
+            top = fmax(top, x[i]);
+        }
+        s.raise(top, it, two);
+        // (-inf: nothing in the slice yet; its x are all -inf too)
+        const double m = (s.m == -INFINITY) ? 0.0 : s.m;
+        const double near = top - m;
+        if (__any(near > kNoTerm)) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s.s1 += exp(x[i] - m);
+        }
+        if (two && __any(near * it > kNoTerm)) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s.s2 += exp((x[i] - m) * it);
+        }
+    };
+    auto close_tile = [&](const double *yt, int na) {
+        if (S == 1) {
+#pragma unroll
+            for (int h = 0; h < RW; h += 4)
+                if (h < na)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        double x[4] = {acc[h][r], acc[h + 1][r], acc[h + 2][r], acc[h + 3][r]};
+                        take(sl[S == 1 ? r : 0], x, yt, 16 * h + 4 * r, 16);
+                    }
+        } else {
+#pragma unroll
+            for (int a = 0; a < RW; ++a)
+                if (a < na) {
+                    double x[4] = {acc[a][0], acc[a][1], acc[a][2], acc[a][3]};
+                    take(sl[0], x, yt, 16 * a, 4);
+                }
+        }
+    };
+
+    load(0, 0);
+    store(0, 0, 0);
+    __syncthreads();
+    int b = 0;
+    for (int t = 0; t < ntiles; ++t) {
+        // accumulators of this tile that hold a centre
+        const int na = min(RW, (K - t * CT + CA - 1) / CA);
+#pragma unroll
+        for (int a = 0; a < RW; ++a) acc[a] = d4{0.0, 0.0, 0.0, 0.0};
+        for (int q = 0; q < nch; ++q, b ^= 1) {
+            const int tq = (q + 1 < nch) ? t : t + 1, qn = (q + 1 < nch) ? q + 1 : 0;
+            const bool more = tq < ntiles;
+            if (more) load(tq, qn);
+            const int steps = (q + 1 < nch) ? DC / 8 : last8;
+            for (int s = 0; s < steps; ++s) {
+                const double *yr = &Ys[b][j * DCP + 8 * s + 2 * g];
+                const d2 bv = *(const d2 *)&Ts[b][(16 * w + j) * DCP + 8 * s + 2 * g];
+                if (na == RW) {
+                    // the centre rows' operands are read one step ahead of
+                    // their MFMAs (the sched_barrier keeps them there)
+                    d2 av = *(const d2 *)yr;
+#pragma unroll
+                    for (int a = 0; a < RW; ++a) {
+                        const d2 an = *(const d2 *)(yr + 16 * (a + 1 < RW ? a + 1 : a) * DCP);
+                        __builtin_amdgcn_sched_barrier(0);
+                        acc[a] = mfma64(av.x, bv.x, acc[a]);
+                        acc[a] = mfma64(av.y, bv.y, acc[a]);
+                        av = an;
+                    }
+                } else {
+#pragma unroll
+                    for (int a = 0; a < RW - 1; ++a)
+                        if (a < na) {
+                            const d2 av = *(const d2 *)(yr + 16 * a * DCP);
+                            acc[a] = mfma64(av.x, bv.x, acc[a]);
+                            acc[a] = mfma64(av.y, bv.y, acc[a]);
+                        }
+                }
+            }
+            if (more) store(b ^ 1, tq, qn);
+            // (before the barrier: the next tile's |y|^2 goes to the other
+            // half of ys, the one after it only past this barrier)
+            if (q + 1 == nch) close_tile(ys[t & 1], na);
+            __syncthreads();
+        }
+    }
+    if (S == 4) {
+        if (n < N) {
+            double *o = part + (long)(q4 + g) * 3 * N + n;
+            o[0] = sl[0].m;
+            o[N] = sl[0].s1;
+            o[2 * N] = sl[0].s2;
+        }
+        return;
+    }
+    // merge the point's sixteen slices in order (slice 4 r + g is element r of
+    // lane j + 16 g); every lane of the point gets the same sums
+    double M = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < (S == 1 ? 4 : 1); ++r) M = fmax(M, sl[r].m);
+    M = fmax(M, __shfl_xor(M, 16));
+    M = fmax(M, __shfl_xor(M, 32));
+    double S1 = 0.0, S2 = 0.0;
+#pragma unroll
+    for (int r = 0; r < (S == 1 ? 4 : 1); ++r) {
+        const double d = (M == -INFINITY) ? 0.0 : sl[r].m - M;
+        const double f1 = exp(d), f2 = two ? exp(d * it) : 0.0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            S1 = fma(__shfl(sl[r].s1, j + 16 * q), __shfl(f1, j + 16 * q), S1);
+            if (two) S2 = fma(__shfl(sl[r].s2, j + 16 * q), __shfl(f2, j + 16 * q), S2);
+        }
+    }
+    double lg = 0.0, lh = 0.0, zc = 0.0;
+    if (g == 0 && n < N) po.put(n, M, S1, S2, lg, lh, zc);
+    put_logs(lg, lh, zc, sm, partLog);
+}
+
+// Finishes the points whose slices part holds: slice t's m, s1 and s2 of point
+// n at part[(3 t + 0 .. 2) N + n].
+__global__ __launch_bounds__(NT) void k_e1_merge(const double *__restrict__ part, long N,
+                                                 PointOut po, double *__restrict__ partLog) {
+    __shared__ double sm[3][NT / 64];
+    const long n = (long)blockIdx.x * NT + threadIdx.x;
+    double lg = 0.0, lh = 0.0, zc = 0.0;
+    if (n < N) {
+        double m[16], s1[16], s2[16], M = -INFINITY, S1 = 0.0, S2 = 0.0;
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+            m[t] = part[3L * t * N + n];
+            s1[t] = part[(3L * t + 1) * N + n];
+            s2[t] = part[(3L * t + 2) * N + n];
+        }
+#pragma unroll
+        for (int t = 0; t < 16; ++t) M = fmax(M, m[t]);
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+            const double d = (M == -INFINITY) ? 0.0 : m[t] - M;
+            S1 = fma(s1[t], exp(d), S1);
+            if (po.two) S2 = fma(s2[t], exp(d * po.it), S2);
+        }
+        po.put(n, M, S1, S2, lg, lh, zc);
+    }
+    put_logs(lg, lh, zc, sm, partLog);
+}
+
+// ---------------------------------------------------------------- pass 2
+// A workgroup owns 64 centres, 16 per wave with their rows in registers as
+// the B operand, and one chunk of points, streamed in 16-point tiles through
+// a double-buffered LDS copy (rows at ld + 4: both operand reads below touch
+// every bank equally).  C[n][k] = T Y^T leaves R in the accumulator layout,
+// which is the A operand layout of RT[k][d] += sum_n R[k][n] T[n][d] with the
+// points of element r, 4 r .. 4 r + 3, as the inner index: R goes from the
+// exponential straight into the second product.
+// Bound by the FP64 pipe: at N = 10^6, D = 166, K = 8000, 105 ms, of which the
+// 4 K N D flops (D padded to 168 and 176) take 71 at 77.7 TFLOP/s, the
+// exponentials about 8 and the last, part-filled round of workgroups 12 (428 ms
+// with FMAs from LDS; half as much again without the read-ahead and the split
+// staging below).  Two workgroups share a CU: 256 registers hold the centre
+// operand and the accumulators up to D = 192, with one half of the next tile's
+// loads in flight.
+template <int DB>
+__global__ __launch_bounds__(NT, 2) void k_e2_f64(
     const double *__restrict__ T, const double *__restrict__ tt, long N,
     const double *__restrict__ Y, const double *__restrict__ yy, int K, int D,
     double nbh, double it, double invK,
     const double *__restrict__ pm, const double *__restrict__ pl, long chunk,
     double *__restrict__ partRT, double *__restrict__ partG) {
-    constexpr int ld = 16 * DJ;
-    __shared__ E2Smem<DJ> sm;
+    constexpr int ld = 16 * DB, LD = ld + 4;
+    constexpr int NL = (DB + 1) / 2;               // 16-byte loads per thread and tile
+    __shared__ __attribute__((aligned(16))) double Tb[2][16 * LD];
+    __shared__ double pt[2][3][16];                // |t|^2, x_max and log S2 of the tile
 
-    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-    const int kq = tid >> 4, dq = tid & 15;          // RT-stage mapping
-    const int k0 = blockIdx.x * TK;
+    const int tid = threadIdx.x, l = tid & 63, w = tid >> 6, j = l & 15, g = l >> 4;
+    const int kw = blockIdx.x * 64 + 16 * w, k = kw + j;
     const long nb = (long)blockIdx.y * chunk;
     const long ne = (nb + chunk < N) ? nb + chunk : N;
+    // (the last 8-wide step of d is all padding when D <= ld - 8)
+    const bool full = D > ld - 8;
 
-    double yk[4]; bool kv[4];
+    d2 yb[2 * DB];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int k = k0 + ty + 16 * j;
-        kv[j] = k < K;
-        yk[j] = kv[j] ? yy[k] : 0.0;
-    }
-    double rt[4][DJ];
+    for (int s = 0; s < 2 * DB; ++s)
+        yb[s] = (k < K) ? d2{Y[(long)k * ld + 8 * s + g], Y[(long)k * ld + 8 * s + 4 + g]} : d2{0.0, 0.0};
+    const double yk = (k < K) ? yy[k] : INFINITY;
+    const double rz = (k < K) ? invK : 0.0;        // R of a zero column
+    d4 acc[DB];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < DJ; ++j) rt[i][j] = 0.0;
-    double gacc[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int b = 0; b < DB; ++b) acc[b] = d4{0.0, 0.0, 0.0, 0.0};
+    double gs[4] = {0.0, 0.0, 0.0, 0.0};           // points n = 4 r + g (mod 16)
 
-    for (long n0 = nb; n0 < ne; n0 += TP) {
-        __syncthreads();
-        for (int e = tid; e < TP * ld; e += NT) {
-            const int r = e / ld, d = e % ld;
-            const long n = n0 + r;
-            sm.Tb[r][d] = (n < ne) ? T[n * ld + d] : 0.0;
+    // staging: sixteen threads per row, 16 bytes each per load; rows past the
+    // end are zero, and so is their R
+    const int sr = tid >> 4, sp = tid & 15;
+    const bool tail = DB % 2 == 0 || sp < 8;       // the last load of an odd row: half of them
+    constexpr int H = (NL + 1) / 2;                // loads in flight: half a tile's
+    d2 rt[H];
+    double rp;
+    const double *psrc = tt;                       // threads 0 .. 47: one of a point's three values
+    if (sr == 1) psrc = pm;
+    if (sr >= 2) psrc = pl;
+    const double pend = (sr == 1) ? INFINITY : 0.0;   // past the end: x_max = +inf, so R = 0
+    auto half_load = [&](int h, long n0) {
+        const double *src = T + min(n0 + sr, ne - 1) * ld + 2 * sp;
+#pragma unroll
+        for (int i = 0; i < H; ++i) {
+            const int f = h * H + i;
+            if (f < NL && (f < NL - 1 || tail)) rt[i] = *(const d2 *)(src + 32 * f);
         }
-        double tn[4], m[4], l[4]; bool nv[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const long n = n0 + tx + 16 * i;
-            nv[i] = n < ne;
-            tn[i] = nv[i] ? tt[n] : 0.0;
-            m[i] = nv[i] ? pm[n] : 0.0;
-            l[i] = nv[i] ? pl[n] : 0.0;
+        if (h == 0) {
+            const double v = psrc[min(n0 + sp, ne - 1)];
+            rp = (n0 + sp < ne) ? v : pend;
         }
-        double acc[4][4];
+    };
+    auto half_store = [&](int h, int b, long n0) {
+        if (n0 + sr >= ne) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc[i][j] = 0.0;
-        for (int d0 = 0; d0 < ld; d0 += DC) {
-            __syncthreads();
-            stage_chunk(sm.Ys, Y, K, k0, ld, d0, tid);
-            __syncthreads();
-#pragma unroll
-            for (int dd = 0; dd < DC; ++dd) {
-                double a[4], b[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) a[i] = sm.Tb[tx + 16 * i][d0 + dd];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) b[j] = sm.Ys[dd][ty + 16 * j];
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) acc[i][j] = fma(a[i], b[j], acc[i][j]);
-            }
+            for (int i = 0; i < H; ++i) rt[i] = d2{0.0, 0.0};
         }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                double r = 0.0;
-                if (nv[i]) {
-                    if (m[i] == -INFINITY) {
-                        r = kv[j] ? invK : 0.0;
-                    } else {
-                        const double x = exponent(acc[i][j], yk[j], tn[i], nbh, kv[j]);
-                        r = (x != -INFINITY) ? exp((x - m[i]) * it - l[i]) : 0.0;
-                    }
-                }
-                gacc[j] += r;
-                sm.Rs[ty + 16 * j][tx + 16 * i] = r;
-            }
+        for (int i = 0; i < H; ++i) {
+            const int f = h * H + i;
+            if (f < NL && (f < NL - 1 || tail)) put_pair(&Tb[b][sr * LD + 32 * f], 2 * sp, rt[i]);
         }
-        __syncthreads();
-#pragma unroll 4
-        for (int n = 0; n < TP; ++n) {
-            double rv[4], tv[DJ];
+        if (h == 0 && tid < 48) pt[b][sr][sp] = rp;
+    };
+    if (nb < ne) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) rv[i] = sm.Rs[kq + 16 * i][n];
-#pragma unroll
-            for (int j = 0; j < DJ; ++j) tv[j] = sm.Tb[n][dq + 16 * j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < DJ; ++j) rt[i][j] = fma(rv[i], tv[j], rt[i][j]);
+        for (int h = 0; h < 2; ++h) {
+            half_load(h, nb);
+            half_store(h, 0, nb);
         }
     }
-
-    // partial RT of this chunk
-    const long c = blockIdx.y;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int k = k0 + kq + 16 * i;
-        if (k >= K) continue;
-#pragma unroll
-        for (int j = 0; j < DJ; ++j) {
-            const int d = dq + 16 * j;
-            if (d < D) partRT[(c * K + k) * D + d] = rt[i][j];
-        }
-    }
-    // partial G: reduce gacc over the 16 threads that share ty
     __syncthreads();
+    int b = 0;
+    // (the sched_barriers keep each operand's LDS read one step ahead of the
+    // MFMAs that use it; the compiler otherwise puts it right before them and
+    // waits out its latency every two MFMAs)
+    for (long n0 = nb; n0 < ne; n0 += 16, b ^= 1) {
+        const bool more = n0 + 16 < ne;
+        if (more) half_load(0, n0 + 16);
+        d4 c = {0.0, 0.0, 0.0, 0.0};
+        const double *ta = &Tb[b][j * LD + 2 * g];
+        d2 a = *(const d2 *)ta;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) sm.gr[tx][ty + 16 * j] = gacc[j];
-    __syncthreads();
-    if (tid < TK) {
-        double s = 0.0;
-        for (int t = 0; t < 16; ++t) s += sm.gr[t][tid];
-        const int k = k0 + tid;
-        if (k < K) partG[c * K + k] = s;
+        for (int s = 0; s < 2 * DB; ++s) {
+            const d2 an = *(const d2 *)(ta + 8 * (s + 1 < 2 * DB ? s + 1 : s));
+            __builtin_amdgcn_sched_barrier(0);
+            if (s < 2 * DB - 1 || full) {
+                c = mfma64(a.x, yb[s].x, c);
+                c = mfma64(a.y, yb[s].y, c);
+            }
+            a = an;
+        }
+        if (more) {
+            half_store(0, b ^ 1, n0 + 16);
+            half_load(1, n0 + 16);
+        }
+        double R[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int n = 4 * r + g;
+            const double x = exponent(c[r], yk, pt[b][0][n], nbh);
+            R[r] = exp((x - pt[b][1][n]) * it - pt[b][2][n]);
+            asm volatile("" : "+v"(R[r]));         // (no branch around the exponential)
+        }
+        const double *tb = &Tb[b][g * LD + dpos(j)];
+        double t0 = tb[0], t1 = tb[DB > 1 ? 16 : 4 * LD];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            R[r] = (pt[b][1][4 * r + g] == -INFINITY) ? rz : R[r];
+            gs[r] += R[r];
+        }
+#pragma unroll
+        for (int i = 0; i < 4 * DB; ++i) {
+            const int i2 = (i + 2 < 4 * DB) ? i + 2 : i;
+            const double t2 = tb[(i2 / DB) * 4 * LD + 16 * (i2 % DB)];
+            __builtin_amdgcn_sched_barrier(0);
+            acc[i % DB] = mfma64(R[i / DB], t0, acc[i % DB]);
+            t0 = t1;
+            t1 = t2;
+        }
+        if (more) half_store(1, b ^ 1, n0 + 16);
+        __syncthreads();
     }
+    const long ch = blockIdx.y;
+#pragma unroll
+    for (int q = 0; q < DB; ++q)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int kk = kw + 4 * r + g, d = 16 * q + j;
+            if (kk < K && d < D) partRT[(ch * K + kk) * D + d] = acc[q][r];
+        }
+    double G = 0.0;                                // the sixteen classes in order
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) G += __shfl(gs[r], j + 16 * q);
+    if (g == 0 && k < K) partG[ch * K + k] = G;
 }
 
-__global__ void k_reduce_parts(const double *__restrict__ partRT, const double *__restrict__ partG,
-                               int NC, int K, int D, double *__restrict__ RT,
-                               double *__restrict__ G) {
+// RT and G from the chunk partials, summed in chunk order with eight loads in
+// flight; the last workgroup sums pass 1's partial log sums into scal instead.
+__global__ __launch_bounds__(256) void k_reduce_parts(
+    const double *__restrict__ partRT, const double *__restrict__ partG, int NC, int K, int D,
+    double *__restrict__ RT, double *__restrict__ G, const double *__restrict__ partLog, long nlog,
+    double *__restrict__ scal) {
+    if (blockIdx.x == gridDim.x - 1) {
+        __shared__ double s[3][256];
+        double a[3] = {0.0, 0.0, 0.0};
+        for (long i = threadIdx.x; i < nlog; i += 256)
+            for (int x = 0; x < 3; ++x) a[x] += partLog[3 * i + x];
+        for (int x = 0; x < 3; ++x) s[x][threadIdx.x] = a[x];
+        __syncthreads();
+        for (int o = 128; o > 0; o >>= 1) {
+            if ((int)threadIdx.x < o)
+                for (int x = 0; x < 3; ++x) s[x][threadIdx.x] += s[x][threadIdx.x + o];
+            __syncthreads();
+        }
+        if (threadIdx.x == 0) {
+            scal[kScalSumLogG] = s[0][0];
+            scal[kScalSumLogH] = s[1][0];
+            scal[kScalNZero] = s[2][0];
+        }
+        return;
+    }
     const long KD = (long)K * D;
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < KD) {
+    const long i = (long)blockIdx.x * 256 + threadIdx.x;
+    auto sum = [&](const double *p, long stride) {
         double s = 0.0;
-        for (int c = 0; c < NC; ++c) s += partRT[c * KD + i];
-        RT[i] = s;
-    }
-    if (i < K) {
-        double s = 0.0;
-        for (int c = 0; c < NC; ++c) s += partG[(long)c * K + i];
-        G[i] = s;
-    }
+        int c = 0;
+        for (; c + 8 <= NC; c += 8) {
+            double v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = p[(c + u) * stride];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) s += v[u];
+        }
+        for (; c < NC; ++c) s += p[c * stride];
+        return s;
+    };
+    if (i < KD) RT[i] = sum(partRT + i, KD);
+    else if (i < KD + K) G[i - KD] = sum(partG + (i - KD), K);
 }
 
 // ---------------------------------------------------------------- debug / MAP
@@ -337,7 +565,7 @@ __global__ void k_resp_dense(const double *__restrict__ T, const double *__restr
     } else {
         double s = 0.0;
         for (int d = 0; d < ld; ++d) s = fma(T[n * ld + d], Y[(long)k * ld + d], s);
-        const double x = exponent(s, yy[k], tt[n], nbh, true);
+        const double x = exponent(s, yy[k], tt[n], nbh);
         r = (x != -INFINITY) ? exp((x - pm[n]) * it - pl[n]) : 0.0;
     }
     R[(long)k * ldR + n] = r;
@@ -360,7 +588,7 @@ __global__ void k_map_f64(const double *__restrict__ T, const double *__restrict
         } else {
             double s = 0.0;
             for (int d = 0; d < ld; ++d) s = fma(T[n * ld + d], Y[(long)k * ld + d], s);
-            const double x = exponent(s, yy[k], tt[n], nbh, true);
+            const double x = exponent(s, yy[k], tt[n], nbh);
             r = (x != -INFINITY) ? exp((x - pm[n]) * it - pl[n]) : 0.0;
         }
         for (int l = 0; l < L; ++l) acc[l] = fma(r, X[(long)k * L + l], acc[l]);
@@ -368,12 +596,16 @@ __global__ void k_map_f64(const double *__restrict__ T, const double *__restrict
     for (int l = 0; l < L; ++l) M[n * L + l] = acc[l];
 }
 
-template <int DJ>
-int launch_e2(dg_ctx *c, double nbh, double it, long chunk, dim3 grid) {
-    hipLaunchKernelGGL(k_e2_f64<DJ>, grid, dim3(NT), 0, c->stream, c->T64, c->tt, c->N, c->Y64,
-                       c->yy, c->K, c->D, nbh, it, 1.0 / c->K, c->pm, c->pl, chunk, c->partRT,
-                       c->partG);
-    return DG_OK;
+// f(std::integral_constant<int, DB>) for DB = db in 1 .. 12, false otherwise
+template <typename F>
+bool with_db(int db, F &&f) {
+    switch (db) {
+#define DG_DB(V) case V: f(std::integral_constant<int, V>{}); return true;
+        DG_DB(1) DG_DB(2) DG_DB(3) DG_DB(4) DG_DB(5) DG_DB(6)
+        DG_DB(7) DG_DB(8) DG_DB(9) DG_DB(10) DG_DB(11) DG_DB(12)
+#undef DG_DB
+        default: return false;
+    }
 }
 
 // ---------------------------------------------------------------- critical temperature
@@ -421,7 +653,7 @@ __global__ __launch_bounds__(NT) void k_ctemp_moments(
                 } else {
                     double s = 0.0;
                     for (int d = 0; d < ld; ++d) s = fma(T[n * ld + d], Ys[d], s);
-                    const double x = exponent(s, yy[k], tt[n], nbh, true);
+                    const double x = exponent(s, yy[k], tt[n], nbh);
                     r = (x != -INFINITY) ? exp((x - pm[n]) * it - pl[n]) : 0.0;
                 }
             }
@@ -482,48 +714,66 @@ __global__ void k_sum_chunks(const double *__restrict__ part, int nc, long len,
 
 }  // namespace
 
-int dg_estep_fp64(dg_ctx *c, int isDA, double temp) {
+// Pass 1 splits a point tile's slices over four workgroups up to 64 x 16 points
+// per CU: below that, whole point tiles are too few to spread evenly (N = 10^5,
+// D = 166, K = 8000: 6.4 ms split, 7.2 whole; N = 260000, K = 1000: 2.17 and
+// 2.25).  Above it the slices' states (384 bytes a point) are not worth their
+// way through memory.
+constexpr long kSplitPoints = 64L * 16 * 256;
+size_t dg_pass1_part(long N) { return N < kSplitPoints ? (size_t)48 * N : 0; }
+long dg_pass1_wgs(long N) { return N < kSplitPoints ? (N + NT - 1) / NT : (N + P1 - 1) / P1; }
+
+int dg_pass1_fp64(dg_ctx *c, int isDA, double temp) {
     const double nbh = -c->beta / 2.0;
     const double it = isDA ? 1.0 / temp : 1.0;
-    const int two = (isDA && it != 1.0) ? 1 : 0;
-    const double logK = log((double)c->K);
-    const int DJ = c->ldt / 16;
-    if (DJ < 1 || DJ > 12) return dg_fail(c, DG_EINVAL, "FP64 path supports D <= 192");
-
-    if (c->timing) DG_HIP(c, hipEventRecord(c->ev[0], c->stream));
-    const unsigned nt = (unsigned)((c->N + TP - 1) / TP);
-    hipLaunchKernelGGL(k_e1_f64, dim3(nt), dim3(NT), 0, c->stream, c->T64, c->tt, c->N, c->Y64,
-                       c->yy, c->K, c->ldt, nbh, it, two, isDA, logK, c->pm, c->pl, c->logg,
-                       c->logh);
-    DG_HIP(c, hipGetLastError());
-    if (c->timing) DG_HIP(c, hipEventRecord(c->ev[1], c->stream));
-
-    const long tiles = (c->N + TP - 1) / TP;
-    const long chunk = ((tiles + c->NC - 1) / c->NC) * TP;
-    dim3 grid((unsigned)((c->K + TK - 1) / TK), (unsigned)c->NC);
-    switch (DJ) {
-        case 1: launch_e2<1>(c, nbh, it, chunk, grid); break;
-        case 2: launch_e2<2>(c, nbh, it, chunk, grid); break;
-        case 3: launch_e2<3>(c, nbh, it, chunk, grid); break;
-        case 4: launch_e2<4>(c, nbh, it, chunk, grid); break;
-        case 5: launch_e2<5>(c, nbh, it, chunk, grid); break;
-        case 6: launch_e2<6>(c, nbh, it, chunk, grid); break;
-        case 7: launch_e2<7>(c, nbh, it, chunk, grid); break;
-        case 8: launch_e2<8>(c, nbh, it, chunk, grid); break;
-        case 9: launch_e2<9>(c, nbh, it, chunk, grid); break;
-        case 10: launch_e2<10>(c, nbh, it, chunk, grid); break;
-        case 11: launch_e2<11>(c, nbh, it, chunk, grid); break;
-        default: launch_e2<12>(c, nbh, it, chunk, grid); break;
+    const PointOut po{c->pm, c->pl, c->logg, c->logh, it, log((double)c->K),
+                      (isDA && it != 1.0) ? 1 : 0, isDA};
+    const unsigned tiles = (unsigned)((c->N + P1 - 1) / P1);
+    auto go = [&](auto kernel, dim3 grid) {
+        hipLaunchKernelGGL(kernel, grid, dim3(NT), 0, c->stream, c->T64, c->tt, c->N, c->Y64, c->yy,
+                           c->K, c->D, c->ldt, nbh, po, c->partLog64, c->partRT);
+    };
+    if (c->N < kSplitPoints) {
+        go(k_e1_f64<4>, dim3(tiles, 4));
+        DG_HIP(c, hipGetLastError());
+        hipLaunchKernelGGL(k_e1_merge, dim3((unsigned)dg_pass1_wgs(c->N)), dim3(NT), 0, c->stream,
+                           c->partRT, c->N, po, c->partLog64);
+    } else {
+        go(k_e1_f64<1>, dim3(tiles));
     }
     DG_HIP(c, hipGetLastError());
-    if (c->timing) DG_HIP(c, hipEventRecord(c->ev[2], c->stream));
+    return DG_OK;
+}
 
-    const long KD = (long)c->K * c->D;
-    const long nred = KD > c->K ? KD : c->K;
-    hipLaunchKernelGGL(k_reduce_parts, dim3((unsigned)((nred + 255) / 256)), dim3(256), 0,
-                       c->stream, c->partRT, c->partG, c->NC, c->K, c->D, c->RT, c->G);
+int dg_pass2_fp64(dg_ctx *c, int isDA, double temp) {
+    const double nbh = -c->beta / 2.0;
+    const double it = isDA ? 1.0 / temp : 1.0;
+    const long tiles = (c->N + TP - 1) / TP;
+    const long chunk = ((tiles + c->NC - 1) / c->NC) * TP;
+    const dim3 grid((unsigned)((c->K + 63) / 64), (unsigned)c->NC);
+    auto go = [&](auto db) {
+        hipLaunchKernelGGL(k_e2_f64<decltype(db)::value>, grid, dim3(NT), 0, c->stream, c->T64, c->tt,
+                           c->N, c->Y64, c->yy, c->K, c->D, nbh, it, 1.0 / c->K, c->pm, c->pl,
+                           chunk, c->partRT, c->partG);
+    };
+    if (!with_db(c->ldt / 16, go)) return dg_fail(c, DG_EINVAL, "FP64 path supports D <= 192");
     DG_HIP(c, hipGetLastError());
-    return dg_reduce_logs(c);
+    return DG_OK;
+}
+
+int dg_estep_fp64(dg_ctx *c, int isDA, double temp) {
+    int rc;
+    if (c->timing) DG_HIP(c, hipEventRecord(c->ev[0], c->stream));
+    if ((rc = dg_pass1_fp64(c, isDA, temp))) return rc;
+    if (c->timing) DG_HIP(c, hipEventRecord(c->ev[1], c->stream));
+    if ((rc = dg_pass2_fp64(c, isDA, temp))) return rc;
+    if (c->timing) DG_HIP(c, hipEventRecord(c->ev[2], c->stream));
+    const long nred = (long)c->K * c->D + c->K;
+    hipLaunchKernelGGL(k_reduce_parts, dim3((unsigned)((nred + 255) / 256 + 1)), dim3(256), 0,
+                       c->stream, c->partRT, c->partG, c->NC, c->K, c->D, c->RT, c->G,
+                       c->partLog64, dg_pass1_wgs(c->N), c->scal);
+    DG_HIP(c, hipGetLastError());
+    return DG_OK;
 }
 
 int dg_resp_dense_fp64(dg_ctx *c, double *dR, long ldR) {

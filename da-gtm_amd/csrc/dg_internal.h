@@ -51,8 +51,9 @@ struct dg_ctx {
     double *pl = nullptr;          // N   per-point log S2 (pass 1)
     double *logg = nullptr;        // N
     double *logh = nullptr;        // N
-    double *partRT = nullptr;      // NC x K x D
+    double *partRT = nullptr;      // NC x K x D; before pass 2, pass 1's slice states
     double *partG = nullptr;       // NC x K
+    double *partLog64 = nullptr;   // pass 1's log sums, 3 per workgroup (behind partG)
     int NC = 1;                    // N chunks of E-pass 2
     double *partAB = nullptr;      // nchAB x (M1*M1 + M1*D) split-K partials of A, B
     int nchAB = 1;                 // centre chunks of the A/B reduction
@@ -221,6 +222,8 @@ int dg_hip_check(dg_ctx *ctx, hipError_t e, const char *what);
     } while (0)
 
 // ---- FP64 kernels (dg_fp64.hip) ----
+long dg_pass1_wgs(long N);        // workgroups that sum pass 1's logs
+size_t dg_pass1_part(long N);     // doubles of partRT that pass 1 needs for its states
 int dg_estep_fp64(dg_ctx *ctx, int isDA, double temp);
 int dg_resp_dense_fp64(dg_ctx *ctx, double *dR, long ldR);
 int dg_map_fp64(dg_ctx *ctx, const double *dX, int L, double *dM);
@@ -262,5 +265,4 @@ int dg_peaks_run(dg_ctx *ctx, int wgs, double *mfma_tflops, double *exp_per_s,
                  double *f64_tflops);
 // dst[r][d] = src[r lds + d] for d < D, 0 for D <= d < ld (device arrays)
 int dg_pad_rows(dg_ctx *ctx, const double *src, long rows, int D, long lds, int ld, double *dst);
-int dg_reduce_logs(dg_ctx *ctx);
 int dg_sum_into(dg_ctx *ctx, const double *v, long n, int slot);

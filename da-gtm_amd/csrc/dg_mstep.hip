@@ -43,45 +43,19 @@ __global__ void k_rownorm(const double *__restrict__ X, long rows, int ld, int D
     k_rownorm_body(blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, X, rows, ld, D, out);
 }
 
-// Deterministic block-tree sum of one or two vectors into scal[slot], scal[slot+1].
-// Single workgroup, FP64.
-__global__ __launch_bounds__(1024) void k_sum2(const double *__restrict__ a,
-                                               const double *__restrict__ b, long n,
-                                               double *__restrict__ scal, int slot) {
-    __shared__ double sa[1024], sb[1024];
-    double x = 0.0, y = 0.0;
-    for (long i = threadIdx.x; i < n; i += 1024) {
-        x += a[i];
-        if (b) y += b[i];
-    }
-    sa[threadIdx.x] = x; sb[threadIdx.x] = y;
+// Deterministic block-tree sum of a vector into scal[slot].  Single workgroup, FP64.
+__global__ __launch_bounds__(1024) void k_sum(const double *__restrict__ a, long n,
+                                              double *__restrict__ scal, int slot) {
+    __shared__ double sa[1024];
+    double x = 0.0;
+    for (long i = threadIdx.x; i < n; i += 1024) x += a[i];
+    sa[threadIdx.x] = x;
     __syncthreads();
     for (int s = 512; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) {
-            sa[threadIdx.x] += sa[threadIdx.x + s];
-            sb[threadIdx.x] += sb[threadIdx.x + s];
-        }
+        if ((int)threadIdx.x < s) sa[threadIdx.x] += sa[threadIdx.x + s];
         __syncthreads();
     }
-    if (threadIdx.x == 0) {
-        scal[slot] = sa[0];
-        if (b) scal[slot + 1] = sb[0];
-    }
-}
-
-// Number of zero columns (pm == -inf) into scal[kScalNZero].
-__global__ __launch_bounds__(1024) void k_count_zero(const double *__restrict__ pm, long n,
-                                                     double *__restrict__ scal) {
-    __shared__ double s[1024];
-    double c = 0.0;
-    for (long i = threadIdx.x; i < n; i += 1024) c += (pm[i] == -INFINITY) ? 1.0 : 0.0;
-    s[threadIdx.x] = c;
-    __syncthreads();
-    for (int w = 512; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) scal[kScalNZero] = s[0];
+    if (threadIdx.x == 0) scal[slot] = sa[0];
 }
 
 // tr(A0) into *out, summed by the first wave; every thread of the workgroup
@@ -1085,18 +1059,8 @@ int dg_rownorms(dg_ctx *c, const double *X, long rows, int ld, int D, double *ou
     return DG_OK;
 }
 
-int dg_reduce_logs(dg_ctx *c) {
-    hipLaunchKernelGGL(k_sum2, dim3(1), dim3(1024), 0, c->stream, c->logg, c->logh, c->N,
-                       c->scal, (int)kScalSumLogG);
-    DG_HIP(c, hipGetLastError());
-    hipLaunchKernelGGL(k_count_zero, dim3(1), dim3(1024), 0, c->stream, c->pm, c->N, c->scal);
-    DG_HIP(c, hipGetLastError());
-    return DG_OK;
-}
-
 int dg_sum_into(dg_ctx *c, const double *v, long n, int slot) {
-    hipLaunchKernelGGL(k_sum2, dim3(1), dim3(1024), 0, c->stream, v, (const double *)nullptr, n,
-                       c->scal, slot);
+    hipLaunchKernelGGL(k_sum, dim3(1), dim3(1024), 0, c->stream, v, n, c->scal, slot);
     DG_HIP(c, hipGetLastError());
     return DG_OK;
 }

@@ -1,0 +1,50 @@
+"""The FP64 E-step at the edges of its tiles, against the CPU oracle.
+
+Sizes around the 16- and 64-point tiles, the 16-, 64- and 512-centre steps, the
+8- and 16-wide d steps and both ways pass 1 splits its work.  Both sides
+sum at most a few thousand FP64 terms of like size, and the exponents stay
+below 100 in magnitude, so they agree to about 100 * 2^-52 * a few: the bars
+are those of test_gpu_fp64.py (1e-11 on the qualities, 1e-10 on the sums)."""
+import numpy as np
+import pytest
+
+import dagtm_gpu as dg
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _problem(N, D, K, far=0):
+    rng = np.random.default_rng(1000 * N + 10 * D + K)
+    T = rng.normal(size=(N, D)) / np.sqrt(D)
+    Y = rng.normal(size=(K, D)) / np.sqrt(D)
+    T[:far] += 60.0                    # every exp underflows: zero columns
+    return T, Y, np.ones((K, 1)), 6.0
+
+
+@pytest.mark.parametrize("N,D,K,far", [
+    (1, 1, 1, 0), (2, 3, 5, 0), (15, 8, 63, 0), (16, 9, 64, 0), (17, 16, 65, 1),
+    (63, 17, 127, 0), (64, 24, 128, 0), (65, 25, 129, 2), (127, 31, 200, 0), (129, 33, 64, 0),
+    (1000, 65, 130, 3), (257, 96, 70, 0), (300, 145, 67, 0), (200, 161, 80, 0), (131, 176, 40, 1),
+    (90, 177, 66, 0), (333, 192, 100, 0),
+    (16500, 12, 1030, 5), (5001, 40, 515, 0),
+    (262143, 4, 17, 2), (262145, 5, 131, 1),            # either side of the split of pass 1
+])
+def test_estep_at_tile_edges(N, D, K, far):
+    print(f"case: N={N} D={D} K={K} far={far}", flush=True)
+    T, Y, FI, beta = _problem(N, D, K, far)
+    for isDA, temp in ((1, 1.7), (0, 1.0)):
+        m = O.Model(T, FI, Y, beta)
+        llh_o, nf_o, nz_o = m.estep(isDA, temp)
+        with dg.Engine(precision=dg.FP64) as e:
+            e.upload(T, FI, Y, beta)
+            llh, nf, nz = e.estep(isDA=isDA, temp=temp)
+            G, RT = e.stats()
+        assert nz == nz_o == far
+        if np.isfinite(llh_o):
+            assert llh == pytest.approx(llh_o, rel=1e-11, abs=1e-12)
+        else:
+            assert llh == llh_o
+        assert nf == pytest.approx(nf_o, rel=1e-11, abs=1e-12)
+        assert np.allclose(G, m.R.sum(1), rtol=1e-10, atol=1e-12)
+        assert np.allclose(RT, m.R @ T, rtol=1e-10, atol=1e-10)
