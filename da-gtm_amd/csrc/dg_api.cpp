@@ -120,7 +120,8 @@ int alloc_kstate(dg_ctx *c) {
     if ((rc = dalloc(c, &c->FI, (size_t)K * M1)) || (rc = dalloc(c, &c->Y64, (size_t)K * ld)) ||
         (rc = dalloc(c, &c->yy, K)) || (rc = dalloc(c, &c->G, K)) || (rc = dalloc(c, &c->Gm, K)) ||
         (rc = dalloc(c, &c->RT, (size_t)K * D)) ||
-        (rc = dalloc(c, &c->partRT, std::max((size_t)c->NC * K * D, dg_pass1_part(N)))) ||
+        (rc = dalloc(c, &c->partRT, std::max({(size_t)c->NC * K * D, dg_pass1_part(N),
+                                             dg_map_part(N, c->K)}))) ||
         (rc = dalloc(c, &c->partG, (size_t)c->NC * K + (size_t)3 * dg_pass1_wgs(N))) ||
         (rc = dalloc(c, &c->partAB, std::max((size_t)c->nchAB * ((size_t)M1 * M1 + (size_t)M1 * D),
                                              (size_t)(K + 63) / 64))))
@@ -371,6 +372,7 @@ int dg_estep(dg_ctx *c, int isDA, double temp, dg_estep_out *out) {
     if (isDA && !(temp > 0.0)) return dg_fail(c, DG_EINVAL, "dg_estep: temp must be > 0");
     int rc;
     if ((rc = select_device(c))) return rc;
+    c->fp64_due = false;
     if (c->mixed()) rc = dg_estep_mixed(c, isDA, temp);
     else rc = dg_estep_fp64(c, isDA, temp);
     if (rc) return rc;
@@ -395,11 +397,20 @@ int dg_estep(dg_ctx *c, int isDA, double temp, dg_estep_out *out) {
     return DG_OK;
 }
 
+// The FP64 outputs of a mixed context (dg_map, dg_next_ctemp, dg_resp_dense)
+// leave G and R T in FP64 for what reads them next, as the rest of their state:
+// computed here, when something does.
+static int due_stats(dg_ctx *c) {
+    if (!c->fp64_due) return DG_OK;
+    c->fp64_due = false;
+    return dg_estep_fp64(c, c->last_isDA, c->last_temp);
+}
+
 int dg_mstep(dg_ctx *c, double *beta_out) {
     if (!c) return DG_EINVAL;
     if (!c->loaded || !c->have_estep) return dg_fail(c, DG_ESTATE, "dg_mstep needs a dg_estep first");
     int rc;
-    if ((rc = select_device(c))) return rc;
+    if ((rc = select_device(c)) || (rc = due_stats(c))) return rc;
     // the G of this M-step is the one the critical-temperature search reads
     // (vggsub of dagtm.cxx:1715, still set when the next E-step converges)
     DG_HIP(c, hipMemcpyAsync(c->Gm, c->G, (size_t)c->K * sizeof(double),
@@ -571,8 +582,8 @@ static int next_ctemp_impl(dg_ctx *c, double temp, double eps, const double *gg,
     int rc;
     if ((rc = select_device(c))) return rc;
     // R in FP64: the mixed path refreshes the FP64 per-point normalisers
-    if (c->mixed() && (rc = dg_estep_fp64(c, c->last_isDA, c->last_temp)))
-        return rc;
+    c->fp64_due = c->mixed();
+    if (c->mixed() && (rc = dg_pass1_fp64(c, c->last_isDA, c->last_temp))) return rc;
     const int K = c->K, D = c->D;
     const long DD = (long)D * D;
     std::vector<double> g(K);
@@ -776,10 +787,7 @@ int dg_map(dg_ctx *c, const double *X, int L, long ldX, double *M, long ldM) {
         dg_estep_out eo;
         if ((rc = dg_estep(c, c->last_isDA, c->last_temp, &eo))) return rc;
     }
-    // output projections run in FP64; the mixed path refreshes the FP64
-    // per-point normalisers from the same model state first
-    if (c->mixed() && (rc = dg_estep_fp64(c, c->last_isDA, c->last_temp)))
-        return rc;
+    c->fp64_due = c->mixed();
     double *dX = nullptr, *dM = nullptr;
     if ((rc = dalloc(c, &dX, (size_t)c->K * L))) return rc;
     if ((rc = dalloc(c, &dM, (size_t)c->N * L))) { dfree(dX); return rc; }
@@ -787,7 +795,7 @@ int dg_map(dg_ctx *c, const double *X, int L, long ldX, double *M, long ldM) {
                                     (size_t)L * sizeof(double), (size_t)c->K,
                                     hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess) {
-        // the mixed path keeps its FP64 state current, so the FP64 kernel serves both
+        // the mixed path keeps its FP64 centres current, so the FP64 kernel serves both
         rc = dg_map_fp64(c, dX, L, dM);
         if (!rc)
             e = hipMemcpy2DAsync(M, (size_t)ldM * sizeof(double), dM, (size_t)L * sizeof(double),
@@ -818,7 +826,7 @@ int dg_map_noalloc(dg_ctx *c, const double *X, int L, long ldX, double *M, long 
         dg_estep_out eo;
         if ((rc = dg_estep(c, c->last_isDA, c->last_temp, &eo))) return rc;
     }
-    if (c->mixed() && (rc = dg_estep_fp64(c, c->last_isDA, c->last_temp))) return rc;
+    c->fp64_due = c->mixed();
     double *dX = c->map_scratch;                       // K x L
     double *dM = c->map_scratch + (size_t)c->K * L;    // N x L
     const size_t row = (size_t)L * sizeof(double);
@@ -843,8 +851,8 @@ int dg_resp_dense(dg_ctx *c, double *R, long ldR) {
     if (!R || ldR < c->N) return dg_fail(c, DG_EINVAL, "dg_resp_dense: bad args");
     int rc;
     if ((rc = select_device(c))) return rc;
-    if (c->mixed() && (rc = dg_estep_fp64(c, c->last_isDA, c->last_temp)))
-        return rc;
+    c->fp64_due = c->mixed();
+    if (c->mixed() && (rc = dg_pass1_fp64(c, c->last_isDA, c->last_temp))) return rc;
     double *dR = nullptr;
     if ((rc = dalloc(c, &dR, (size_t)c->K * c->N))) return rc;
     rc = dg_resp_dense_fp64(c, dR, c->N);
@@ -886,7 +894,7 @@ int dg_get_stats(dg_ctx *c, double *G, double *RT, long ldRT) {
     if (!c) return DG_EINVAL;
     if (!c->loaded || !c->have_estep) return dg_fail(c, DG_ESTATE, "dg_get_stats needs a dg_estep");
     int rc;
-    if ((rc = select_device(c))) return rc;
+    if ((rc = select_device(c)) || (rc = due_stats(c))) return rc;
     if (G)
         DG_HIP(c, hipMemcpyAsync(G, c->G, (size_t)c->K * sizeof(double), hipMemcpyDeviceToHost,
                                  c->stream));

@@ -129,138 +129,103 @@ __device__ __forceinline__ void put_logs(double lg, double lh, double zc,
     }
 }
 
+// ---- the cross terms of 64 points with the centres
 // 64 points (16 per wave) against the centres in tiles of 128: a wave holds
-// eight 16 x 16 accumulators.  The operands pass through LDS in 16-wide d
-// chunks, double buffered, the next chunk's loads in registers while one is
-// multiplied.  Lane (j, g) holds point j and rows 4 r + g of an accumulator.
-//   S = 1: the workgroup takes every centre, row i of accumulator a of tile t
-//          being centre 128 t + 16 a + i; the lane keeps slices 4 r + g and
-//          the workgroup finishes its points.
-//   S = 4: it takes the slices 4 q .. 4 q + 3, q = blockIdx.y, accumulator a
-//          of tile t holding those of the 64 centres from 64 (8 t + a) on (row
-//          i: centre 16 (i / 4) + 4 q + i % 4 of them); the lane keeps slice
-//          4 q + g, and k_e1_merge finishes the points.
-// Bound by the FP64 pipe, which the matrix instructions, the exponentials (two
-// per element away from temperature 1, left out where no term of a wave can
-// change its sum) and the exponents share: at N = 10^6, D = 166, K = 8000,
-// temperature 2, 62 ms, of which the 2 K N D flops take 35 at the pipe's measured
-// 77.7 TFLOP/s (4 x 4 register tiles of FMAs: 132 ms, their eight LDS reads per
-// 16 FMAs cost twice the pipe's time).  N = 1640, K = 5832: 0.26 ms (3.27).
+// eight 16 x 16 accumulators, whose lane (j, g) has point j and rows 4 r + g.
+// Row i of accumulator a of tile t is centre 128 t + 16 a + i (S = 1), or one of
+// the 64 centres from 64 (8 t + a) on, the (16 (i / 4) + 4 q + i % 4)-th (S = 4,
+// q4 = 4 q).  The operands pass through LDS in 16-wide d chunks, double
+// buffered, the next chunk's loads in registers while one is multiplied.
+// close(t, yt, na, acc) gets each finished tile of [t0, t1): yt its |y|^2 in LDS
+// (+inf past the last centre), na how many accumulators hold a centre.  With xs
+// (S = 1), xs[t & 1][q] holds the centres' X[k][q], 0 for q >= L and past the end.
 constexpr int P1 = 64, C1 = 128, RW = C1 / 16;
 
+struct CrossSmem {
+    double Ts[2][P1 * DCP];
+    double Ys[2][C1 * DCP];
+    double ys[2][C1];
+};
+
+// the centre in a row of a tile
 template <int S>
-__global__ __launch_bounds__(NT, 2) void k_e1_f64(
-    const double *__restrict__ T, const double *__restrict__ tt, long N,
-    const double *__restrict__ Y, const double *__restrict__ yy, int K, int D, int ld, double nbh,
-    PointOut po, double *__restrict__ partLog, double *__restrict__ part) {
+__device__ __forceinline__ int centre_of(int t, int row, int q4) {
+    const int i = row & 15;
+    return t * C1 * S + (row >> 4) * 16 * S + (S == 1 ? i : 16 * (i >> 2) + q4 + (i & 3));
+}
+
+template <int S, typename Close>
+__device__ __forceinline__ void cross_sweep(
+    CrossSmem &sm, const double *__restrict__ T, long N, const double *__restrict__ Y,
+    const double *__restrict__ yy, int K, int D, int ld, long n0, int t0, int t1, int q4,
+    Close &&close, const double *__restrict__ X = nullptr, int L = 0,
+    double (*xs)[3][C1] = nullptr) {
     constexpr int LT = P1 / 32, LY = C1 / 32;      // 16-byte loads per thread and chunk
     constexpr int CT = C1 * S;                     // centres from one tile to the next
     constexpr int CA = 16 * S;                     // from one accumulator to the next
-    __shared__ __attribute__((aligned(16))) double Ts[2][P1 * DCP];
-    __shared__ __attribute__((aligned(16))) double Ys[2][C1 * DCP];
-    __shared__ double ys[2][C1];
-    __shared__ double sm[3][NT / 64];
-
     const int tid = threadIdx.x, l = tid & 63, w = tid >> 6, j = l & 15, g = l >> 4;
-    const int q4 = 4 * blockIdx.y;
-    const long n0 = (long)blockIdx.x * P1, n = n0 + 16 * w + j;
-    const int ntiles = (K + CT - 1) / CT;
     const int nch = (D + DC - 1) / DC;                // d chunks per centre tile
     const int last8 = (D - (nch - 1) * DC + 7) / 8;   // 8-wide steps of the last one
-    const double it = po.it;
-    const int two = po.two;
-    auto centre = [&](int t, int row) {
-        const int i = row & 15;
-        return t * CT + (row >> 4) * CA + (S == 1 ? i : 16 * (i >> 2) + q4 + (i & 3));
-    };
-
     // staging: eight threads per row of a chunk, 16 bytes each; rows past the
-    // end repeat the last one (|y|^2 = +inf there, and no point is stored)
+    // end repeat the last one (|y|^2 = +inf there, and no point is stored).
+    // Scalar bases and 32-bit lane offsets that change once per tile at most: a
+    // vector instruction here holds up the FP64 matrix instructions of its SIMD.
     const int sr = tid >> 3, sp = tid & 7;
+    const double *Tw = T + n0 * ld;
+    unsigned ot[LT], oy[LY];
+#pragma unroll
+    for (int i = 0; i < LT; ++i) ot[i] = (unsigned)(min(n0 + sr + 32 * i, N - 1) - n0) * ld + 2 * sp;
+    auto at = [](const double *base, unsigned o) { return *(const d2 *)(base + o); };
     d2 rt[LT], ry[LY];
-    double ryy = INFINITY;
+    double ryy = INFINITY, rx[3] = {0.0, 0.0, 0.0};
     auto load = [&](int t, int q) {                    // tile t, d chunk q
+        if (q == 0) {
 #pragma unroll
-        for (int i = 0; i < LT; ++i)
-            rt[i] = *(const d2 *)(T + min(n0 + sr + 32 * i, N - 1) * ld + q * DC + 2 * sp);
+            for (int i = 0; i < LY; ++i)
+                oy[i] = (unsigned)min(centre_of<S>(t, sr + 32 * i, q4), K - 1) * ld + 2 * sp;
+            if (tid < C1) {
+                const int k = centre_of<S>(t, tid, q4);
+                ryy = (k < K) ? yy[k] : INFINITY;
+                if (xs)
 #pragma unroll
-        for (int i = 0; i < LY; ++i)
-            ry[i] = *(const d2 *)(Y + (long)min(centre(t, sr + 32 * i), K - 1) * ld + q * DC + 2 * sp);
-        if (q == 0 && tid < C1) {
-            const int k = centre(t, tid);
-            ryy = (k < K) ? yy[k] : INFINITY;
+                    for (int x = 0; x < 3; ++x) rx[x] = (k < K && x < L) ? X[(long)k * L + x] : 0.0;
+            }
         }
+#pragma unroll
+        for (int i = 0; i < LT; ++i) rt[i] = at(Tw + q * DC, ot[i]);
+#pragma unroll
+        for (int i = 0; i < LY; ++i) ry[i] = at(Y + q * DC, oy[i]);
     };
     auto store = [&](int b, int t, int q) {
 #pragma unroll
-        for (int i = 0; i < LT; ++i) put_pair(&Ts[b][(sr + 32 * i) * DCP], 2 * sp, rt[i]);
+        for (int i = 0; i < LT; ++i) put_pair(&sm.Ts[b][(sr + 32 * i) * DCP], 2 * sp, rt[i]);
 #pragma unroll
-        for (int i = 0; i < LY; ++i) put_pair(&Ys[b][(sr + 32 * i) * DCP], 2 * sp, ry[i]);
-        if (q == 0 && tid < C1) ys[t & 1][tid] = ryy;
+        for (int i = 0; i < LY; ++i) put_pair(&sm.Ys[b][(sr + 32 * i) * DCP], 2 * sp, ry[i]);
+        if (q == 0 && tid < C1) {
+            sm.ys[t & 1][tid] = ryy;
+            if (xs)
+#pragma unroll
+                for (int x = 0; x < 3; ++x) xs[t & 1][x][tid] = rx[x];
+        }
     };
-
-    const double tn = (n < N) ? tt[n] : 0.0;
-    Slice sl[S == 1 ? 4 : 1];
+    if (t0 >= t1) return;
     d4 acc[RW];
-    // slice s takes in the four centres it has of 64: exponents x of rows
-    // row0 + step i
-    auto take = [&](Slice &s, double (&x)[4], const double *yt, int row0, int step) {
-        double top = -INFINITY;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            x[i] = exponent(x[i], yt[row0 + step * i + g], tn, nbh);
-            top = fmax(top, x[i]);
-        }
-        s.raise(top, it, two);
-        // (-inf: nothing in the slice yet; its x are all -inf too)
-        const double m = (s.m == -INFINITY) ? 0.0 : s.m;
-        const double near = top - m;
-        if (__any(near > kNoTerm)) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) s.s1 += exp(x[i] - m);
-        }
-        if (two && __any(near * it > kNoTerm)) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) s.s2 += exp((x[i] - m) * it);
-        }
-    };
-    auto close_tile = [&](const double *yt, int na) {
-        if (S == 1) {
-#pragma unroll
-            for (int h = 0; h < RW; h += 4)
-                if (h < na)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        double x[4] = {acc[h][r], acc[h + 1][r], acc[h + 2][r], acc[h + 3][r]};
-                        take(sl[S == 1 ? r : 0], x, yt, 16 * h + 4 * r, 16);
-                    }
-        } else {
-#pragma unroll
-            for (int a = 0; a < RW; ++a)
-                if (a < na) {
-                    double x[4] = {acc[a][0], acc[a][1], acc[a][2], acc[a][3]};
-                    take(sl[0], x, yt, 16 * a, 4);
-                }
-        }
-    };
-
-    load(0, 0);
-    store(0, 0, 0);
+    load(t0, 0);
+    store(0, t0, 0);
     __syncthreads();
     int b = 0;
-    for (int t = 0; t < ntiles; ++t) {
-        // accumulators of this tile that hold a centre
+    for (int t = t0; t < t1; ++t) {
         const int na = min(RW, (K - t * CT + CA - 1) / CA);
 #pragma unroll
         for (int a = 0; a < RW; ++a) acc[a] = d4{0.0, 0.0, 0.0, 0.0};
         for (int q = 0; q < nch; ++q, b ^= 1) {
             const int tq = (q + 1 < nch) ? t : t + 1, qn = (q + 1 < nch) ? q + 1 : 0;
-            const bool more = tq < ntiles;
+            const bool more = tq < t1;
             if (more) load(tq, qn);
             const int steps = (q + 1 < nch) ? DC / 8 : last8;
             for (int s = 0; s < steps; ++s) {
-                const double *yr = &Ys[b][j * DCP + 8 * s + 2 * g];
-                const d2 bv = *(const d2 *)&Ts[b][(16 * w + j) * DCP + 8 * s + 2 * g];
+                const double *yr = &sm.Ys[b][j * DCP + 8 * s + 2 * g];
+                const d2 bv = *(const d2 *)&sm.Ts[b][(16 * w + j) * DCP + 8 * s + 2 * g];
                 if (na == RW) {
                     // the centre rows' operands are read one step ahead of
                     // their MFMAs (the sched_barrier keeps them there)
@@ -286,10 +251,83 @@ __global__ __launch_bounds__(NT, 2) void k_e1_f64(
             if (more) store(b ^ 1, tq, qn);
             // (before the barrier: the next tile's |y|^2 goes to the other
             // half of ys, the one after it only past this barrier)
-            if (q + 1 == nch) close_tile(ys[t & 1], na);
+            if (q + 1 == nch) {
+                // (opaque: else what close derives from t is computed, and kept
+                // in registers, before the chunk loop)
+                int tc = t;
+                asm volatile("" : "+s"(tc));
+                close(tc, sm.ys[tc & 1], na, acc);
+            }
             __syncthreads();
         }
     }
+}
+
+// Pass 1.  S = 1: the workgroup takes every centre, its lanes keep slices
+// 4 r + g, and it finishes its points.  S = 4: it takes the slices 4 q .. 4 q + 3,
+// q = blockIdx.y, its lanes keep slice 4 q + g, and k_e1_merge finishes the points.
+// Bound by the FP64 pipe, which the matrix instructions, the exponentials (two
+// per element away from temperature 1, left out where no term of a wave can
+// change its sum) and the exponents share: at N = 10^6, D = 166, K = 8000,
+// temperature 2, 62 ms, of which the 2 K N D flops take 35 at the pipe's measured
+// 77.7 TFLOP/s (4 x 4 register tiles of FMAs: 132 ms, their eight LDS reads per
+// 16 FMAs cost twice the pipe's time).  N = 1640, K = 5832: 0.26 ms (3.27).
+template <int S>
+__global__ __launch_bounds__(NT, 2) void k_e1_f64(
+    const double *__restrict__ T, const double *__restrict__ tt, long N,
+    const double *__restrict__ Y, const double *__restrict__ yy, int K, int D, int ld, double nbh,
+    PointOut po, double *__restrict__ partLog, double *__restrict__ part) {
+    __shared__ __attribute__((aligned(16))) CrossSmem cs;
+    __shared__ double sm[3][NT / 64];
+    const int tid = threadIdx.x, l = tid & 63, w = tid >> 6, j = l & 15, g = l >> 4;
+    const int q4 = 4 * blockIdx.y;
+    const long n0 = (long)blockIdx.x * P1, n = n0 + 16 * w + j;
+    const double it = po.it;
+    const int two = po.two;
+    const double tn = (n < N) ? tt[n] : 0.0;
+    Slice sl[S == 1 ? 4 : 1];
+    // slice s takes in the four centres it has of 64: exponents x of rows
+    // row0 + step i
+    auto take = [&](Slice &s, double (&x)[4], const double *yt, int row0, int step) {
+        double top = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            x[i] = exponent(x[i], yt[row0 + step * i + g], tn, nbh);
+            top = fmax(top, x[i]);
+        }
+        s.raise(top, it, two);
+        // (-inf: nothing in the slice yet; its x are all -inf too)
+        const double m = (s.m == -INFINITY) ? 0.0 : s.m;
+        const double near = top - m;
+        if (__any(near > kNoTerm)) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s.s1 += exp(x[i] - m);
+        }
+        if (two && __any(near * it > kNoTerm)) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s.s2 += exp((x[i] - m) * it);
+        }
+    };
+    cross_sweep<S>(cs, T, N, Y, yy, K, D, ld, n0, 0, (K + C1 * S - 1) / (C1 * S), q4,
+                   [&](int, const double *yt, int na, d4 (&acc)[RW]) {
+        if (S == 1) {
+#pragma unroll
+            for (int h = 0; h < RW; h += 4)
+                if (h < na)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        double x[4] = {acc[h][r], acc[h + 1][r], acc[h + 2][r], acc[h + 3][r]};
+                        take(sl[S == 1 ? r : 0], x, yt, 16 * h + 4 * r, 16);
+                    }
+        } else {
+#pragma unroll
+            for (int a = 0; a < RW; ++a)
+                if (a < na) {
+                    double x[4] = {acc[a][0], acc[a][1], acc[a][2], acc[a][3]};
+                    take(sl[0], x, yt, 16 * a, 4);
+                }
+        }
+    });
     if (S == 4) {
         if (n < N) {
             double *o = part + (long)(q4 + g) * 3 * N + n;
@@ -407,11 +445,13 @@ __global__ __launch_bounds__(NT, 2) void k_e2_f64(
     if (sr >= 2) psrc = pl;
     const double pend = (sr == 1) ? INFINITY : 0.0;   // past the end: x_max = +inf, so R = 0
     auto half_load = [&](int h, long n0) {
-        const double *src = T + min(n0 + sr, ne - 1) * ld + 2 * sp;
+        // (a scalar base and a 32-bit lane offset, as in cross_sweep)
+        const double *base = T + n0 * ld;
+        const unsigned o = (unsigned)min(sr, (int)min(ne - 1 - n0, 15L)) * ld + 2 * sp;
 #pragma unroll
         for (int i = 0; i < H; ++i) {
             const int f = h * H + i;
-            if (f < NL && (f < NL - 1 || tail)) rt[i] = *(const d2 *)(src + 32 * f);
+            if (f < NL && (f < NL - 1 || tail)) rt[i] = *(const d2 *)(base + 32 * f + o);
         }
         if (h == 0) {
             const double v = psrc[min(n0 + sp, ne - 1)];
@@ -549,51 +589,133 @@ __global__ __launch_bounds__(256) void k_reduce_parts(
     else if (i < KD + K) G[i - KD] = sum(partG + (i - KD), K);
 }
 
-// ---------------------------------------------------------------- debug / MAP
-// One thread per (k, n): R_kn from the pass-1 normaliser.
-__global__ void k_resp_dense(const double *__restrict__ T, const double *__restrict__ tt, long N,
-                             const double *__restrict__ Y, const double *__restrict__ yy, int K,
-                             int ld, double nbh, double it, double invK,
-                             const double *__restrict__ pm, const double *__restrict__ pl,
-                             double *__restrict__ R, long ldR) {
-    const long n = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int k = blockIdx.y;
-    if (n >= N) return;
-    double r;
-    if (pm[n] == -INFINITY) {
-        r = invK;
-    } else {
-        double s = 0.0;
-        for (int d = 0; d < ld; ++d) s = fma(T[n * ld + d], Y[(long)k * ld + d], s);
-        const double x = exponent(s, yy[k], tt[n], nbh);
-        r = (x != -INFINITY) ? exp((x - pm[n]) * it - pl[n]) : 0.0;
-    }
-    R[(long)k * ldR + n] = r;
+// ---------------------------------------------------------------- dense R, MAP
+// R_kn of the centres from k0 = 0 .. K - 1 (K, Y and yy of a range of them) from
+// the pass-1 normalisers, to R[k ldR + n].  Workgroup (point tile, range of
+// tiles_per centre tiles).  Bound by the FP64 pipe for D beyond a few, else by
+// the 8 K N bytes it writes: N = 6007, D = 12, K = 900 in 22 us (one thread per
+// element over D, its row uncoalesced: 289).
+__global__ __launch_bounds__(NT, 2) void k_resp_dense(
+    const double *__restrict__ T, const double *__restrict__ tt, long N,
+    const double *__restrict__ Y, const double *__restrict__ yy, int K, int D, int ld, double nbh,
+    double it, double invK, const double *__restrict__ pm, const double *__restrict__ pl,
+    int tiles_per, double *__restrict__ R, long ldR) {
+    __shared__ __attribute__((aligned(16))) CrossSmem cs;
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6, j = l & 15, g = l >> 4;
+    const long n0 = (long)blockIdx.x * P1, n = n0 + 16 * w + j, nn = min(n, N - 1);
+    const int t0 = blockIdx.y * tiles_per, t1 = min((K + C1 - 1) / C1, t0 + tiles_per);
+    const double tn = tt[nn], m = pm[nn], ls = pl[nn];
+    const long off = g * ldR + 16 * w + j;
+    cross_sweep<1>(cs, T, N, Y, yy, K, D, ld, n0, t0, t1, 0,
+                   [&](int t, const double *yt, int na, d4 (&acc)[RW]) {
+#pragma unroll
+        for (int a = 0; a < RW; ++a)
+            if (a < na) {
+                double v[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const double x = exponent(acc[a][r], yt[16 * a + 4 * r + g], tn, nbh);
+                    v[r] = exp((x - m) * it - ls);
+                    asm volatile("" : "+v"(v[r]));             // (no branch around it)
+                }
+                const int k = t * C1 + 16 * a;
+                double *row = R + (long)k * ldR + n0;          // (wave-uniform)
+#pragma unroll
+                for (int r = 0; r < 4; ++r, row += 4 * ldR)
+                    if (k + 4 * r + g < K && n < N) row[off] = (m == -INFINITY) ? invK : v[r];
+            }
+    });
 }
 
-// MAP: M[n][l] = sum_k R_kn X[k][l], one thread per point (L <= 3).
-__global__ void k_map_f64(const double *__restrict__ T, const double *__restrict__ tt, long N,
-                          const double *__restrict__ Y, const double *__restrict__ yy, int K,
-                          int ld, double nbh, double it, double invK,
-                          const double *__restrict__ pm, const double *__restrict__ pl,
-                          const double *__restrict__ X, int L, double *__restrict__ M) {
-    const long n = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= N) return;
-    double acc[3] = {0.0, 0.0, 0.0};
-    const bool zc = pm[n] == -INFINITY;
-    for (int k = 0; k < K; ++k) {
-        double r;
-        if (zc) {
-            r = invK;
-        } else {
-            double s = 0.0;
-            for (int d = 0; d < ld; ++d) s = fma(T[n * ld + d], Y[(long)k * ld + d], s);
-            const double x = exponent(s, yy[k], tt[n], nbh);
-            r = (x != -INFINITY) ? exp((x - pm[n]) * it - pl[n]) : 0.0;
+// MAP in one pass: per point the online sums of p = exp((x - m) / temp) and of
+// p X[k][l] (L <= 3) over a range of centres; k_map_merge makes M = sum p X /
+// sum p of them.  No normaliser is needed beforehand, so a projection costs one
+// pass over the K x N distances in either precision.  part[(5 range + f) N + n]:
+// m, sum p, and the three sums.  FP64 pipe: 2 K N D flops, K N exponentials.
+// N = 30011, D = 166, K = 8000: 1.95 ms (one thread per point over all centres,
+// after two FP64 passes for its normaliser: 497).
+__global__ __launch_bounds__(NT, 2) void k_map_f64(
+    const double *__restrict__ T, const double *__restrict__ tt, long N,
+    const double *__restrict__ Y, const double *__restrict__ yy, int K, int D, int ld, double nbh,
+    double it, int tiles_per, const double *__restrict__ X, int L, double *__restrict__ part) {
+    __shared__ __attribute__((aligned(16))) CrossSmem cs;
+    __shared__ double xs[2][3][C1];
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6, j = l & 15, g = l >> 4;
+    const long n0 = (long)blockIdx.x * P1, n = n0 + 16 * w + j;
+    const int t0 = blockIdx.y * tiles_per, t1 = min((K + C1 - 1) / C1, t0 + tiles_per);
+    const double tn = tt[min(n, N - 1)];
+    double m = -INFINITY, s = 0.0, ax[3] = {0.0, 0.0, 0.0};
+    auto take = [&](int t, int a, const double *yt, const d4 &c) {
+        double x[4], top = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            x[r] = exponent(c[r], yt[16 * a + 4 * r + g], tn, nbh);
+            top = fmax(top, x[r]);
         }
-        for (int l = 0; l < L; ++l) acc[l] = fma(r, X[(long)k * L + l], acc[l]);
+        if (top > m) {                             // new running max: rescale the sums
+            const double f = exp((m - top) * it);
+            s *= f;
+#pragma unroll
+            for (int q = 0; q < 3; ++q) ax[q] *= f;
+            m = top;
+        }
+        const double ms = (m == -INFINITY) ? 0.0 : m;
+        // (the sum is at least 1, and all that is left out of it below 2^-66)
+        if (__any((top - ms) * it > -60.0)) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const double v = exp((x[r] - ms) * it);
+                s += v;
+#pragma unroll
+                for (int q = 0; q < 3; ++q) ax[q] = fma(v, xs[t & 1][q][16 * a + 4 * r + g], ax[q]);
+            }
+        }
+    };
+    cross_sweep<1>(cs, T, N, Y, yy, K, D, ld, n0, t0, t1, 0,
+                   [&](int t, const double *yt, int na, d4 (&acc)[RW]) {
+#pragma unroll
+        for (int a = 0; a < RW; ++a)
+            if (a < na) take(t, a, yt, acc[a]);
+    }, X, L, xs);
+    // the four lanes j, j + 16, j + 32, j + 48 hold the same point
+    double M = fmax(m, __shfl_xor(m, 16));
+    M = fmax(M, __shfl_xor(M, 32));
+    const double f = exp((M == -INFINITY) ? 0.0 : (m - M) * it);
+    double v[4] = {s * f, ax[0] * f, ax[1] * f, ax[2] * f};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        v[q] += __shfl_xor(v[q], 16);
+        v[q] += __shfl_xor(v[q], 32);
     }
-    for (int l = 0; l < L; ++l) M[n * L + l] = acc[l];
+    if (g == 0 && n < N) {
+        double *o = part + 5L * blockIdx.y * N + n;
+        o[0] = M;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) o[(q + 1) * N] = v[q];
+    }
+}
+
+__global__ __launch_bounds__(NT) void k_map_merge(const double *__restrict__ part, int ranges,
+                                                  long N, double it, int K, double invK,
+                                                  const double *__restrict__ X, int L,
+                                                  double *__restrict__ M) {
+    const long n = (long)blockIdx.x * NT + threadIdx.x;
+    if (n >= N) return;
+    double top = -INFINITY, v[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int c = 0; c < ranges; ++c) top = fmax(top, part[5L * c * N + n]);
+    if (top == -INFINITY) {                        // zero column: R = 1/K
+        v[0] = 1.0;
+        for (int k = 0; k < K; ++k)
+            for (int q = 0; q < L; ++q) v[q + 1] = fma(invK, X[(long)k * L + q], v[q + 1]);
+    } else {
+        for (int c = 0; c < ranges; ++c) {
+            const double *p = part + 5L * c * N + n;
+            const double f = exp((p[0] - top) * it);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[q] = fma(p[(q + 1) * N], f, v[q]);
+        }
+    }
+    for (int q = 0; q < L; ++q) M[n * L + q] = v[q + 1] / v[0];
 }
 
 // f(std::integral_constant<int, DB>) for DB = db in 1 .. 12, false otherwise
@@ -776,12 +898,26 @@ int dg_estep_fp64(dg_ctx *c, int isDA, double temp) {
     return DG_OK;
 }
 
+// k_resp_dense and k_map_f64 split the centre tiles into ranges until there are
+// about 2048 workgroups (two are resident on each of 256 CUs)
+struct Ranges {
+    int tiles_per, count;
+};
+static Ranges centre_ranges(long N, int K) {
+    const long pt = (N + P1 - 1) / P1, ct = (K + C1 - 1) / C1;
+    const long want = std::max(1L, std::min(ct, (2048 + pt - 1) / pt));
+    const int per = (int)((ct + want - 1) / want);
+    return {per, (int)((ct + per - 1) / per)};
+}
+
+size_t dg_map_part(long N, int K) { return (size_t)5 * N * centre_ranges(N, K).count; }
+
 int dg_resp_dense_fp64(dg_ctx *c, double *dR, long ldR) {
     const double it = c->last_isDA ? 1.0 / c->last_temp : 1.0;
-    dim3 grid((unsigned)((c->N + 255) / 256), (unsigned)c->K);
-    hipLaunchKernelGGL(k_resp_dense, grid, dim3(256), 0, c->stream, c->T64, c->tt, c->N, c->Y64,
-                       c->yy, c->K, c->ldt, -c->beta / 2.0, it, 1.0 / c->K, c->pm, c->pl, dR,
-                       ldR);
+    const Ranges r = centre_ranges(c->N, c->K);
+    hipLaunchKernelGGL(k_resp_dense, dim3((unsigned)((c->N + P1 - 1) / P1), (unsigned)r.count),
+                       dim3(NT), 0, c->stream, c->T64, c->tt, c->N, c->Y64, c->yy, c->K, c->D,
+                       c->ldt, -c->beta / 2.0, it, 1.0 / c->K, c->pm, c->pl, r.tiles_per, dR, ldR);
     DG_HIP(c, hipGetLastError());
     return DG_OK;
 }
@@ -807,9 +943,13 @@ int dg_ctemp_moments_fp64(dg_ctx *c, int k0, int KB, int nc, double *dPart, doub
 
 int dg_map_fp64(dg_ctx *c, const double *dX, int L, double *dM) {
     const double it = c->last_isDA ? 1.0 / c->last_temp : 1.0;
-    hipLaunchKernelGGL(k_map_f64, dim3((unsigned)((c->N + 255) / 256)), dim3(256), 0, c->stream,
-                       c->T64, c->tt, c->N, c->Y64, c->yy, c->K, c->ldt, -c->beta / 2.0, it,
-                       1.0 / c->K, c->pm, c->pl, dX, L, dM);
+    const Ranges r = centre_ranges(c->N, c->K);
+    hipLaunchKernelGGL(k_map_f64, dim3((unsigned)((c->N + P1 - 1) / P1), (unsigned)r.count), dim3(NT),
+                       0, c->stream, c->T64, c->tt, c->N, c->Y64, c->yy, c->K, c->D, c->ldt,
+                       -c->beta / 2.0, it, r.tiles_per, dX, L, c->partRT);
+    DG_HIP(c, hipGetLastError());
+    hipLaunchKernelGGL(k_map_merge, dim3((unsigned)((c->N + NT - 1) / NT)), dim3(NT), 0, c->stream,
+                       c->partRT, r.count, c->N, it, c->K, 1.0 / c->K, dX, L, dM);
     DG_HIP(c, hipGetLastError());
     return DG_OK;
 }

@@ -27,6 +27,8 @@ struct dg_ctx {
     int D = 0, K = 0, M1 = 0;
     bool loaded = false;
     bool have_estep = false;       // G/RT/pm/pl valid for the current Y
+    bool fp64_due = false;         // mixed: an FP64 output was made from this E-step, so the
+                                   // next reader of G and R T gets them from an FP64 E-step
     bool have_w = false;           // W holds the last M-step's (or a caller's) weights
     bool last_isDA = true;
     double last_temp = 1.0;
@@ -51,7 +53,8 @@ struct dg_ctx {
     double *pl = nullptr;          // N   per-point log S2 (pass 1)
     double *logg = nullptr;        // N
     double *logh = nullptr;        // N
-    double *partRT = nullptr;      // NC x K x D; before pass 2, pass 1's slice states
+    double *partRT = nullptr;      // NC x K x D; also pass 1's slice states (before
+                                   // pass 2) and the projection's sums
     double *partG = nullptr;       // NC x K
     double *partLog64 = nullptr;   // pass 1's log sums, 3 per workgroup (behind partG)
     int NC = 1;                    // N chunks of E-pass 2
@@ -224,7 +227,9 @@ int dg_hip_check(dg_ctx *ctx, hipError_t e, const char *what);
 // ---- FP64 kernels (dg_fp64.hip) ----
 long dg_pass1_wgs(long N);        // workgroups that sum pass 1's logs
 size_t dg_pass1_part(long N);     // doubles of partRT that pass 1 needs for its states
+size_t dg_map_part(long N, int K);   // doubles of partRT that dg_map_fp64 needs
 int dg_estep_fp64(dg_ctx *ctx, int isDA, double temp);
+int dg_pass1_fp64(dg_ctx *ctx, int isDA, double temp);   // its first half: pm, pl, log g, log h
 int dg_resp_dense_fp64(dg_ctx *ctx, double *dR, long ldR);
 int dg_map_fp64(dg_ctx *ctx, const double *dX, int L, double *dM);
 // S1, S2 of centres k0 .. k0+KB-1 into dS (KB x 2 x D x D, lower triangle

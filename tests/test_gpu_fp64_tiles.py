@@ -48,3 +48,31 @@ def test_estep_at_tile_edges(N, D, K, far):
         assert nf == pytest.approx(nf_o, rel=1e-11, abs=1e-12)
         assert np.allclose(G, m.R.sum(1), rtol=1e-10, atol=1e-12)
         assert np.allclose(RT, m.R @ T, rtol=1e-10, atol=1e-10)
+
+
+@pytest.mark.parametrize("N,D,K,far,L", [
+    (1, 1, 1, 0, 1), (15, 8, 63, 1, 2), (64, 17, 128, 0, 3), (65, 25, 129, 2, 1), (1000, 40, 1100, 3, 2),
+    (333, 192, 100, 0, 3), (9000, 12, 300, 4, 2),
+])
+def test_outputs_at_tile_edges(N, D, K, far, L):
+    """Projection and dense R (always FP64) in both precisions, and G and R T
+    read after them, against the oracle: R at most 1 and K of them to a sum, so
+    1e-12 on R and 1e-11 on the projection of coordinates in [-1, 1]."""
+    print(f"case: N={N} D={D} K={K} far={far} L={L}", flush=True)
+    T, Y, FI, beta = _problem(N, D, K, far)
+    X = np.random.default_rng(N + K).uniform(-1.0, 1.0, (K, L))
+    m = O.Model(T, FI, Y, beta)
+    m.estep(1, 1.7)
+    for prec in (dg.FP64, dg.MIXED):
+        if prec == dg.MIXED and D > 128:
+            continue                   # float data: the mixed path stops at 128
+        with dg.Engine(precision=prec) as e:
+            e.upload(T, FI, Y, beta)
+            e.estep(True, 1.7)
+            assert np.abs(e.map(X) - m.R.T @ X).max() < 1e-11
+            assert np.abs(e.map_noalloc(X) - m.R.T @ X).max() < 1e-11
+            G, RT = e.stats()
+            assert np.abs(e.resp_dense() - m.R).max() < 1e-12
+            assert np.array_equal(G, e.stats()[0])
+        assert np.allclose(G, m.R.sum(1), rtol=1e-10, atol=1e-12)
+        assert np.allclose(RT, m.R @ T, rtol=1e-10, atol=1e-10)
