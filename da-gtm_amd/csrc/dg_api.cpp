@@ -584,9 +584,8 @@ static int next_ctemp_impl(dg_ctx *c, double temp, double eps, const double *gg,
     // R in FP64: the mixed path refreshes the FP64 per-point normalisers
     c->fp64_due = c->mixed();
     if (c->mixed() && (rc = dg_pass1_fp64(c, c->last_isDA, c->last_temp))) return rc;
-    const int K = c->K, D = c->D;
-    const long DD = (long)D * D;
-    std::vector<double> g(K);
+    const int K = c->K;
+    std::vector<double> g(K), ck(K);
     if (gg) {
         std::copy(gg, gg + K, g.begin());
     } else {
@@ -594,73 +593,35 @@ static int next_ctemp_impl(dg_ctx *c, double temp, double eps, const double *gg,
                                  hipMemcpyDeviceToHost, c->stream));
         DG_HIP(c, hipStreamSynchronize(c->stream));
     }
-    // centres per batch: S1 and S2 of a batch take at most 256 MB
-    const int KB = (int)std::max(1L, std::min((long)K, (1L << 25) / (2 * DD)));
-    const int nt = (D + 63) / 64, pairs = nt * (nt + 1) / 2;
-    const long tiles = (c->N + 63) / 64;
-    long nc = (2048 + (long)pairs * KB - 1) / ((long)pairs * KB);
-    nc = std::max(1L, std::min({nc, 64L, tiles}));
-    const size_t slen = (size_t)KB * 2 * DD;
-    DevBuf bPart, bS;
-    if ((rc = dalloc(c, &bPart.p, slen * nc))) return rc;
-    if (nc > 1 && (rc = dalloc(c, &bS.p, slen))) return rc;
-    double *dPart = bPart.p, *dS = bS.p;
-    std::vector<double> hS(slen), ck(K);
-    const double GG_MIN = 1e-250;   // mpicomm.c:617-628
-    int bad = 0;
-    unsigned nth = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
-    for (int k0 = 0; k0 < K && !rc; k0 += KB) {
-        const int kb = std::min(KB, K - k0);
-        rc = dg_ctemp_moments_fp64(c, k0, kb, (int)nc, dPart, nc > 1 ? dS : dPart);
-        hipError_t e = hipSuccess;
-        if (!rc) e = hipMemcpyAsync(hS.data(), nc > 1 ? dS : dPart, (size_t)kb * 2 * DD * sizeof(double),
-                                    hipMemcpyDeviceToHost, c->stream);
-        if (!rc && e == hipSuccess) e = hipStreamSynchronize(c->stream);
-        if (e != hipSuccess) rc = dg_hip_check(c, e, "dg_next_ctemp");
-        if (rc) break;
-        // per centre: eig(H) of mpicomm.c:599-626 with H = [[2S1 - S2, -S2], [-S2, 2S1 - S2]]
-        // is eig(2 S1) together with eig(2 S1 - 2 S2) (H is block-symmetric)
-        std::atomic<int> fail{0};
-        auto work = [&](unsigned t) noexcept {
-            std::vector<double> A, w;
-            try {
-                A.resize((size_t)DD);
-                w.resize(D);
-            } catch (...) {
-                fail.fetch_or(2);
-                return;
-            }
-            for (int i = (int)t; i < kb; i += (int)nth) {
-                const int k = k0 + i;
-                if (g[k] == 0.0) { ck[k] = HUGE_VAL; continue; }
-                const double *S1 = hS.data() + (size_t)i * 2 * DD, *S2 = S1 + DD;
-                const double sc = g[k] < GG_MIN ? 1.0 / GG_MIN : 1.0;
-                const double limit = (temp - eps) * g[k] * 2.0 / c->beta;
-                double lmax = -HUGE_VAL;
-                for (int part = 0; part < 2; ++part) {
-                    for (int a = 0; a < D; ++a)
-                        for (int b = 0; b <= a; ++b) {
-                            const double s1 = 2.0 * S1[(size_t)a * D + b];
-                            const double v = part ? s1 - 2.0 * S2[(size_t)a * D + b] : s1;
-                            A[(size_t)a * D + b] = v * sc;
-                        }
-                    const int er = dg_sym_eigvals(D, A.data(), D, w.data());
-                    if (er) { fail.fetch_or(er == 2 ? 2 : 1); return; }
-                    for (int j = 0; j < D; ++j) {
-                        const double l = (w[j] / sc >= limit) ? 0.0 : w[j] / sc;   // comm.c:2149-2161
-                        if (l > lmax) lmax = l;
-                    }
-                }
-                ck[k] = c->beta / 2.0 / g[k] * lmax;
-            }
-        };
-        run_threads(nth, work);
-        bad |= fail.load();
+    // per centre: eig(H) of mpicomm.c:599-626 with H = [[2S1 - S2, -S2], [-S2, 2S1 - S2]]
+    // is eig(2 S1) together with eig(2 S1 - 2 S2) (H is block-symmetric).  A
+    // centre of hardly any weight has its matrices scaled up (mpicomm.c:617-628).
+    const double GG_MIN = 1e-250;
+    const DgCtempPlan p = dg_ctemp_plan(c);
+    std::vector<double> lim((size_t)2 * K), val((size_t)2 * K);
+    for (int k0 = 0; k0 < K; k0 += p.KB) {
+        const int kb = std::min(p.KB, K - k0);
+        for (int i = 0; i < kb; ++i) {
+            lim[(size_t)2 * k0 + i] = (temp - eps) * g[k0 + i] * 2.0 / c->beta;
+            lim[(size_t)2 * k0 + kb + i] = g[k0 + i] == 0.0 ? 0.0 : g[k0 + i] < GG_MIN ? 1.0 / GG_MIN : 1.0;
+        }
     }
-    if (rc) return rc;
-    // bit 1: an eigenvalue iteration did not converge; bit 2: host allocation failed
-    if (bad & 2) return dg_fail(c, DG_ENOMEM, "dg_next_ctemp: host allocation failed");
-    if (bad & 1) return dg_fail(c, DG_ESOLVE, "dg_next_ctemp: eigenvalue iteration did not converge");
+    DevBuf buf;
+    if ((rc = dalloc(c, &buf.p, p.buf_len() + (size_t)4 * K))) return rc;
+    double *dLim = buf.p + p.buf_len(), *dVal = dLim + (size_t)2 * K;
+    DG_HIP(c, hipMemcpyAsync(dLim, lim.data(), (size_t)2 * K * sizeof(double), hipMemcpyHostToDevice,
+                             c->stream));
+    for (int k0 = 0; k0 < K; k0 += p.KB)
+        if ((rc = dg_ctemp_fp64(c, k0, std::min(p.KB, K - k0), p, dLim, buf.p, dVal))) return rc;
+    DG_HIP(c, hipMemcpyAsync(val.data(), dVal, (size_t)2 * K * sizeof(double), hipMemcpyDeviceToHost,
+                             c->stream));
+    DG_HIP(c, hipStreamSynchronize(c->stream));
+    for (int k = 0; k < K; ++k) {
+        const double a = val[(size_t)2 * k], b = val[(size_t)2 * k + 1];
+        if (g[k] != 0.0 && (std::isnan(a) || std::isnan(b)))
+            return dg_fail(c, DG_ESOLVE, "dg_next_ctemp: no eigenvalues (data not finite)");
+        ck[k] = g[k] == 0.0 ? HUGE_VAL : c->beta / 2.0 / g[k] * std::max(a, b);
+    }
     double cmax = -HUGE_VAL;
     for (int k = 0; k < K; ++k) cmax = std::max(cmax, ck[k]);
     *ctemp_max = cmax;

@@ -733,95 +733,116 @@ bool with_db(int db, F &&f) {
 // ---------------------------------------------------------------- critical temperature
 // Responsibility-weighted second moments of the data centred on one centre,
 // S1 = sum_n r_kn x x^T and S2 = sum_n r_kn^2 x x^T with x = t_n - y_k (the
-// 2 S1 and -S2 of mpicomm.c:580-597).  One workgroup per (64 x 64 tile of the
-// lower triangle, centre k0 + blockIdx.y, N chunk); R_kn is recomputed with
-// k_resp_dense's formula.  Each thread owns a 4 x 4 micro-tile of both sums,
-// accumulated over the chunk's points in order.  The chunk's partial goes to
-// part[((chunk * KB + kb) * 2 + s) * D * D + a * D + b] for the tile only.
-constexpr int CM = 64;   // moment tile edge
+// 2 S1 and -S2 of mpicomm.c:580-597), r_kn = R[k N + n] of k_resp_dense.  One
+// workgroup per (tile pair of the lower triangle, centre, N chunk); a tile is
+// 16 RB wide and its waves take sixteen points in turn, straight from global
+// memory: a lane's operands of four points are r x and r^2 x of its row and x of
+// its column.  The waves' sums are added in order, and the chunk's partial goes
+// to part[((chunk * KB + kb) * 2 + s) * D * D + a * D + b].
+// Bound by the FP64 pipe: 4 flops for each entry, point and centre.  N = 5003,
+// D = 32, K = 400: 158 us with R (4 x 4 tiles of FMAs from LDS and one thread per
+// point for its R: 1107 us).  D = 166: 69 % of the pipe's rate.
+// diag: the pair's columns are its rows, and its upper tiles are not wanted.
+template <int RB, bool diag>
+__device__ __forceinline__ void moments_body(
+    double (*red)[2 * RB * RB][256], const int ti, const int tj, const double *__restrict__ T, long N,
+    const double *__restrict__ Y, int D, int ld, const double *__restrict__ R, long chunk,
+    double *__restrict__ part) {
+    const int tid = threadIdx.x, l = tid & 63, w = tid >> 6, j = l & 15, g = l >> 4;
+    const long kb = blockIdx.y;
+    const long n0 = (long)blockIdx.z * chunk, n1 = min(N, n0 + chunk);
+    // (columns past the row's end repeat its last one; their results are not stored)
+    int ca[RB], cb[RB];
+    double ya[RB], yb[RB];
+#pragma unroll
+    for (int x = 0; x < RB; ++x) {
+        ca[x] = min(16 * (RB * ti + x) + j, ld - 1);
+        cb[x] = min(16 * (RB * tj + x) + j, ld - 1);
+        ya[x] = Y[kb * ld + ca[x]];
+        yb[x] = Y[kb * ld + cb[x]];
+    }
+    const double *r = R + kb * N;
+    d4 s1[RB][RB], s2[RB][RB];
+#pragma unroll
+    for (int x = 0; x < RB; ++x)
+#pragma unroll
+        for (int y = 0; y < RB; ++y) s1[x][y] = s2[x][y] = d4{0.0, 0.0, 0.0, 0.0};
+    double rv[4], ta[4][RB], tb[4][RB];    // the next sixteen points: four quads
+    auto load = [&](long base) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const long n = base + 4 * u + g, nc = min(n, n1 - 1);
+            const double v = r[nc];
+            rv[u] = (n < n1) ? v : 0.0;
+#pragma unroll
+            for (int x = 0; x < RB; ++x) {
+                ta[u][x] = T[nc * ld + ca[x]];
+                if (!diag) tb[u][x] = T[nc * ld + cb[x]];
+            }
+        }
+    };
+    long base = n0 + 16 * w;
+    if (base < n1) load(base);
+    for (; base < n1; base += 64) {
+        double a1[4][RB], a2[4][RB], bx[4][RB];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int x = 0; x < RB; ++x) {
+                const double xa = ta[u][x] - ya[x];
+                a1[u][x] = xa * rv[u];
+                a2[u][x] = a1[u][x] * rv[u];
+                bx[u][x] = diag ? xa : tb[u][x] - yb[x];
+            }
+        if (base + 64 < n1) load(base + 64);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int x = 0; x < RB; ++x)
+#pragma unroll
+                for (int y = 0; y < RB; ++y)
+                    if (y <= x || !diag) {
+                        s1[x][y] = mfma64(a1[u][x], bx[u][y], s1[x][y]);
+                        s2[x][y] = mfma64(a2[u][x], bx[u][y], s2[x][y]);
+                    }
+    }
+#pragma unroll
+    for (int x = 0; x < RB; ++x)
+#pragma unroll
+        for (int y = 0; y < RB; ++y)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                red[w][2 * (RB * x + y)][64 * q + l] = s1[x][y][q];
+                red[w][2 * (RB * x + y) + 1][64 * q + l] = s2[x][y][q];
+            }
+    __syncthreads();
+    const long DD = (long)D * D;
+    double *o = part + ((long)blockIdx.z * gridDim.y + kb) * 2 * DD;
+#pragma unroll
+    for (int x = 0; x < RB; ++x)
+#pragma unroll
+        for (int y = 0; y < RB; ++y) {
+            // thread tid: element tid / 64 of lane tid % 64
+            const int a = 16 * (RB * ti + x) + 4 * w + g, b = 16 * (RB * tj + y) + j;
+            if (a < D && b < D && (y <= x || !diag))
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    const int f = 2 * (RB * x + y) + s;
+                    o[s * DD + (long)a * D + b] =
+                        ((red[0][f][tid] + red[1][f][tid]) + red[2][f][tid]) + red[3][f][tid];
+                }
+        }
+}
 
-__global__ __launch_bounds__(NT) void k_ctemp_moments(
-    const double *__restrict__ T, const double *__restrict__ tt, long N,
-    const double *__restrict__ Y, const double *__restrict__ yy, int k0, int D, int ld,
-    double nbh, double it, double invK, const double *__restrict__ pm,
-    const double *__restrict__ pl, long chunk, double *__restrict__ part) {
-    __shared__ double Xa[CM][CM + 1];
-    __shared__ double Xb[CM][CM + 1];
-    __shared__ double Ys[192];
-    __shared__ double rs[CM];
-    const int tid = threadIdx.x;
+template <int RB>
+__global__ __launch_bounds__(NT, 2) void k_ctemp_moments(
+    const double *__restrict__ T, long N, const double *__restrict__ Y, int D, int ld,
+    const double *__restrict__ R, long chunk, double *__restrict__ part) {
+    __shared__ double red[4][2 * RB * RB][256];
     int p = blockIdx.x, ti = 0;            // lower-triangle pair p -> (ti >= tj)
     while (p > ti) { p -= ti + 1; ++ti; }
-    const int tj = p;
-    const int kb = blockIdx.y, k = k0 + kb;
-    const long n0 = (long)blockIdx.z * chunk;
-    const long n1 = min(N, n0 + chunk);
-    const int a0 = ti * CM, b0 = tj * CM;
-    const int tx = tid & 15, ty = tid >> 4;
-    for (int d = tid; d < ld; d += NT) Ys[d] = Y[(long)k * ld + d];
-    double s1[4][4], s2[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) s1[i][j] = s2[i][j] = 0.0;
-    __syncthreads();
-    for (long base = n0; base < n1; base += CM) {
-        if (tid < CM) {
-            const long n = base + tid;
-            double r = 0.0;
-            if (n < n1) {
-                if (pm[n] == -INFINITY) {
-                    r = invK;
-                } else {
-                    double s = 0.0;
-                    for (int d = 0; d < ld; ++d) s = fma(T[n * ld + d], Ys[d], s);
-                    const double x = exponent(s, yy[k], tt[n], nbh);
-                    r = (x != -INFINITY) ? exp((x - pm[n]) * it - pl[n]) : 0.0;
-                }
-            }
-            rs[tid] = r;
-        }
-        for (int e = tid; e < CM * CM; e += NT) {
-            const int q = e / CM, dd = e % CM;
-            const long n = base + q;
-            const int a = a0 + dd, b = b0 + dd;
-            Xa[q][dd] = (n < n1 && a < D) ? T[n * ld + a] - Ys[a] : 0.0;
-            Xb[q][dd] = (n < n1 && b < D) ? T[n * ld + b] - Ys[b] : 0.0;
-        }
-        __syncthreads();
-        const int np = (int)min((long)CM, n1 - base);
-        for (int q = 0; q < np; ++q) {
-            const double r = rs[q];
-            double ra[4], xb[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) ra[i] = Xa[q][tx + 16 * i] * r;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) xb[j] = Xb[q][ty + 16 * j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const double rra = ra[i] * r;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    s1[i][j] = fma(ra[i], xb[j], s1[i][j]);
-                    s2[i][j] = fma(rra, xb[j], s2[i][j]);
-                }
-            }
-        }
-        __syncthreads();
-    }
-    const long DD = (long)D * D;
-    double *o1 = part + ((long)blockIdx.z * gridDim.y + kb) * 2 * DD;
-    double *o2 = o1 + DD;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int a = a0 + tx + 16 * i, b = b0 + ty + 16 * j;
-            if (a < D && b < D) {
-                o1[(long)a * D + b] = s1[i][j];
-                o2[(long)a * D + b] = s2[i][j];
-            }
-        }
+    if (p == ti) moments_body<RB, true>(red, ti, p, T, N, Y, D, ld, R, chunk, part);
+    else moments_body<RB, false>(red, ti, p, T, N, Y, D, ld, R, chunk, part);
 }
 
 // out[i] = sum over the nc chunk partials of part[c * len + i], in chunk order.
@@ -832,6 +853,153 @@ __global__ void k_sum_chunks(const double *__restrict__ part, int nc, long len,
     double s = 0.0;
     for (int c = 0; c < nc; ++c) s += part[(long)c * len + i];
     out[i] = s;
+}
+
+// The eigenvalue of one centre's S that the critical temperature takes.  Workgroup
+// (kb, part): of A = sc (2 S1) or sc (2 S1 - 2 S2), n x n, the largest eigenvalue
+// below sc limit, and 0 in the place of those at or above it (comm.c:2149-2161):
+// val[2 kb + part] = their maximum / sc.  A's lower triangle is packed in LDS,
+// reduced to tridiagonal form by Householder reflections (Golub & Van Loan,
+// Matrix Computations, 4th ed., 8.3.1), and the one eigenvalue wanted is found by
+// Sturm counts (8.4.1) at 64 points of the interval at a time, one per lane.
+// Bound by the chain of reflections (two reductions and a matrix-vector product
+// each).  800 matrices of n = 32 in 180 us, 1216 of n = 166 in 6.1 ms; on 16 host
+// threads, with S to copy there first, the search took 2.7 ms longer at n = 32
+// and 0.2 s at n = 166.
+__global__ __launch_bounds__(256) void k_ctemp_eig(const double *__restrict__ S, int n,
+                                                   const double *__restrict__ limit,
+                                                   const double *__restrict__ scale,
+                                                   double *__restrict__ val) {
+    extern __shared__ double A[];                  // n (n + 1) / 2, then v, p, d, e of n each
+    __shared__ double red[4];
+    const int tid = threadIdx.x, nt = blockDim.x, l = tid & 63, w = tid >> 6;
+    const long kb = blockIdx.x;
+    const int sub = blockIdx.y;
+    const double sc = scale[kb], lim = limit[kb] * sc;
+    if (sc == 0.0) return;                         // a centre without weight: not asked for
+    double *v = A + n * (n + 1) / 2, *p = v + n, *d = p + n, *e = d + n;
+    const double *S1 = S + kb * 2 * n * n, *S2 = S1 + (long)n * n;
+    auto at = [&](int i, int j) -> double & { return A[i * (i + 1) / 2 + j]; };   // j <= i
+    auto sum = [&](double x) {                     // over the workgroup, in every thread
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
+        __syncthreads();                           // the last sum's readers are done
+        if (l == 0) red[w] = x;
+        __syncthreads();
+        double s = red[0];
+        for (int q = 1; q < nt / 64; ++q) s += red[q];
+        return s;
+    };
+    for (int i = w; i < n; i += nt / 64)
+        for (int j = l; j <= i; j += 64) {
+            const double a = 2.0 * S1[(long)i * n + j];
+            at(i, j) = (sub ? a - 2.0 * S2[(long)i * n + j] : a) * sc;
+        }
+    __syncthreads();
+    for (int k = 0; k + 2 < n; ++k) {
+        // the reflection that annihilates A[k + 2 .., k]: v = x - alpha e1
+        double s = 0.0;
+        for (int i = k + 2 + tid; i < n; i += nt) s = fma(at(i, k), at(i, k), s);
+        s = sum(s);
+        const double x0 = at(k + 1, k), norm = sqrt(fma(x0, x0, s));
+        const double alpha = (x0 > 0.0) ? -norm : norm, v0 = x0 - alpha, vv = fma(v0, v0, s);
+        if (tid == 0) {
+            d[k] = at(k, k);
+            e[k] = alpha;
+        }
+        if (vv == 0.0 || s == 0.0) {               // (uniform) nothing to annihilate
+            if (tid == 0) e[k] = x0;
+            continue;
+        }
+        for (int i = k + 1 + tid; i < n; i += nt) v[i] = (i == k + 1) ? v0 : at(i, k);
+        __syncthreads();
+        // p = 2 A v / vv, then p -= (v.p / vv) v, and A -= v p^T + p v^T
+        double vp = 0.0, pi = 0.0;
+        const int i = k + 1 + tid;                 // n <= 192 rows: one to a thread (or none)
+        for (int i0 = i; i0 < n; i0 += nt) {
+            double q[4] = {0.0, 0.0, 0.0, 0.0};    // (four chains in flight)
+            auto elem = [&](int j) { return j <= i0 ? at(i0, j) : at(j, i0); };
+            int j = k + 1;
+            for (; j + 4 <= n; j += 4)
+#pragma unroll
+                for (int u = 0; u < 4; ++u) q[u] = fma(elem(j + u), v[j + u], q[u]);
+            for (; j < n; ++j) q[0] = fma(elem(j), v[j], q[0]);
+            pi = 2.0 * ((q[0] + q[1]) + (q[2] + q[3])) / vv;
+            p[i0] = pi;
+            vp = fma(v[i0], pi, vp);
+        }
+        const double c = sum(vp) / vv;
+        for (int i0 = i; i0 < n; i0 += nt) p[i0] -= c * v[i0];
+        __syncthreads();
+        for (int r = k + 1 + w; r < n; r += nt / 64) {
+            const double vr = v[r], pr = p[r];
+            for (int j = k + 1 + l; j <= r; j += 64) at(r, j) -= vr * p[j] + pr * v[j];
+        }
+        __syncthreads();
+    }
+    if (tid == 0) {
+        if (n > 1) {
+            d[n - 2] = at(n - 2, n - 2);
+            e[n - 2] = at(n - 1, n - 2);
+        }
+        d[n - 1] = at(n - 1, n - 1);
+        e[n - 1] = 0.0;
+    }
+    __syncthreads();
+    if (w > 0) return;
+    // Gershgorin bounds, and the smallest pivot a count may divide by
+    double lo = INFINITY, hi = -INFINITY;
+    bool finite = true;
+    for (int i = l; i < n; i += 64) {
+        const double r = fabs(e[i]) + (i ? fabs(e[i - 1]) : 0.0);
+        finite = finite && fabs(d[i]) + r < INFINITY;
+        lo = fmin(lo, d[i] - r);
+        hi = fmax(hi, d[i] + r);
+    }
+    if (!__all(finite)) {                          // NaN or infinite data: no eigenvalues
+        if (l == 0) val[2 * kb + sub] = NAN;
+        return;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        lo = fmin(lo, __shfl_xor(lo, o));
+        hi = fmax(hi, __shfl_xor(hi, o));
+    }
+    const double tnorm = fmax(fabs(lo), fabs(hi));
+    const double pivmin = fmax(2.3e-308, 2.3e-16 * 2.3e-16 * tnorm);
+    auto below = [&](double x) {                   // eigenvalues below x
+        int c = 0;
+        double q = 1.0, e2 = 0.0;
+        for (int i = 0; i < n; ++i) {
+            q = d[i] - x - e2 / q;
+            if (fabs(q) < pivmin) q = -pivmin;
+            c += (q < 0.0) ? 1 : 0;
+            e2 = e[i] * e[i];
+        }
+        return c;
+    };
+    const double pad = 4.0 * 2.3e-16 * n * tnorm + pivmin;
+    const int idx = below(lim);                    // the idx-th smallest is the largest below
+    double best = (idx < n) ? 0.0 : -INFINITY;
+    double a = lo - pad, b = fmin(hi + pad, lim);
+    if (idx > 0 && (idx == n || b > 0.0)) {
+        if (idx < n && a < 0.0 && below(0.0) >= idx) {
+            // none between 0 and the limit: 0 stands
+        } else {
+            for (int it = 0; it < 64; ++it) {
+                const double h = (b - a) / 65.0, x = a + h * (l + 1);
+                const unsigned long long up = __ballot(below(x) >= idx);
+                const int f = up ? __builtin_ctzll(up) : 64;
+                const double na = (f > 0) ? a + h * f : a, nb = (f < 64) ? a + h * (f + 1) : b;
+                const bool done = !(nb - na < b - a) || nb - na <= 2.3e-16 * fmax(fabs(na), fabs(nb));
+                a = na;
+                b = nb;
+                if (done) break;
+            }
+            best = fmax(best, 0.5 * (a + b));
+        }
+    }
+    if (l == 0) val[2 * kb + sub] = best / sc;
 }
 
 }  // namespace
@@ -922,23 +1090,54 @@ int dg_resp_dense_fp64(dg_ctx *c, double *dR, long ldR) {
     return DG_OK;
 }
 
-int dg_ctemp_moments_fp64(dg_ctx *c, int k0, int KB, int nc, double *dPart, double *dS) {
+int dg_ctemp_fp64(dg_ctx *c, int k0, int KB, const DgCtempPlan &p, const double *dLimit,
+                  double *buf, double *dVal) {
     const double it = c->last_isDA ? 1.0 / c->last_temp : 1.0;
-    const int nt = (c->D + CM - 1) / CM;
-    const long tiles = (c->N + CM - 1) / CM;
-    const long chunk = ((tiles + nc - 1) / nc) * CM;
-    dim3 grid((unsigned)(nt * (nt + 1) / 2), (unsigned)KB, (unsigned)nc);
-    hipLaunchKernelGGL(k_ctemp_moments, grid, dim3(NT), 0, c->stream, c->T64, c->tt, c->N,
-                       c->Y64, c->yy, k0, c->D, c->ldt, -c->beta / 2.0, it, 1.0 / c->K, c->pm,
-                       c->pl, chunk, dPart);
+    const int D = c->D;
+    double *R = buf, *part = buf + p.r_len, *S = p.nc > 1 ? part + p.s_len * p.nc : part;
+    // R of these centres, then their moments, then the eigenvalues
+    const Ranges r = centre_ranges(c->N, KB);
+    hipLaunchKernelGGL(k_resp_dense, dim3((unsigned)((c->N + P1 - 1) / P1), (unsigned)r.count),
+                       dim3(NT), 0, c->stream, c->T64, c->tt, c->N, c->Y64 + (long)k0 * c->ldt,
+                       c->yy + k0, KB, D, c->ldt, -c->beta / 2.0, it, 1.0 / c->K, c->pm, c->pl,
+                       r.tiles_per, R, c->N);
     DG_HIP(c, hipGetLastError());
-    if (nc > 1) {
-        const long len = (long)KB * 2 * c->D * c->D;
+    const long chunk = ((c->N + (long)p.nc * 64 - 1) / ((long)p.nc * 64)) * 64;
+    const dim3 grid((unsigned)p.pairs, (unsigned)KB, (unsigned)p.nc);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(NT), 0, c->stream, c->T64, c->N,
+                           c->Y64 + (long)k0 * c->ldt, D, c->ldt, R, chunk, part);
+    };
+    if (D <= 16) go(k_ctemp_moments<1>);
+    else go(k_ctemp_moments<2>);
+    DG_HIP(c, hipGetLastError());
+    if (p.nc > 1) {
+        const long len = (long)KB * 2 * D * D;
         hipLaunchKernelGGL(k_sum_chunks, dim3((unsigned)((len + 255) / 256)), dim3(256), 0,
-                           c->stream, dPart, nc, len, dS);
+                           c->stream, part, p.nc, len, S);
         DG_HIP(c, hipGetLastError());
     }
+    // (a wave is enough for 64 rows; 145 KB of LDS at D = 192)
+    const size_t lds = ((size_t)D * (D + 1) / 2 + 4 * D) * sizeof(double);
+    hipLaunchKernelGGL(k_ctemp_eig, dim3((unsigned)KB, 2), dim3(D <= 64 ? 64 : 256), lds, c->stream, S,
+                       D, dLimit + 2 * (long)k0, dLimit + 2 * (long)k0 + KB, dVal + 2 * (long)k0);
+    DG_HIP(c, hipGetLastError());
     return DG_OK;
+}
+
+// At most 256 MB of S1 and S2 and 1 GB of R to a batch of centres; about 2048
+// workgroups of moments, with 256 points to each at least.
+DgCtempPlan dg_ctemp_plan(const dg_ctx *c) {
+    DgCtempPlan p;
+    const long D = c->D, DD = D * D;
+    p.KB = (int)std::max(1L, std::min({(long)c->K, (1L << 25) / (2 * DD), (1L << 27) / c->N}));
+    const long nt = D <= 16 ? 1 : (D + 31) / 32;
+    p.pairs = (int)(nt * (nt + 1) / 2);
+    const long want = (2048 + (long)p.pairs * p.KB - 1) / ((long)p.pairs * p.KB);
+    p.nc = (int)std::max(1L, std::min({want, 64L, (c->N + 255) / 256}));
+    p.r_len = (size_t)p.KB * c->N;
+    p.s_len = (size_t)p.KB * 2 * DD;
+    return p;
 }
 
 int dg_map_fp64(dg_ctx *c, const double *dX, int L, double *dM) {

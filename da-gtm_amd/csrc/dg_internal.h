@@ -232,11 +232,20 @@ int dg_estep_fp64(dg_ctx *ctx, int isDA, double temp);
 int dg_pass1_fp64(dg_ctx *ctx, int isDA, double temp);   // its first half: pm, pl, log g, log h
 int dg_resp_dense_fp64(dg_ctx *ctx, double *dR, long ldR);
 int dg_map_fp64(dg_ctx *ctx, const double *dX, int L, double *dM);
-// S1, S2 of centres k0 .. k0+KB-1 into dS (KB x 2 x D x D, lower triangle
-// valid) from nc N-chunk partials in dPart (dS == dPart when nc == 1).
-int dg_ctemp_moments_fp64(dg_ctx *ctx, int k0, int KB, int nc, double *dPart, double *dS);
+// The critical temperatures' eigenvalues for centres k0 .. k0 + KB - 1, from the FP64
+// normalisers: dVal[2 k + part] for part 0 (2 S1) and 1 (2 S1 - 2 S2).  dLimit
+// holds, for each batch, its KB limits and then its KB scales at 2 k0; buf the
+// batch's R, moment partials and, with several chunks, their sums.
+struct DgCtempPlan {
+    int KB, nc, pairs;        // centres per batch, N chunks, tile pairs of a moment
+    size_t r_len, s_len;      // doubles of R and of one set of S1, S2
+    size_t buf_len() const { return r_len + s_len * (nc > 1 ? nc + 1 : 1); }
+};
+DgCtempPlan dg_ctemp_plan(const dg_ctx *ctx);
+int dg_ctemp_fp64(dg_ctx *ctx, int k0, int KB, const DgCtempPlan &p, const double *dLimit,
+                  double *buf, double *dVal);
 
-// ---- host eigenvalues (dg_eig.cpp) ----
+// ---- host eigenvalues (dg_eig.cpp): the plain statement that the tests hold against LAPACK ----
 extern "C" int dg_sym_eigvals(int n, const double *A, long lda, double *w);
 
 // ---- mixed kernels (dg_mixed.hip) ----

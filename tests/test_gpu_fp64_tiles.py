@@ -76,3 +76,36 @@ def test_outputs_at_tile_edges(N, D, K, far, L):
             assert np.array_equal(G, e.stats()[0])
         assert np.allclose(G, m.R.sum(1), rtol=1e-10, atol=1e-12)
         assert np.allclose(RT, m.R @ T, rtol=1e-10, atol=1e-10)
+
+
+@pytest.mark.parametrize("N,D,K", [
+    (40, 1, 3), (61, 2, 5), (64, 15, 4), (65, 16, 9), (200, 17, 5), (700, 33, 20), (90, 64, 3),
+    (150, 65, 4), (300, 128, 2), (260, 192, 3),
+])
+def test_ctemp_at_tile_edges(N, D, K):
+    """The critical temperatures of every centre from numpy's moments and
+    eigvalsh, at the edges of the moments' tiles and of the eigenvalue kernel:
+    both sides are off by some units of 2^-52 of a matrix' norm, n <= 192 of
+    them at worst, so 1e-11 of the norm."""
+    print(f"case: ctemp N={N} D={D} K={K}", flush=True)
+    T, Y, FI, beta = _problem(N, D, K)
+    temp, eps = 1.7, 1e-6
+    m = O.Model(T, FI, Y, beta)
+    m.estep(1, temp)
+    g = m.R.sum(1)
+    with dg.Engine(precision=dg.FP64) as e:
+        e.upload(T, FI, Y, beta)
+        e.estep(True, temp)
+        for t in (temp, 0.05, 1e6):            # some, hardly any, all eigenvalues below
+            cmax, ck = e.next_ctemp(t, eps, g)
+            for k in range(K):
+                x, r = T - Y[k], m.R[k][:, None]
+                S1, S2 = (x * r).T @ x, (x * r * r).T @ x
+                w = np.concatenate([np.linalg.eigvalsh(2 * S1), np.linalg.eigvalsh(2 * (S1 - S2))])
+                norm = np.abs(w).max()
+                lim = (t - eps) * g[k] * 2 / beta
+                if np.abs(w - lim).min() < 1e-10 * norm:
+                    continue                   # on the limit: either side may take it
+                want = beta / 2 / g[k] * np.where(w >= lim, 0.0, w).max()
+                assert abs(ck[k] - want) <= 1e-11 * beta / 2 / g[k] * norm
+            assert cmax == ck.max()
