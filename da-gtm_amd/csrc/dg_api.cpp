@@ -116,12 +116,13 @@ int alloc_kstate(dg_ctx *c) {
     long nch = (K + 63) / 64;
     if (nch > 64) nch = 64;
     c->nchAB = (int)(nch < 1 ? 1 : nch);
+    c->partRT_len = std::max({(size_t)c->NC * K * D, dg_pass1_part(N),
+                              dg_map_part(N, c->K) + (size_t)3 * (K + N)});
     int rc;
     if ((rc = dalloc(c, &c->FI, (size_t)K * M1)) || (rc = dalloc(c, &c->Y64, (size_t)K * ld)) ||
         (rc = dalloc(c, &c->yy, K)) || (rc = dalloc(c, &c->G, K)) || (rc = dalloc(c, &c->Gm, K)) ||
         (rc = dalloc(c, &c->RT, (size_t)K * D)) ||
-        (rc = dalloc(c, &c->partRT, std::max({(size_t)c->NC * K * D, dg_pass1_part(N),
-                                             dg_map_part(N, c->K)}))) ||
+        (rc = dalloc(c, &c->partRT, c->partRT_len)) ||
         (rc = dalloc(c, &c->partG, (size_t)c->NC * K + (size_t)3 * dg_pass1_wgs(N))) ||
         (rc = dalloc(c, &c->partAB, std::max((size_t)c->nchAB * ((size_t)M1 * M1 + (size_t)M1 * D),
                                              (size_t)(K + 63) / 64))))
@@ -132,13 +133,17 @@ int alloc_kstate(dg_ctx *c) {
     return DG_OK;
 }
 
-// Host rows (stride lds) -> device rows (stride ldd >= cols, zero padding).
-// Pageable host memory moves far faster as one block than as many short
-// rows (10^6 rows of 166 doubles: 9.4 s strided, 0.2 s as one block), so the
-// host block -- (rows - 1) lds + cols doubles, nothing past the last row's
-// data -- goes over in one copy and is repacked on the device.
+// Rows cross between host and device as one block each way: a strided copy
+// of pageable host memory goes row by row, at 6 to 9 microseconds a row (10^6
+// rows of 166 doubles up: 9.4 s, as one block 0.2 s; 8000 rows of 166 down:
+// 53 ms, as one block 1 ms).
+
+// Host rows (stride lds) -> device rows (stride ldd >= cols, zero padding).  The
+// host block -- (rows - 1) lds + cols doubles, nothing past the last row's data
+// -- is repacked on the device; `scratch` (room doubles) is used for it where it
+// is large enough.
 int upload_rows(dg_ctx *c, double *dst, int ldd, const double *src, long lds, long rows,
-                int cols) {
+                int cols, double *scratch = nullptr, size_t room = 0) {
     const size_t n = (size_t)(rows - 1) * lds + cols;
     if (lds == cols && ldd == cols) {
         DG_HIP(c, hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
@@ -146,12 +151,40 @@ int upload_rows(dg_ctx *c, double *dst, int ldd, const double *src, long lds, lo
     }
     DevBuf tmp;
     int rc;
-    if ((rc = dalloc(c, &tmp.p, n))) return rc;
-    DG_HIP(c, hipMemcpyAsync(tmp.p, src, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    if ((rc = dg_pad_rows(c, tmp.p, rows, cols, lds, ldd, dst))) return rc;
-    // the block is freed on return: wait for the repack that reads it
-    DG_HIP(c, hipStreamSynchronize(c->stream));
+    if (room < n) {
+        if ((rc = dalloc(c, &tmp.p, n))) return rc;
+        scratch = tmp.p;
+    }
+    DG_HIP(c, hipMemcpyAsync(scratch, src, n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    if ((rc = dg_pad_rows(c, scratch, rows, cols, lds, ldd, dst))) return rc;
+    // a block of its own is freed on return: wait for the repack that reads it
+    if (tmp.p) DG_HIP(c, hipStreamSynchronize(c->stream));
     return DG_OK;
+}
+
+// Dense device rows -> host rows (stride ldd >= cols); what lies between the
+// host's rows is not touched.  Returns when the rows are there.
+int download_rows(dg_ctx *c, double *dst, long ldd, const double *src, long rows, long cols) {
+    const size_t row = (size_t)cols * sizeof(double);
+    if (ldd == cols) {
+        DG_HIP(c, hipMemcpyAsync(dst, src, (size_t)rows * row, hipMemcpyDeviceToHost, c->stream));
+        DG_HIP(c, hipStreamSynchronize(c->stream));
+        return DG_OK;
+    }
+    // padded host rows: through a host block of at most 32 MB (or one row)
+    const long step = std::max(1L, std::min(rows, (long)((32u << 20) / row)));
+    double *block = static_cast<double *>(std::malloc((size_t)step * row));
+    if (!block) return dg_fail(c, DG_ENOMEM, "host allocation");
+    hipError_t e = hipSuccess;
+    for (long r0 = 0; r0 < rows && e == hipSuccess; r0 += step) {
+        const long n = std::min(step, rows - r0);
+        e = hipMemcpyAsync(block, src + r0 * cols, (size_t)n * row, hipMemcpyDeviceToHost, c->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+        for (long r = 0; r < n && e == hipSuccess; ++r)
+            std::memcpy(dst + (r0 + r) * ldd, block + r * cols, row);
+    }
+    std::free(block);
+    return e == hipSuccess ? DG_OK : dg_hip_check(c, e, "copy to the host");
 }
 
 int sync_scalars(dg_ctx *c) {
@@ -328,8 +361,8 @@ int dg_upload(dg_ctx *c, const double *T, long N, int D, long ldT, const double 
         return rc;
     }
     if ((rc = upload_rows(c, c->T64, (int)ld, T, ldT, N, D)) ||
-        (rc = upload_rows(c, c->FI, M1, FI, ldFI, K, M1)) ||
-        (rc = upload_rows(c, c->Y64, (int)ld, Y, ldY, K, D))) {
+        (rc = upload_rows(c, c->FI, M1, FI, ldFI, K, M1, c->partRT, c->partRT_len)) ||
+        (rc = upload_rows(c, c->Y64, (int)ld, Y, ldY, K, D, c->partRT, c->partRT_len))) {
         free_problem(c);
         return rc;
     }
@@ -355,7 +388,7 @@ int dg_set_state(dg_ctx *c, const double *Y, long ldY, double beta) {
     if (!Y || ldY < c->D || !(beta > 0.0)) return dg_fail(c, DG_EINVAL, "dg_set_state: bad args");
     int rc;
     if ((rc = select_device(c))) return rc;
-    if ((rc = upload_rows(c, c->Y64, c->ldt, Y, ldY, c->K, c->D))) return rc;
+    if ((rc = upload_rows(c, c->Y64, c->ldt, Y, ldY, c->K, c->D, c->partRT, c->partRT_len))) return rc;
     if ((rc = dg_rownorms(c, c->Y64, c->K, c->ldt, c->D, c->yy))) return rc;
     DG_HIP(c, hipMemsetAsync(c->Gm, 0, (size_t)c->K * sizeof(double), c->stream));
     c->beta = beta;
@@ -749,24 +782,10 @@ int dg_map(dg_ctx *c, const double *X, int L, long ldX, double *M, long ldM) {
         if ((rc = dg_estep(c, c->last_isDA, c->last_temp, &eo))) return rc;
     }
     c->fp64_due = c->mixed();
-    double *dX = nullptr, *dM = nullptr;
-    if ((rc = dalloc(c, &dX, (size_t)c->K * L))) return rc;
-    if ((rc = dalloc(c, &dM, (size_t)c->N * L))) { dfree(dX); return rc; }
-    hipError_t e = hipMemcpy2DAsync(dX, (size_t)L * sizeof(double), X, (size_t)ldX * sizeof(double),
-                                    (size_t)L * sizeof(double), (size_t)c->K,
-                                    hipMemcpyHostToDevice, c->stream);
-    if (e == hipSuccess) {
-        // the mixed path keeps its FP64 centres current, so the FP64 kernel serves both
-        rc = dg_map_fp64(c, dX, L, dM);
-        if (!rc)
-            e = hipMemcpy2DAsync(M, (size_t)ldM * sizeof(double), dM, (size_t)L * sizeof(double),
-                                 (size_t)L * sizeof(double), (size_t)c->N, hipMemcpyDeviceToHost,
-                                 c->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    }
-    dfree(dX); dfree(dM);
-    if (e != hipSuccess) return dg_hip_check(c, e, "dg_map");
-    return rc;
+    // the coordinates and the projection behind the projection's sums
+    double *dX = c->partRT + dg_map_part(c->N, c->K), *dM = dX + (size_t)c->K * L;
+    if ((rc = upload_rows(c, dX, L, X, ldX, c->K, L)) || (rc = dg_map_fp64(c, dX, L, dM))) return rc;
+    return download_rows(c, M, ldM, dM, c->N, L);
 }
 
 int dg_map_noalloc(dg_ctx *c, const double *X, int L, long ldX, double *M, long ldM) {
@@ -797,13 +816,7 @@ int dg_map_noalloc(dg_ctx *c, const double *X, int L, long ldX, double *M, long 
         DG_HIP(c, hipMemcpy2DAsync(dX, row, X, (size_t)ldX * sizeof(double), row, (size_t)c->K,
                                    hipMemcpyHostToDevice, c->stream));
     if ((rc = dg_map_fp64(c, dX, L, dM))) return rc;
-    if (ldM == L)
-        DG_HIP(c, hipMemcpyAsync(M, dM, (size_t)c->N * row, hipMemcpyDeviceToHost, c->stream));
-    else
-        DG_HIP(c, hipMemcpy2DAsync(M, (size_t)ldM * sizeof(double), dM, row, row, (size_t)c->N,
-                                   hipMemcpyDeviceToHost, c->stream));
-    DG_HIP(c, hipStreamSynchronize(c->stream));
-    return DG_OK;
+    return download_rows(c, M, ldM, dM, c->N, L);
 }
 
 int dg_resp_dense(dg_ctx *c, double *R, long ldR) {
@@ -814,19 +827,14 @@ int dg_resp_dense(dg_ctx *c, double *R, long ldR) {
     if ((rc = select_device(c))) return rc;
     c->fp64_due = c->mixed();
     if (c->mixed() && (rc = dg_pass1_fp64(c, c->last_isDA, c->last_temp))) return rc;
-    double *dR = nullptr;
-    if ((rc = dalloc(c, &dR, (size_t)c->K * c->N))) return rc;
-    rc = dg_resp_dense_fp64(c, dR, c->N);
-    hipError_t e = hipSuccess;
-    if (!rc) {
-        e = hipMemcpy2DAsync(R, (size_t)ldR * sizeof(double), dR, (size_t)c->N * sizeof(double),
-                             (size_t)c->N * sizeof(double), (size_t)c->K, hipMemcpyDeviceToHost,
-                             c->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    DevBuf own;
+    double *dR = c->partRT;
+    if ((size_t)c->K * c->N > c->partRT_len) {
+        if ((rc = dalloc(c, &own.p, (size_t)c->K * c->N))) return rc;
+        dR = own.p;
     }
-    dfree(dR);
-    if (e != hipSuccess) return dg_hip_check(c, e, "dg_resp_dense");
-    return rc;
+    if ((rc = dg_resp_dense_fp64(c, dR, c->N))) return rc;
+    return download_rows(c, R, ldR, dR, c->K, c->N);
 }
 
 int dg_download(dg_ctx *c, double *W, long ldW, double *Y, long ldY, double *beta) {
@@ -836,15 +844,16 @@ int dg_download(dg_ctx *c, double *W, long ldW, double *Y, long ldY, double *bet
     if ((rc = select_device(c))) return rc;
     if (W) {
         if (ldW < c->D) return dg_fail(c, DG_EINVAL, "dg_download: ldW < D");
-        DG_HIP(c, hipMemcpy2DAsync(W, (size_t)ldW * sizeof(double), c->W,
-                                   (size_t)c->D * sizeof(double), (size_t)c->D * sizeof(double),
-                                   (size_t)c->M1, hipMemcpyDeviceToHost, c->stream));
+        if ((rc = download_rows(c, W, ldW, c->W, c->M1, c->D))) return rc;
     }
     if (Y) {
         if (ldY < c->D) return dg_fail(c, DG_EINVAL, "dg_download: ldY < D");
-        DG_HIP(c, hipMemcpy2DAsync(Y, (size_t)ldY * sizeof(double), c->Y64,
-                                   (size_t)c->ldt * sizeof(double), (size_t)c->D * sizeof(double),
-                                   (size_t)c->K, hipMemcpyDeviceToHost, c->stream));
+        const double *src = c->Y64;
+        if (c->ldt != c->D) {                      // its rows without their padding
+            if ((rc = dg_pad_rows(c, c->Y64, c->K, c->D, c->ldt, c->D, c->partRT))) return rc;
+            src = c->partRT;
+        }
+        if ((rc = download_rows(c, Y, ldY, src, c->K, c->D))) return rc;
     }
     DG_HIP(c, hipStreamSynchronize(c->stream));
     if (beta) *beta = c->beta;
@@ -861,9 +870,7 @@ int dg_get_stats(dg_ctx *c, double *G, double *RT, long ldRT) {
                                  c->stream));
     if (RT) {
         if (ldRT < c->D) return dg_fail(c, DG_EINVAL, "dg_get_stats: ldRT < D");
-        DG_HIP(c, hipMemcpy2DAsync(RT, (size_t)ldRT * sizeof(double), c->RT,
-                                   (size_t)c->D * sizeof(double), (size_t)c->D * sizeof(double),
-                                   (size_t)c->K, hipMemcpyDeviceToHost, c->stream));
+        if ((rc = download_rows(c, RT, ldRT, c->RT, c->K, c->D))) return rc;
     }
     DG_HIP(c, hipStreamSynchronize(c->stream));
     return DG_OK;

@@ -55,6 +55,7 @@ struct dg_ctx {
     double *logh = nullptr;        // N
     double *partRT = nullptr;      // NC x K x D; also pass 1's slice states (before
                                    // pass 2) and the projection's sums
+    size_t partRT_len = 0;         // its doubles (at least K x D; scratch between E-steps)
     double *partG = nullptr;       // NC x K
     double *partLog64 = nullptr;   // pass 1's log sums, 3 per workgroup (behind partG)
     int NC = 1;                    // N chunks of E-pass 2
