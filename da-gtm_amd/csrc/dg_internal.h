@@ -147,6 +147,9 @@ struct BInst {
 
 __host__ __device__ inline int bk_cdiv(long a, long b) { return (int)((a + b - 1) / b); }
 
+// edge of k_partAB's output tiles
+__host__ __device__ inline int dg_ab_tile(int M1) { return M1 > 256 ? 128 : 64; }
+
 // workgroups of instance I in the flat grid of a kind
 __host__ __device__ inline int bk_count(const BInst &I, int kind) {
     const auto cdiv = bk_cdiv;
@@ -155,7 +158,8 @@ __host__ __device__ inline int bk_count(const BInst &I, int kind) {
         case BK_REDUCE32: return cdiv(I.K, kBRK) * cdiv(I.D, kBRD);
         case BK_ZERO_FIX: return I.D;
         case BK_COPY_G: return cdiv(I.K, 256);
-        case BK_PART_AB: return cdiv(I.M1, kBGT) * cdiv(I.M1 + I.D, kBGT) * I.nchAB;
+        case BK_PART_AB:
+            return cdiv(I.M1, dg_ab_tile(I.M1)) * cdiv(I.M1 + I.D, dg_ab_tile(I.M1)) * I.nchAB;
         case BK_SUM_AB: return cdiv((long)I.M1 * I.M1 + (long)I.M1 * I.D, 256);
         case BK_TRSM_LDS: return cdiv(I.D, 32);
         case BK_PHIW: return cdiv(I.K, kBGT) * cdiv(I.D, kBGT);

@@ -395,90 +395,132 @@ __global__ __launch_bounds__(64) void k_bc_trace(const double *__restrict__ A0, 
     if (threadIdx.x == 0) scal[kScalJitter] = s;
 }
 
-// Tiled FP64 products of the M-step: 64 x 64 output tiles, 256 threads with
-// 4 x 4 results each (rows ty + 16 a, columns tx + 16 b: conflict-free LDS
-// reads), the inner dimension in steps of 16 staged through LDS.
+typedef double d4 __attribute__((ext_vector_type(4)));
+
+// D[i][j] += sum_q A[i][q] B[q][j], 16 x 16 x 4: lane l holds A[l % 16][l / 16],
+// B[l / 16][l % 16] and, in element r, D[4 r + l / 16][l % 16].  It rounds like a
+// chain of FMAs in the order of q, so the products below have the bits of plain
+// loops over their inner index.
+__device__ __forceinline__ d4 mfma64(double a, double b, d4 c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
+// Tiles of the M-step's products: 64 x 64 results to a workgroup.
 constexpr int GT = 64, GK = 16;
+
+// A tile of [A | B] holds nothing that is read: all of it above A's diagonal
+// (the factorisation takes the lower triangle).
+__device__ __forceinline__ bool upper_tile(int ti, int tj, int M1) {
+    return tj > ti && (tj + 1) * dg_ab_tile(M1) <= M1;
+}
 
 // Split-K partials of [A | B] = FI^T [diag(G) FI | RT], an M1 x (M1 + D)
 // product over the centres: workgroup (bx, by, c) computes one output tile
-// over centres [c kc, min(K, (c + 1) kc)); part is nch x M1 x (M1 + D).
+// over centres [c kc, min(K, (c + 1) kc)); part is nch x M1 x (M1 + D).  A wave
+// takes a quarter of it (16 RB x 16 RB) straight from global memory, where a row
+// of FI or RT is a run of whole cache lines; 4 U centres are multiplied while the
+// next ones are on their way.  dg_ab_tile chooses 64 x 64 tiles (RB = 2), which
+// spread a small M1 over the chip, or for M1 > 256 128 x 128 (RB = 4), whose
+// operands take half as much of L2's rate: at M1 = 1001 it bound the small ones.
+// FP64 pipe: K = 32768, M1 = 1001, D = 166: 3043 -> 1410 us (64 x 64: 2100);
+// K = 8000, M1 = 126: 41 -> 28 us (4 x 4 register tiles of FMAs from LDS, and
+// A's upper half computed too).
+template <int RB>
 __device__ __forceinline__ void k_partAB_body(
     const int bx, const int by, const int bz, const int gx, const double *__restrict__ FI,
     const double *__restrict__ G, const double *__restrict__ RT, int K, int M1, int D, int kc,
     double *__restrict__ part) {
-    __shared__ double As[GK][GT], Bs[GK][GT];
+    if (upper_tile(bx, by, M1)) return;
     const int NCOL = M1 + D;
-    const int i0 = bx * GT, j0 = by * GT, c = bz;
+    const int c = bz;
     const int k0 = c * kc, k1 = (k0 + kc < K) ? k0 + kc : K;
-    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-    double acc[4][4];
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6, j = l & 15, g = l >> 4;
+    const int i0 = 16 * RB * (2 * bx + (w & 1)), j0 = 16 * RB * (2 * by + (w >> 1));
+    const long E = (long)M1 * NCOL;
+    if (i0 >= M1 || j0 >= NCOL) return;
+    // per lane: its columns of A's operand and of B's at centre k0 + g (past the
+    // end: the last ones again, whose results are not stored), moved on by adds
+    const double *pa[RB], *pb[RB], *pg = G + k0 + g;
+    long sb[RB];
+    bool wg[RB];
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int x = 0; x < RB; ++x) {
+        pa[x] = FI + (long)(k0 + g) * M1 + min(i0 + 16 * x + j, M1 - 1);
+        const int col = min(j0 + 16 * x + j, NCOL - 1);
+        wg[x] = col < M1;
+        sb[x] = 4 * (wg[x] ? M1 : D);
+        pb[x] = wg[x] ? FI + (long)(k0 + g) * M1 + col : RT + (long)(k0 + g) * D + (col - M1);
+    }
+    constexpr int U = RB == 2 ? 4 : 2;
+    double ra[U][RB], rb[U][RB], rg[U];
+    auto load = [&](int kb, bool whole) {          // centres kb .. kb + 4 U - 1
 #pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = 0.0;
-    // the next step's operands are loaded into registers while this step's
-    // are multiplied from LDS (four elements of each per thread)
-    static_assert(GK * GT == 4 * 256, "four staged elements per thread");
-    double ra[4], rb[4];
-    auto gload = [&](int kb) {
+        for (int u = 0; u < U; ++u) {
+            const bool in = whole || kb + 4 * u + g < k1;
+            rg[u] = in ? *pg : 0.0;
+            pg += 4;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int e = tid + 256 * u;
-            const int kk = e / GT, col = e % GT, k = kb + kk;
-            double av = 0.0, bv = 0.0;
-            if (k < k1) {
-                const int i = i0 + col, jj = j0 + col;
-                if (i < M1) av = FI[(long)k * M1 + i];
-                if (jj < M1) bv = G[k] * FI[(long)k * M1 + jj];
-                else if (jj < NCOL) bv = RT[(long)k * D + (jj - M1)];
+            for (int x = 0; x < RB; ++x) {
+                ra[u][x] = in ? *pa[x] : 0.0;
+                rb[u][x] = in ? *pb[x] : 0.0;
+                pa[x] += 4L * M1;
+                pb[x] += sb[x];
             }
-            ra[u] = av;
-            rb[u] = bv;
         }
     };
-    if (k0 < k1) gload(k0);
-    for (int kb = k0; kb < k1; kb += GK) {
+    d4 acc[RB][RB];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int e = tid + 256 * u;
-            As[e / GT][e % GT] = ra[u];
-            Bs[e / GT][e % GT] = rb[u];
-        }
-        __syncthreads();
-        if (kb + GK < k1) gload(kb + GK);
+    for (int x = 0; x < RB; ++x)
 #pragma unroll
-        for (int kk = 0; kk < GK; ++kk) {
-            double av[4], bv[4];
+        for (int y = 0; y < RB; ++y) acc[x][y] = d4{0.0, 0.0, 0.0, 0.0};
+    auto next = [&](int kb) {
+        if (kb + 4 * U <= k1) load(kb, true);
+        else if (kb < k1) load(kb, false);
+    };
+    next(k0);
+    for (int kb = k0; kb < k1; kb += 4 * U) {
+        double av[U][RB], bv[U][RB];
 #pragma unroll
-            for (int a = 0; a < 4; ++a) av[a] = As[kk][ty + 16 * a];
+        for (int u = 0; u < U; ++u)
 #pragma unroll
-            for (int b = 0; b < 4; ++b) bv[b] = Bs[kk][tx + 16 * b];
+            for (int x = 0; x < RB; ++x) {
+                av[u][x] = ra[u][x];
+                bv[u][x] = wg[x] ? rg[u] * rb[u][x] : rb[u][x];
+            }
+        next(kb + 4 * U);
 #pragma unroll
-            for (int a = 0; a < 4; ++a)
+        for (int u = 0; u < U; ++u)
 #pragma unroll
-                for (int b = 0; b < 4; ++b) acc[a][b] = fma(av[a], bv[b], acc[a][b]);
-        }
-        __syncthreads();
+            for (int x = 0; x < RB; ++x)
+#pragma unroll
+                for (int y = 0; y < RB; ++y) acc[x][y] = mfma64(av[u][x], bv[u][y], acc[x][y]);
     }
-    const long E = (long)M1 * NCOL;
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int x = 0; x < RB; ++x)
 #pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            const int i = i0 + ty + 16 * a, j = j0 + tx + 16 * b;
-            if (i < M1 && j < NCOL) part[(long)c * E + (long)i * NCOL + j] = acc[a][b];
-        }
+        for (int y = 0; y < RB; ++y)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int i = i0 + 16 * x + 4 * r + g, jj = j0 + 16 * y + j;
+                if (i < M1 && jj < NCOL) part[(long)c * E + (long)i * NCOL + jj] = acc[x][y][r];
+            }
 }
 
-__global__ __launch_bounds__(256) void k_partAB(const double *__restrict__ FI,
-                                                const double *__restrict__ G,
-                                                const double *__restrict__ RT, int K, int M1,
-                                                int D, int kc, double *__restrict__ part) {
-    k_partAB_body(blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, FI, G, RT, K, M1, D, kc, part);
+// The hardware hands workgroup i to XCD i mod 8: all tiles of a chunk go to one
+// XCD, whose L2 then holds the chunk's rows (4.7 MB at M1 = 1001, kc = 512).
+template <int RB>
+__global__ __launch_bounds__(256, 2) void k_partAB(const double *__restrict__ FI,
+                                                   const double *__restrict__ G,
+                                                   const double *__restrict__ RT, int K, int M1,
+                                                   int D, int kc, int nch,
+                                                   double *__restrict__ part) {
+    const int nx = (M1 + 32 * RB - 1) / (32 * RB), ny = (M1 + D + 32 * RB - 1) / (32 * RB);
+    const int i = blockIdx.x >> 3, tile = i % (nx * ny), c = i / (nx * ny) * 8 + (blockIdx.x & 7);
+    if (c < nch) k_partAB_body<RB>(tile % nx, tile / nx, c, 0, FI, G, RT, K, M1, D, kc, part);
 }
 
-// A0 / B from the chunk partials, summed in chunk order.
+// A0 / B from the chunk partials, summed in chunk order (A0 without the tiles
+// that k_partAB leaves out).
 __device__ __forceinline__ void k_sumAB_body(
     const int bx, const int by, const int bz, const int gx, const double *__restrict__ part,
     int nch, int M1, int D, double *__restrict__ A0, double *__restrict__ B) {
@@ -486,6 +528,8 @@ __device__ __forceinline__ void k_sumAB_body(
     const long E = (long)M1 * NCOL;
     const long e = (long)bx * blockDim.x + threadIdx.x;
     if (e >= E) return;
+    const int i = (int)(e / NCOL), j = (int)(e % NCOL);
+    if (j < M1 && upper_tile(i / dg_ab_tile(M1), j / dg_ab_tile(M1), M1)) return;
     // eight loads in flight, then their sums in chunk order
     double s = 0.0;
     int c = 0;
@@ -497,7 +541,6 @@ __device__ __forceinline__ void k_sumAB_body(
         for (int u = 0; u < 8; ++u) s += v[u];
     }
     for (; c < nch; ++c) s += part[(long)c * E + e];
-    const int i = (int)(e / NCOL), j = (int)(e % NCOL);
     if (j < M1) A0[(long)i * M1 + j] = s;
     else B[(long)i * D + (j - M1)] = s;
 }
@@ -960,15 +1003,16 @@ __global__ __launch_bounds__(256) void kb_copy_g(const BInst *__restrict__ tab,
     if (I.do_m && k < I.K) I.Gm[k] = I.G[k];
 }
 
-__global__ __launch_bounds__(256) void kb_partAB(const BInst *__restrict__ tab,
+__global__ __launch_bounds__(256, 2) void kb_partAB(const BInst *__restrict__ tab,
                                                  const int2 *__restrict__ map) {
     const int2 m = map[blockIdx.x];
     const BInst &I = tab[m.x];
     if (!I.do_m) return;
-    const int nx = (I.M1 + GT - 1) / GT, ny = (I.M1 + I.D + GT - 1) / GT;
+    const int t = dg_ab_tile(I.M1), nx = bk_cdiv(I.M1, t), ny = bk_cdiv(I.M1 + I.D, t);
     const int kc = (I.K + I.nchAB - 1) / I.nchAB;
-    k_partAB_body(m.y % nx, (m.y / nx) % ny, m.y / (nx * ny), 0, I.FI, I.G, I.RT, I.K, I.M1, I.D,
-                  kc, I.partAB);
+    const int x = m.y % nx, y = (m.y / nx) % ny, z = m.y / (nx * ny);
+    if (t == 64) k_partAB_body<2>(x, y, z, 0, I.FI, I.G, I.RT, I.K, I.M1, I.D, kc, I.partAB);
+    else k_partAB_body<4>(x, y, z, 0, I.FI, I.G, I.RT, I.K, I.M1, I.D, kc, I.partAB);
 }
 
 __global__ void kb_sumAB(const BInst *__restrict__ tab, const int2 *__restrict__ map) {
@@ -1124,10 +1168,14 @@ int dg_mstep_run(dg_ctx *c, double jitter) {
     const long E = (long)M1 * M1 + (long)M1 * D;
     const int nch = c->nchAB;
     const int kc = (K + nch - 1) / nch;
-    hipLaunchKernelGGL(k_partAB,
-                       dim3((unsigned)((M1 + GT - 1) / GT), (unsigned)((M1 + D + GT - 1) / GT),
-                            (unsigned)nch),
-                       dim3(256), 0, c->stream, c->FI, c->G, c->RT, K, M1, D, kc, c->partAB);
+    const int t = dg_ab_tile(M1);
+    const dim3 abgrid((unsigned)(8 * bk_cdiv(M1, t) * bk_cdiv(M1 + D, t) * bk_cdiv(nch, 8)));
+    if (t == 64)
+        hipLaunchKernelGGL(k_partAB<2>, abgrid, dim3(256), 0, c->stream, c->FI, c->G, c->RT, K, M1, D,
+                           kc, nch, c->partAB);
+    else
+        hipLaunchKernelGGL(k_partAB<4>, abgrid, dim3(256), 0, c->stream, c->FI, c->G, c->RT, K, M1, D,
+                           kc, nch, c->partAB);
     DG_HIP(c, hipGetLastError());
     hipLaunchKernelGGL(k_sumAB, dim3((unsigned)((E + 255) / 256)), dim3(256), 0, c->stream,
                        c->partAB, nch, M1, D, c->A0, c->Bm);

@@ -109,3 +109,31 @@ def test_ctemp_at_tile_edges(N, D, K):
                 want = beta / 2 / g[k] * np.where(w >= lim, 0.0, w).max()
                 assert abs(ck[k] - want) <= 1e-11 * beta / 2 / g[k] * norm
             assert cmax == ck.max()
+
+
+@pytest.mark.parametrize("N,D,K,M1", [
+    (40, 1, 3, 1), (60, 3, 17, 5), (200, 17, 64, 26), (150, 12, 65, 31), (300, 33, 130, 32),
+    (260, 50, 127, 63), (300, 15, 500, 64), (300, 166, 260, 65), (400, 180, 600, 126),
+    (300, 20, 700, 127), (300, 40, 700, 130), (400, 65, 900, 257), (300, 33, 1100, 400),
+])
+def test_mstep_at_tile_edges(N, D, K, M1):
+    """One M-step at the edges of the products' and the factorisation's tiles,
+    against the same equations solved by numpy from the engine's own G and R T.
+    A ridge of 1e-2 tr(A) / n keeps the condition below 1e2 n, and the chains are
+    at most 1100 terms long, so 1e-10 of the largest entry."""
+    print(f"case: mstep N={N} D={D} K={K} M1={M1}", flush=True)
+    T, Y, _, beta = _problem(N, D, K)
+    FI = np.random.default_rng(M1).normal(size=(K, M1))
+    lam = 1e-2 * N / K * beta * K / 10.0
+    with dg.Engine(precision=dg.FP64, lam=lam) as e:
+        e.upload(T, FI, Y, beta)
+        e.estep(True, 1.7)
+        G, RT = e.stats()
+        b = e.mstep()
+        W, Yn, _ = e.download()
+    Wr = np.linalg.solve(FI.T @ (FI * G[:, None]) + lam / beta * np.eye(M1), FI.T @ RT)
+    Yr = FI @ Wr
+    assert np.abs(W - Wr).max() <= 1e-10 * np.abs(Wr).max()
+    assert np.abs(Yn - Yr).max() <= 1e-10 * np.abs(Yr).max()
+    s = (T * T).sum() - 2 * (Yr * RT).sum() + (G * (Yr * Yr).sum(1)).sum()
+    assert b == pytest.approx(N * D / s, rel=1e-10)
