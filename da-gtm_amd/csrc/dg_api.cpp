@@ -125,7 +125,7 @@ int alloc_kstate(dg_ctx *c) {
         (rc = dalloc(c, &c->partRT, c->partRT_len)) ||
         (rc = dalloc(c, &c->partG, (size_t)c->NC * K + (size_t)3 * dg_pass1_wgs(N))) ||
         (rc = dalloc(c, &c->partAB, std::max((size_t)c->nchAB * ((size_t)M1 * M1 + (size_t)M1 * D),
-                                             (size_t)(K + 63) / 64))))
+                                             (size_t)2 * bk_cdiv(K, kBCentres)))))
         return rc;
     c->partLog64 = c->partG + (size_t)c->NC * K;
     DG_HIP(c, hipMemsetAsync(c->Y64, 0, (size_t)K * ld * sizeof(double), c->stream));
@@ -444,10 +444,6 @@ int dg_mstep(dg_ctx *c, double *beta_out) {
     if (!c->loaded || !c->have_estep) return dg_fail(c, DG_ESTATE, "dg_mstep needs a dg_estep first");
     int rc;
     if ((rc = select_device(c)) || (rc = due_stats(c))) return rc;
-    // the G of this M-step is the one the critical-temperature search reads
-    // (vggsub of dagtm.cxx:1715, still set when the next E-step converges)
-    DG_HIP(c, hipMemcpyAsync(c->Gm, c->G, (size_t)c->K * sizeof(double),
-                             hipMemcpyDeviceToDevice, c->stream));
     if (c->timing) DG_HIP(c, hipEventRecord(c->ev[4], c->stream));
     if ((rc = dg_mstep_run(c, 0.0))) return rc;
     if (c->timing) DG_HIP(c, hipEventRecord(c->ev[5], c->stream));
@@ -474,7 +470,7 @@ int dg_mstep(dg_ctx *c, double *beta_out) {
     c->have_w = true;
     const double s = c->sum_tt + c->h_scal[kScalBetaSum];
     c->beta = ((double)c->N * c->D) / s;
-    if (c->mixed() && (rc = dg_mixed_prepare_y(c))) return rc;
+    if (c->mixed() && (rc = dg_mixed_prepare_y(c, true))) return rc;
     if (beta_out) *beta_out = c->beta;
     return DG_OK;
 }

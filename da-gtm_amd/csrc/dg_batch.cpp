@@ -232,7 +232,6 @@ int dg_batch_run_mixed(std::vector<dg_ctx *> &ctx, const dg_anneal_params *param
         b.gr.wg[kind] = r.second;
     };
     whole(b.h_list, n, BK_MAKE_AK);
-    whole(b.h_list, n, BK_ABSMAX_PART);
     whole(b.h_list, n, BK_MAKE_Y16);
     for (BClass &k : b.cls) {
         const auto r1 = add_map(b.h_list + k.first, k.n, BK_REDUCE32);
@@ -245,7 +244,7 @@ int dg_batch_run_mixed(std::vector<dg_ctx *> &ctx, const dg_anneal_params *param
         at_cls.push_back(r2);
         at_cls.push_back(r3);
     }
-    for (int kind : {BK_COPY_G, BK_PART_AB, BK_SUM_AB, BK_PHIW, BK_ROWNORM, BK_BETA_PART})
+    for (int kind : {BK_PART_AB, BK_SUM_AB, BK_CENTRES})
         whole(b.h_list + n, n, kind);
     whole(b.h_list + n, b.nlds, BK_TRSM_LDS);
     DG_HIP(nullptr, hipMalloc((void **)&b.d_map, sizeof(int2) * std::max<size_t>(1, hmap.size())));

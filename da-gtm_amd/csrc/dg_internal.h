@@ -101,6 +101,7 @@ enum {
     kScalBetaSum = 3,   // sum R o dist(Y_new, T)
     kScalJitter = 4,    // jitter used by the last factorisation
     kScalSolveOK = 5,   // 1 if the factorisation succeeded
+    kScalYMax = 6,      // max |Y| (and 7: entries not exact in FP16, of the data)
     kScalCount = 8
 };
 
@@ -109,14 +110,12 @@ enum {
 // each instance with exactly its own workgroup count (bk_count): a device map
 // per launch gives workgroup g its (table index, workgroup within instance).
 enum BKind {
-    BK_MAKE_AK, BK_REDUCE32, BK_ZERO_FIX, BK_COPY_G, BK_PART_AB, BK_SUM_AB, BK_TRSM_LDS,
-    BK_PHIW, BK_ROWNORM, BK_BETA_PART, BK_ABSMAX_PART, BK_MAKE_Y16, BK_BLOCK_LISTS, BK_COUNT
+    BK_MAKE_AK, BK_REDUCE32, BK_ZERO_FIX, BK_PART_AB, BK_SUM_AB, BK_TRSM_LDS, BK_CENTRES,
+    BK_MAKE_Y16, BK_BLOCK_LISTS, BK_COUNT
 };
 // tile sizes the flat grids are counted in (checked against the kernels)
 constexpr int kBRK = 64, kBRD = 16;     // k_reduce32: centres x dims per workgroup
-constexpr int kBGT = 64;                 // M-step products: output tile
-constexpr int kBBetaWG = 64;             // k_beta_part: centres per workgroup
-constexpr int kBAmaxWG = 256;            // k_absmax_part: most workgroups
+constexpr int kBCentres = 16;            // k_centres: centres per workgroup
 // One instance of a batched step, as the batched kernels read it from a
 // device table: the shape, the device buffers of its context and the
 // parameters of the current step.  Built on the host from each context.
@@ -136,7 +135,7 @@ struct BInst {
     int screen;                    // pass 1 screens tiles
     int2 *brange;                  // pass-2 block runs per (chunk, group)
     float skipBelow;
-    double *mscal, *partLog, *amaxPart;
+    double *mscal, *partLog;
     // step parameters
     float beta_f, it;
     int isDA, two, do_e, do_m;
@@ -157,18 +156,11 @@ __host__ __device__ inline int bk_count(const BInst &I, int kind) {
         case BK_MAKE_AK: return cdiv(I.Kp, 256);
         case BK_REDUCE32: return cdiv(I.K, kBRK) * cdiv(I.D, kBRD);
         case BK_ZERO_FIX: return I.D;
-        case BK_COPY_G: return cdiv(I.K, 256);
         case BK_PART_AB:
             return cdiv(I.M1, dg_ab_tile(I.M1)) * cdiv(I.M1 + I.D, dg_ab_tile(I.M1)) * I.nchAB;
-        case BK_SUM_AB: return cdiv((long)I.M1 * I.M1 + (long)I.M1 * I.D, 256);
+        case BK_SUM_AB: return cdiv((long)I.M1 * I.M1 + (long)I.M1 * I.D, 256) + cdiv(I.K, 256);
         case BK_TRSM_LDS: return cdiv(I.D, 32);
-        case BK_PHIW: return cdiv(I.K, kBGT) * cdiv(I.D, kBGT);
-        case BK_ROWNORM: return cdiv(I.K, 256);
-        case BK_BETA_PART: return cdiv(I.K, kBBetaWG);
-        case BK_ABSMAX_PART: {
-            const long w = ((long)I.K * I.D + 4095) / 4096;
-            return (int)(w < kBAmaxWG ? w : kBAmaxWG);
-        }
+        case BK_CENTRES: return cdiv(I.K, kBCentres);
         case BK_MAKE_Y16: return cdiv(I.Kp, 4);
         case BK_BLOCK_LISTS: return (I.Kp / 128) * I.NC;
         default: return 0;
@@ -260,7 +252,8 @@ int dg_mixed_prepare_t(dg_ctx *ctx);
 // largest useful one (both multiples of 8).
 long dg_mixed_nc_limits(const dg_ctx *ctx, long *lo, long *hi);
 int dg_mixed_nc(const dg_ctx *ctx);   // chunk count in use
-int dg_mixed_prepare_y(dg_ctx *ctx);
+// the FP16 split of the centres; have_max: scal[kScalYMax] is set
+int dg_mixed_prepare_y(dg_ctx *ctx, bool have_max = false);
 // orders the mixed path's points by the centre tile holding their largest
 // responsibility under the current centres (one pass-1 sweep), then rebuilds
 // the FP16 operands in that order; DG_MIXED_ORDER=0 keeps the input order

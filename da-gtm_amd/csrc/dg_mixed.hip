@@ -1706,7 +1706,7 @@ __global__ void kb_zero_ints(int *__restrict__ p, int n) {
     if (i < n) p[i] = 0;
 }
 
-static_assert(RK == kBRK && RD == kBRD && kAmaxWG == kBAmaxWG && CT == 128,
+static_assert(RK == kBRK && RD == kBRD && CT == 128,
               "flat-grid tile sizes");
 
 // Flat-grid kernels: workgroup blockIdx.x belongs to instance map[.].x and is
@@ -1752,28 +1752,12 @@ __global__ __launch_bounds__(NTH) void kb_block_ranges(const BInst *__restrict__
     block_range_body(m.y, I.bnd, I.Np, I.CL, I.Kp / CT, I.skipBelow, I.brange);
 }
 
-__global__ __launch_bounds__(256) void kb_absmax_part(const BInst *__restrict__ tab,
-                                                      const int2 *__restrict__ map) {
-    const int2 m = map[blockIdx.x];
-    const BInst &I = tab[m.x];
-    if (!I.do_m) return;
-    k_absmax_part_body(m.y, 0, 0, bk_count(I, BK_ABSMAX_PART), I.Y64, (long)I.K, I.ldt, I.D,
-                       I.amaxPart);
-}
-
-__global__ __launch_bounds__(256) void kb_absmax_final(const BInst *__restrict__ tab,
-                                                       const int *__restrict__ list) {
-    const BInst &I = tab[list[blockIdx.x]];
-    if (!I.do_m) return;
-    k_absmax_final_body(0, 0, 0, 1, I.amaxPart, bk_count(I, BK_ABSMAX_PART), I.scal + 6);
-}
-
 __global__ __launch_bounds__(256) void kb_make_y16(const BInst *__restrict__ tab,
                                                    const int2 *__restrict__ map) {
     const int2 m = map[blockIdx.x];
     const BInst &I = tab[m.x];
     if (!I.do_m) return;
-    k_make_y16_body(m.y, 0, 0, 0, I.Y64, I.ldt, I.K, I.Kp, I.D, I.ldh, I.scal + 6, I.Y16,
+    k_make_y16_body(m.y, 0, 0, 0, I.Y64, I.ldt, I.K, I.Kp, I.D, I.ldh, I.scal + kScalYMax, I.Y16,
                     I.yy32, I.mscal);
 }
 
@@ -1984,12 +1968,12 @@ int dg_mixed_prepare_t(dg_ctx *c) {
                        c->D, b->amaxPart);
     DG_HIP(c, hipGetLastError());
     hipLaunchKernelGGL(k_absmax_final, dim3(1), dim3(256), 0, c->stream, b->amaxPart, kAmaxWG,
-                       c->scal + 6);
+                       c->scal + kScalYMax);
     DG_HIP(c, hipGetLastError());
     DG_HIP(c, hipMemcpyAsync(c->h_scal, c->scal, kScalCount * sizeof(double),
                              hipMemcpyDeviceToHost, c->stream));
     DG_HIP(c, hipStreamSynchronize(c->stream));
-    const double amax = c->h_scal[6], inexact = c->h_scal[7];
+    const double amax = c->h_scal[kScalYMax], inexact = c->h_scal[kScalYMax + 1];
     c->t_exact = (inexact == 0.0 && amax <= 2048.0) ? 1 : 0;
     b->TT = c->t_exact ? 1 : 2;
     if (b->TT == 2 && KS > 8)
@@ -2098,18 +2082,20 @@ int dg_mixed_order(dg_ctx *c) {
     return build_t16(c, b);
 }
 
-int dg_mixed_prepare_y(dg_ctx *c) {
+int dg_mixed_prepare_y(dg_ctx *c, bool have_max) {
     MixedBufs *b = mb(c);
     if (!b || !c->mixed_ready) return dg_fail(c, DG_ESTATE, "mixed buffers not prepared");
-    const int nwg = (int)std::min<long>(kAmaxWG, ((long)c->K * c->D + 4095) / 4096);
-    hipLaunchKernelGGL(k_absmax_part, dim3((unsigned)nwg), dim3(256), 0, c->stream, c->Y64,
-                       (long)c->K, c->ldt, c->D, b->amaxPart);
-    DG_HIP(c, hipGetLastError());
-    hipLaunchKernelGGL(k_absmax_final, dim3(1), dim3(256), 0, c->stream, b->amaxPart, nwg,
-                       c->scal + 6);
-    DG_HIP(c, hipGetLastError());
+    if (!have_max) {
+        const int nwg = (int)std::min<long>(kAmaxWG, ((long)c->K * c->D + 4095) / 4096);
+        hipLaunchKernelGGL(k_absmax_part, dim3((unsigned)nwg), dim3(256), 0, c->stream, c->Y64,
+                           (long)c->K, c->ldt, c->D, b->amaxPart);
+        DG_HIP(c, hipGetLastError());
+        hipLaunchKernelGGL(k_absmax_final, dim3(1), dim3(256), 0, c->stream, b->amaxPart, nwg,
+                           c->scal + kScalYMax);
+        DG_HIP(c, hipGetLastError());
+    }
     hipLaunchKernelGGL(k_make_y16, dim3((unsigned)((b->Kp + 3) / 4)), dim3(256), 0, c->stream,
-                       c->Y64, c->ldt, c->K, b->Kp, c->D, c->ldh, c->scal + 6, b->Y16, c->yy32,
+                       c->Y64, c->ldt, c->K, b->Kp, c->D, c->ldh, c->scal + kScalYMax, b->Y16, c->yy32,
                        b->mscal);
     DG_HIP(c, hipGetLastError());
     return DG_OK;
@@ -2159,7 +2145,7 @@ int dg_batch_fill_mixed(const dg_ctx *c, BInst *I) {
     I->screen = b->screen ? 1 : 0;
     I->brange = b->brange;
     I->skipBelow = skip_below(32 * ((16 * b->KS + 31) / 32) > c->D);
-    I->mscal = b->mscal; I->partLog = b->partLog; I->amaxPart = b->amaxPart;
+    I->mscal = b->mscal; I->partLog = b->partLog;
     return DG_OK;
 }
 
@@ -2212,9 +2198,6 @@ int dg_batch_estep(hipStream_t st, const BInst *tab, const int *list, int n, con
 int dg_batch_prepare_y(hipStream_t st, const BInst *tab, const int *list, int n,
                        const BGrids &gr) {
     if (n <= 0) return DG_OK;
-    hipLaunchKernelGGL(kb_absmax_part, dim3((unsigned)gr.wg[BK_ABSMAX_PART]), dim3(256), 0, st, tab,
-                       gr.map[BK_ABSMAX_PART]);
-    hipLaunchKernelGGL(kb_absmax_final, dim3((unsigned)n), dim3(256), 0, st, tab, list);
     hipLaunchKernelGGL(kb_make_y16, dim3((unsigned)gr.wg[BK_MAKE_Y16]), dim3(256), 0, st, tab,
                        gr.map[BK_MAKE_Y16]);
     return hipGetLastError() == hipSuccess ? DG_OK : DG_EHIP;

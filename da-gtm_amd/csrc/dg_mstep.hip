@@ -405,9 +405,6 @@ __device__ __forceinline__ d4 mfma64(double a, double b, d4 c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
-// Tiles of the M-step's products: 64 x 64 results to a workgroup.
-constexpr int GT = 64, GK = 16;
-
 // A tile of [A | B] holds nothing that is read: all of it above A's diagonal
 // (the factorisation takes the lower triangle).
 __device__ __forceinline__ bool upper_tile(int ti, int tj, int M1) {
@@ -520,13 +517,22 @@ __global__ __launch_bounds__(256, 2) void k_partAB(const double *__restrict__ FI
 }
 
 // A0 / B from the chunk partials, summed in chunk order (A0 without the tiles
-// that k_partAB leaves out).
+// that k_partAB leaves out); the workgroups after those copy G to Gm, which the
+// critical-temperature search reads (vggsub of dagtm.cxx:1715, still set when
+// the next E-step converges).
 __device__ __forceinline__ void k_sumAB_body(
     const int bx, const int by, const int bz, const int gx, const double *__restrict__ part,
-    int nch, int M1, int D, double *__restrict__ A0, double *__restrict__ B) {
+    int nch, int M1, int D, double *__restrict__ A0, double *__restrict__ B, int K,
+    const double *__restrict__ G, double *__restrict__ Gm) {
     const int NCOL = M1 + D;
     const long E = (long)M1 * NCOL;
-    const long e = (long)bx * blockDim.x + threadIdx.x;
+    const long e = (long)bx * 256 + threadIdx.x;
+    const int nE = bk_cdiv(E, 256);
+    if (bx >= nE) {
+        const int k = (bx - nE) * 256 + threadIdx.x;
+        if (k < K) Gm[k] = G[k];
+        return;
+    }
     if (e >= E) return;
     const int i = (int)(e / NCOL), j = (int)(e % NCOL);
     if (j < M1 && upper_tile(i / dg_ab_tile(M1), j / dg_ab_tile(M1), M1)) return;
@@ -545,9 +551,12 @@ __device__ __forceinline__ void k_sumAB_body(
     else B[(long)i * D + (j - M1)] = s;
 }
 
-__global__ void k_sumAB(const double *__restrict__ part, int nch, int M1, int D,
-                        double *__restrict__ A0, double *__restrict__ B) {
-    k_sumAB_body(blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, part, nch, M1, D, A0, B);
+__global__ __launch_bounds__(256) void k_sumAB(const double *__restrict__ part, int nch, int M1,
+                                               int D, double *__restrict__ A0,
+                                               double *__restrict__ B, int K,
+                                               const double *__restrict__ G,
+                                               double *__restrict__ Gm) {
+    k_sumAB_body(blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, part, nch, M1, D, A0, B, K, G, Gm);
 }
 
 constexpr int kLdsN = 126;   // largest M+1 whose factor fits in LDS
@@ -827,161 +836,199 @@ __global__ __launch_bounds__(kTrsmNT) void k_trsm_lds(const double *__restrict__
                                        nrhs, W, scal);
 }
 
-// Y = FI W into the padded FP64 layout (K x ld, columns >= D untouched):
-// 64 x 64 output tiles over (centre, d), the M1 inner dimension in steps of 16.
-__device__ __forceinline__ void k_phiw_body(
-    const int bx, const int by, const int bz, const int gx, const double *__restrict__ FI,
-    const double *__restrict__ W, int K, int M1, int D, int ld, double *__restrict__ Y) {
-    __shared__ double As[GK][GT + 1], Bs[GK][GT];
-    const int k0 = bx * GT, d0 = by * GT;
-    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-    double acc[4][4];
+// The new centres and what the M-step takes from them, sixteen centres to a
+// workgroup:
+//   Y = FI W into the padded layout (K x ld, columns >= D untouched),
+//   yy_k = |y_k|^2, a chain in d,
+//   part[bx] = sum over its centres of G_k |y_k|^2 - 2 y_k . RT_k, in order
+//   (with part null, Y and yy only),
+//   amax[bx] = max |Y| over them (with amax null: not wanted).
+// FI's rows pass through LDS 64 functions at a time, the wave's share of W's
+// columns (16 d-blocks w, w + 4, w + 8) straight from L2.  D <= 192.
+// Bound by latency at M1 = 126 (32 steps of one load and one MFMA chain each) and
+// by the FP64 pipe at M1 = 1001.  K = 8000, M1 = 126, D = 166: 23 us (Y, norms,
+// sums and maximum as five kernels, the first with 4 x 4 tiles of FMAs: 71);
+// K = 32768, M1 = 1001: 344 us (541); K = 400, M1 = 26, D = 12: 7 us (20, without
+// a maximum).
+constexpr int CW = 16;                             // centres per workgroup
+__device__ __forceinline__ void k_centres_body(
+    const int bx, const double *__restrict__ FI, const double *__restrict__ W, int K, int M1, int D,
+    int ld, const double *__restrict__ G, const double *__restrict__ RT, double *__restrict__ Y,
+    double *__restrict__ yy, double *__restrict__ part, double *__restrict__ amax) {
+    constexpr int FC = 64, FP = FC + 4;            // functions per chunk, row stride in LDS
+    constexpr int YP = 192 + 2;
+    __shared__ double Fs[2][CW][FP];
+    __shared__ double Yt[CW][YP];
+    __shared__ double nrm[CW], dots[CW], mx[4];
+    const int tid = threadIdx.x, l = tid & 63, w = tid >> 6, j = l & 15, g = l >> 4;
+    const int k0 = bx * CW;
+    const int nd = (D + 15) / 16;                  // d-blocks, w, w + 4, w + 8 this wave's
+    const int sr = tid >> 4, sp = tid & 15;        // staging: 16 threads to a row of FI
+    const double *frow = FI + (long)min(k0 + sr, K - 1) * M1;
+    double rf[4];
+    auto load = [&](int f0) {
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = 0.0;
-    // the next step's operands are loaded into registers while this step's
-    // are multiplied from LDS (four elements of each per thread)
-    static_assert(GK * GT == 4 * 256, "four staged elements per thread");
-    double ra[4], rb[4];
-    auto gload = [&](int ib) {
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int e = tid + 256 * u;
-            const int row = e / GK, ii = e % GK;          // FI rows read along i
-            const int k = k0 + row, i = ib + ii;
-            ra[u] = (k < K && i < M1) ? FI[(long)k * M1 + i] : 0.0;
-            const int kk = e / GT, col = e % GT;          // W rows read along d
-            const int i2 = ib + kk, d = d0 + col;
-            rb[u] = (i2 < M1 && d < D) ? W[(long)i2 * D + d] : 0.0;
+        for (int i = 0; i < 4; ++i) {
+            const int f = f0 + sp + 16 * i;
+            rf[i] = (f < M1) ? frow[f] : 0.0;
         }
     };
-    gload(0);
-    for (int ib = 0; ib < M1; ib += GK) {
+    auto store = [&](int b) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int e = tid + 256 * u;
-            As[e % GK][e / GK] = ra[u];
-            Bs[e / GT][e % GT] = rb[u];
-        }
-        __syncthreads();
-        if (ib + GK < M1) gload(ib + GK);
+        for (int i = 0; i < 4; ++i) Fs[b][sr][sp + 16 * i] = rf[i];
+    };
+    int col[3];
 #pragma unroll
-        for (int kk = 0; kk < GK; ++kk) {
-            double av[4], bv[4];
+    for (int q = 0; q < 3; ++q) col[q] = min(16 * (w + 4 * q) + j, D - 1);
+    d4 acc[3];
 #pragma unroll
-            for (int a = 0; a < 4; ++a) av[a] = As[kk][ty + 16 * a];
-#pragma unroll
-            for (int b = 0; b < 4; ++b) bv[b] = Bs[kk][tx + 16 * b];
-#pragma unroll
-            for (int a = 0; a < 4; ++a)
-#pragma unroll
-                for (int b = 0; b < 4; ++b) acc[a][b] = fma(av[a], bv[b], acc[a][b]);
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            const int k = k0 + ty + 16 * a, d = d0 + tx + 16 * b;
-            if (k < K && d < D) Y[(long)k * ld + d] = acc[a][b];
-        }
-}
-
-__global__ __launch_bounds__(256) void k_phiw(const double *__restrict__ FI,
-                                              const double *__restrict__ W, int K, int M1, int D,
-                                              int ld, double *__restrict__ Y) {
-    k_phiw_body(blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, FI, W, K, M1, D, ld, Y);
-}
-
-// Per-workgroup partials of sum_k (G_k |y_k|^2 - 2 y_k . RT_k) over 64
-// centres each (one wave per centre, 16 centres per wave); k_beta_final sums
-// them in workgroup order into scal[kScalBetaSum].
-constexpr int kBetaWG = 64;
-__device__ __forceinline__ void k_beta_part_body(
-    const int bx, const int by, const int bz, const int gx, const double *__restrict__ Y,
-    int ld, const double *__restrict__ yy, const double *__restrict__ G,
-    const double *__restrict__ RT, int K, int D, double *__restrict__ part) {
-    __shared__ double s[4];
-    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-    double acc = 0.0;                              // lane 0: this wave's sum
-    const int kw = bx * kBetaWG + w * (kBetaWG / 4);
-    constexpr int DM = 3;
-    if (D <= 64 * DM) {
-        // the next centre's operands are loaded while this one's dot product
-        // is reduced (same products and sums as the loop below)
-        double yv[DM], rv[DM], gy[2];
-        auto load = [&](int k) {
-#pragma unroll
-            for (int m = 0; m < DM; ++m) {
-                const int d = l + 64 * m;
-                const bool in = k < K && d < D;
-                yv[m] = in ? Y[(long)k * ld + d] : 0.0;
-                rv[m] = in ? RT[(long)k * D + d] : 0.0;
-            }
-            gy[0] = (k < K) ? G[k] : 0.0;
-            gy[1] = (k < K) ? yy[k] : 0.0;
-        };
-        load(kw);
-        for (int q = 0; q < kBetaWG / 4; ++q) {
-            const int k = kw + q;
-            if (k >= K) break;
-            double y[DM], r[DM];
-#pragma unroll
-            for (int m = 0; m < DM; ++m) { y[m] = yv[m]; r[m] = rv[m]; }
-            const double gk = gy[0], yk = gy[1];
-            if (q + 1 < kBetaWG / 4) load(k + 1);
-            double dot = 0.0;
-#pragma unroll
-            for (int m = 0; m < DM; ++m)
-                if (l + 64 * m < D) dot = fma(y[m], r[m], dot);
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) dot += __shfl_xor(dot, o);
-            acc += gk * yk - 2.0 * dot;
-        }
-    } else {
-        for (int q = 0; q < kBetaWG / 4; ++q) {
-            const int k = kw + q;
-            if (k >= K) break;
-            double dot = 0.0;
-            for (int d = l; d < D; d += 64) dot = fma(Y[(long)k * ld + d], RT[(long)k * D + d], dot);
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) dot += __shfl_xor(dot, o);
-            acc += G[k] * yy[k] - 2.0 * dot;
-        }
-    }
-    if (l == 0) s[w] = acc;
+    for (int q = 0; q < 3; ++q) acc[q] = d4{0.0, 0.0, 0.0, 0.0};
+    load(0);
+    store(0);
     __syncthreads();
-    if (threadIdx.x == 0) part[bx] = (s[0] + s[1]) + (s[2] + s[3]);
+    int b = 0;
+    for (int f0 = 0; f0 < M1; f0 += FC, b ^= 1) {
+        if (f0 + FC < M1) load(f0 + FC);
+        const int steps = (min(FC, M1 - f0) + 3) / 4;
+        if (w < nd) {
+            // (functions past the end: FI's are 0 in LDS, W's row the last one)
+            constexpr int U = 4;
+            double wv[U][3];
+            auto loadw = [&](int s0) {
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const double *wr = W + (long)min(f0 + 4 * (s0 + u) + g, M1 - 1) * D;
+#pragma unroll
+                    for (int q = 0; q < 3; ++q)
+                        if (q == 0 || w + 4 * q < nd) wv[u][q] = wr[col[q]];
+                }
+            };
+            loadw(0);
+            for (int s0 = 0; s0 < steps; s0 += U) {
+                double av[U], bv[U][3];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int f = 4 * (s0 + u) + g;
+                    av[u] = Fs[b][j][f < FC ? f : 0];
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) bv[u][q] = wv[u][q];
+                }
+                if (s0 + U < steps) loadw(s0 + U);
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    if (s0 + u < steps)
+#pragma unroll
+                        for (int q = 0; q < 3; ++q)
+                            if (q == 0 || w + 4 * q < nd) acc[q] = mfma64(av[u], bv[u][q], acc[q]);
+            }
+        }
+        if (f0 + FC < M1) store(b ^ 1);
+        __syncthreads();
+    }
+    double top = 0.0;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        const int d = 16 * (w + 4 * q) + j;
+        if (d < D)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int c = 4 * r + g, k = k0 + c;
+                Yt[c][d] = acc[q][r];
+                if (k < K) {
+                    Y[(long)k * ld + d] = acc[q][r];
+                    top = fmax(top, fabs(acc[q][r]));
+                }
+            }
+    }
+    if (amax) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) top = fmax(top, __shfl_xor(top, o));
+        if (l == 0) mx[w] = top;
+    }
+    __syncthreads();
+    // |y|^2: the last wave, one centre to a lane
+    if (w == 3 && l < CW) {
+        double s = 0.0;
+        int d = 0;
+        for (; d + 8 <= D; d += 8) {
+            double v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = Yt[l][d + u];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) s = fma(v[u], v[u], s);
+        }
+        for (; d < D; ++d) s = fma(Yt[l][d], Yt[l][d], s);
+        nrm[l] = s;
+        if (k0 + l < K) yy[k0 + l] = s;
+    }
+    if (!part) return;
+    // y . RT: a wave to a centre, lanes along d, waves 0 .. 2 in turn (wave 3
+    // once it has the norms)
+    for (int c = w; c < CW; c += 4) {
+        const int k = k0 + c;
+        double dot = 0.0;
+        if (k < K)
+            for (int d = l; d < D; d += 64) dot = fma(Yt[c][d], RT[(long)k * D + d], dot);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) dot += __shfl_xor(dot, o);
+        if (l == 0) dots[c] = dot;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        double s = 0.0;
+        for (int c = 0; c < CW; ++c) {
+            if (k0 + c >= K) break;
+            s += G[k0 + c] * nrm[c] - 2.0 * dots[c];
+        }
+        part[bx] = s;
+        if (amax) amax[bx] = fmax(fmax(mx[0], mx[1]), fmax(mx[2], mx[3]));
+    }
 }
 
-__global__ __launch_bounds__(256) void k_beta_part(const double *__restrict__ Y, int ld,
-                                                   const double *__restrict__ yy,
-                                                   const double *__restrict__ G,
-                                                   const double *__restrict__ RT, int K, int D,
-                                                   double *__restrict__ part) {
-    k_beta_part_body(blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, Y, ld, yy, G, RT, K, D, part);
+__global__ __launch_bounds__(256, 2) void k_centres(
+    const double *__restrict__ FI, const double *__restrict__ W, int K, int M1, int D, int ld,
+    const double *__restrict__ G, const double *__restrict__ RT, double *__restrict__ Y,
+    double *__restrict__ yy, double *__restrict__ part, double *__restrict__ amax) {
+    k_centres_body(blockIdx.x, FI, W, K, M1, D, ld, G, RT, Y, yy, part, amax);
 }
 
-__device__ __forceinline__ void k_beta_final_body(
-    const int bx, const int by, const int bz, const int gx, const double *__restrict__ part,
-    int n, double *__restrict__ scal) {
-    __shared__ double s[256];
-    double a = 0.0;
-    for (int i = threadIdx.x; i < n; i += 256) a += part[i];
+// scal[kScalBetaSum] = the sum of the n sixteen-centre partials, four by four
+// (64 centres) and then as a tree; with amax, scal[kScalYMax] = its largest.
+__device__ __forceinline__ void k_beta_final_body(const double *__restrict__ part, int n,
+                                                  const double *__restrict__ amax,
+                                                  double *__restrict__ scal) {
+    __shared__ double s[256], m[256];
+    double a = 0.0, top = 0.0;
+    for (int i = 4 * threadIdx.x; i < n; i += 4 * 256) {
+        double v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = (i + u < n) ? part[i + u] : 0.0;
+        a += (v[0] + v[1]) + (v[2] + v[3]);
+        if (amax)
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (i + u < n) top = fmax(top, amax[i + u]);
+    }
     s[threadIdx.x] = a;
+    m[threadIdx.x] = top;
     __syncthreads();
     for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
+        if ((int)threadIdx.x < w) {
+            s[threadIdx.x] += s[threadIdx.x + w];
+            m[threadIdx.x] = fmax(m[threadIdx.x], m[threadIdx.x + w]);
+        }
         __syncthreads();
     }
-    if (threadIdx.x == 0) scal[kScalBetaSum] = s[0];
+    if (threadIdx.x == 0) {
+        scal[kScalBetaSum] = s[0];
+        if (amax) scal[kScalYMax] = m[0];
+    }
 }
 
 __global__ __launch_bounds__(256) void k_beta_final(const double *__restrict__ part, int n,
+                                                    const double *__restrict__ amax,
                                                     double *__restrict__ scal) {
-    k_beta_final_body(blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, part, n, scal);
+    k_beta_final_body(part, n, amax, scal);
 }
 
 // ---------------------------------------------------------------- batched
@@ -991,18 +1038,10 @@ __global__ __launch_bounds__(256) void k_beta_final(const double *__restrict__ p
 // workgroups past them return before any barrier.  Every instance computes
 // exactly what its own single-instance launch computes.
 
-static_assert(GT == kBGT && kBetaWG == kBBetaWG, "flat-grid tile sizes");
+static_assert(CW == kBCentres, "flat-grid tile sizes");
 
 // Flat-grid kernels: workgroup blockIdx.x belongs to instance map[.].x and is
 // its workgroup map[.].y (grids sized by bk_count for each instance).
-__global__ __launch_bounds__(256) void kb_copy_g(const BInst *__restrict__ tab,
-                                                 const int2 *__restrict__ map) {
-    const int2 m = map[blockIdx.x];
-    const BInst &I = tab[m.x];
-    const int k = m.y * 256 + threadIdx.x;
-    if (I.do_m && k < I.K) I.Gm[k] = I.G[k];
-}
-
 __global__ __launch_bounds__(256, 2) void kb_partAB(const BInst *__restrict__ tab,
                                                  const int2 *__restrict__ map) {
     const int2 m = map[blockIdx.x];
@@ -1015,11 +1054,11 @@ __global__ __launch_bounds__(256, 2) void kb_partAB(const BInst *__restrict__ ta
     else k_partAB_body<4>(x, y, z, 0, I.FI, I.G, I.RT, I.K, I.M1, I.D, kc, I.partAB);
 }
 
-__global__ void kb_sumAB(const BInst *__restrict__ tab, const int2 *__restrict__ map) {
+__global__ __launch_bounds__(256) void kb_sumAB(const BInst *__restrict__ tab, const int2 *__restrict__ map) {
     const int2 m = map[blockIdx.x];
     const BInst &I = tab[m.x];
     if (!I.do_m) return;
-    k_sumAB_body(m.y, 0, 0, 0, I.partAB, I.nchAB, I.M1, I.D, I.A0, I.Bm);
+    k_sumAB_body(m.y, 0, 0, 0, I.partAB, I.nchAB, I.M1, I.D, I.A0, I.Bm, I.K, I.G, I.Gm);
 }
 
 __global__ __launch_bounds__(1024) void kb_chol_lds(const BInst *__restrict__ tab,
@@ -1044,35 +1083,21 @@ __global__ __launch_bounds__(1024) void kb_chol_solve(const BInst *__restrict__ 
     k_chol_solve_body(0, 0, 0, 1, I.A0, I.A, I.M1, I.ridge, I.Bm, I.D, I.W, I.scal);
 }
 
-__global__ __launch_bounds__(256) void kb_phiw(const BInst *__restrict__ tab,
-                                               const int2 *__restrict__ map) {
+__global__ __launch_bounds__(256, 2) void kb_centres(const BInst *__restrict__ tab,
+                                                     const int2 *__restrict__ map) {
     const int2 m = map[blockIdx.x];
     const BInst &I = tab[m.x];
     if (!I.do_m) return;
-    const int nx = (I.K + GT - 1) / GT;
-    k_phiw_body(m.y % nx, m.y / nx, 0, 0, I.FI, I.W, I.K, I.M1, I.D, I.ldt, I.Y64);
-}
-
-__global__ void kb_rownorm_y(const BInst *__restrict__ tab, const int2 *__restrict__ map) {
-    const int2 m = map[blockIdx.x];
-    const BInst &I = tab[m.x];
-    if (!I.do_m) return;
-    k_rownorm_body(m.y, 0, 0, 0, I.Y64, I.K, I.ldt, I.D, I.yy);
-}
-
-__global__ __launch_bounds__(256) void kb_beta_part(const BInst *__restrict__ tab,
-                                                    const int2 *__restrict__ map) {
-    const int2 m = map[blockIdx.x];
-    const BInst &I = tab[m.x];
-    if (!I.do_m) return;
-    k_beta_part_body(m.y, 0, 0, 0, I.Y64, I.ldt, I.yy, I.G, I.RT, I.K, I.D, I.partAB);
+    k_centres_body(m.y, I.FI, I.W, I.K, I.M1, I.D, I.ldt, I.G, I.RT, I.Y64, I.yy, I.partAB,
+                   I.partAB + bk_cdiv(I.K, CW));
 }
 
 __global__ __launch_bounds__(256) void kb_beta_final(const BInst *__restrict__ tab,
                                                      const int *__restrict__ list) {
     const BInst &I = tab[list[blockIdx.x]];
     if (!I.do_m) return;
-    k_beta_final_body(0, 0, 0, 1, I.partAB, bk_count(I, BK_BETA_PART), I.scal);
+    const int n = bk_cdiv(I.K, CW);
+    k_beta_final_body(I.partAB, n, I.partAB + n, I.scal);
 }
 
 }  // namespace
@@ -1110,11 +1135,11 @@ int dg_sum_into(dg_ctx *c, const double *v, long n, int slot) {
 }
 
 int dg_centres_from_w(dg_ctx *c) {
-    const int D = c->D, K = c->K;
-    hipLaunchKernelGGL(k_phiw, dim3((unsigned)((K + GT - 1) / GT), (unsigned)((D + GT - 1) / GT)),
-                       dim3(256), 0, c->stream, c->FI, c->W, K, c->M1, D, c->ldt, c->Y64);
+    hipLaunchKernelGGL(k_centres, dim3((unsigned)bk_cdiv(c->K, CW)), dim3(256), 0, c->stream, c->FI,
+                       c->W, c->K, c->M1, c->D, c->ldt, nullptr, nullptr, c->Y64, c->yy, nullptr,
+                       nullptr);
     DG_HIP(c, hipGetLastError());
-    return dg_rownorms(c, c->Y64, K, c->ldt, D, c->yy);
+    return DG_OK;
 }
 
 // (A0 + (ridge + jit) I) W = Bm for M + 1 > 126 by the blocked kernels;
@@ -1177,8 +1202,8 @@ int dg_mstep_run(dg_ctx *c, double jitter) {
         hipLaunchKernelGGL(k_partAB<4>, abgrid, dim3(256), 0, c->stream, c->FI, c->G, c->RT, K, M1, D,
                            kc, nch, c->partAB);
     DG_HIP(c, hipGetLastError());
-    hipLaunchKernelGGL(k_sumAB, dim3((unsigned)((E + 255) / 256)), dim3(256), 0, c->stream,
-                       c->partAB, nch, M1, D, c->A0, c->Bm);
+    hipLaunchKernelGGL(k_sumAB, dim3((unsigned)(bk_cdiv(E, 256) + bk_cdiv(K, 256))), dim3(256), 0,
+                       c->stream, c->partAB, nch, M1, D, c->A0, c->Bm, K, c->G, c->Gm);
     DG_HIP(c, hipGetLastError());
     const double ridge = (c->cfg.lambda > 0.0) ? c->cfg.lambda / c->beta : 0.0;
     if (M1 <= kLdsN) {
@@ -1194,14 +1219,13 @@ int dg_mstep_run(dg_ctx *c, double jitter) {
         if (rc) return rc;
     }
     DG_HIP(c, hipGetLastError());
-    int rc = dg_centres_from_w(c);
-    if (rc) return rc;
-    // beta partials reuse the (now consumed) A/B partial buffer
-    const int nb = (K + kBetaWG - 1) / kBetaWG;
-    hipLaunchKernelGGL(k_beta_part, dim3((unsigned)nb), dim3(256), 0, c->stream, c->Y64, c->ldt,
-                       c->yy, c->G, c->RT, K, D, c->partAB);
+    // the centres' partials reuse the (now consumed) A/B partial buffer
+    const int nb = bk_cdiv(K, CW);
+    double *amax = c->mixed() ? c->partAB + nb : nullptr;
+    hipLaunchKernelGGL(k_centres, dim3((unsigned)nb), dim3(256), 0, c->stream, c->FI, c->W, K, M1, D,
+                       c->ldt, c->G, c->RT, c->Y64, c->yy, c->partAB, amax);
     DG_HIP(c, hipGetLastError());
-    hipLaunchKernelGGL(k_beta_final, dim3(1), dim3(256), 0, c->stream, c->partAB, nb, c->scal);
+    hipLaunchKernelGGL(k_beta_final, dim3(1), dim3(256), 0, c->stream, c->partAB, nb, amax, c->scal);
     DG_HIP(c, hipGetLastError());
     return DG_OK;
 }
@@ -1209,7 +1233,7 @@ int dg_mstep_run(dg_ctx *c, double jitter) {
 // M-step of the instances in list (n of them; nlds with M + 1 <= 126 first in
 // list, the others after), on one stream; gr holds the flat grids over that
 // list (the LDS triangular solves over its first nlds entries).  Each
-// instance's steps are those of dg_mstep_run after the copy of G into Gm.
+// instance's steps are those of dg_mstep_run.
 int dg_batch_mstep(hipStream_t st, const BInst *tab, const int *list, int n, int nlds,
                    const BGrids &gr) {
     if (n <= 0) return DG_OK;
@@ -1217,7 +1241,6 @@ int dg_batch_mstep(hipStream_t st, const BInst *tab, const int *list, int n, int
         hipLaunchKernelGGL(kernel, dim3((unsigned)gr.wg[kind]), dim3(threads), 0, st, tab,
                            gr.map[kind]);
     };
-    flat(kb_copy_g, BK_COPY_G, 256);
     flat(kb_partAB, BK_PART_AB, 256);
     flat(kb_sumAB, BK_SUM_AB, 256);
     if (nlds > 0) {
@@ -1227,9 +1250,7 @@ int dg_batch_mstep(hipStream_t st, const BInst *tab, const int *list, int n, int
     if (n > nlds)
         hipLaunchKernelGGL(kb_chol_solve, dim3((unsigned)(n - nlds)), dim3(1024), 0, st, tab,
                            list + nlds);
-    flat(kb_phiw, BK_PHIW, 256);
-    flat(kb_rownorm_y, BK_ROWNORM, 256);
-    flat(kb_beta_part, BK_BETA_PART, 256);
+    flat(kb_centres, BK_CENTRES, 256);
     hipLaunchKernelGGL(kb_beta_final, dim3((unsigned)n), dim3(256), 0, st, tab, list);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? DG_OK : DG_EHIP;
