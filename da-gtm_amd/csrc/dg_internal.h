@@ -159,7 +159,7 @@ __host__ __device__ inline int bk_count(const BInst &I, int kind) {
         case BK_PART_AB:
             return cdiv(I.M1, dg_ab_tile(I.M1)) * cdiv(I.M1 + I.D, dg_ab_tile(I.M1)) * I.nchAB;
         case BK_SUM_AB: return cdiv((long)I.M1 * I.M1 + (long)I.M1 * I.D, 256) + cdiv(I.K, 256);
-        case BK_TRSM_LDS: return cdiv(I.D, 32);
+        case BK_TRSM_LDS: return cdiv(I.D, 16);
         case BK_CENTRES: return cdiv(I.K, kBCentres);
         case BK_MAKE_Y16: return cdiv(I.Kp, 4);
         case BK_BLOCK_LISTS: return (I.Kp / 128) * I.NC;

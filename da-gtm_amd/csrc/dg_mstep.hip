@@ -10,6 +10,8 @@
 //          sum_n |t_n|^2 - 2 sum_k y_k.RT_k + sum_k G_k |y_k|^2
 //          (exact because every column of R sums to one, mpicomm.c:382-391)
 #include <cmath>
+#include <type_traits>
+#include <utility>
 
 #include "dg_internal.h"
 
@@ -560,7 +562,7 @@ __global__ __launch_bounds__(256) void k_sumAB(const double *__restrict__ part, 
 }
 
 constexpr int kLdsN = 126;   // largest M+1 whose factor fits in LDS
-static_assert(kLdsN <= 128, "the Cholesky and solve kernels give each thread at most 4 rows");
+static_assert(kLdsN <= 128, "a wave holds two rows of a panel per lane, eight 16-row blocks");
 
 // Broadcast lane l's value of x (l wave-uniform) to the whole wavefront.
 __device__ __forceinline__ double lane_bcast(double x, int l) {
@@ -572,24 +574,74 @@ __device__ __forceinline__ double lane_bcast(double x, int l) {
 
 constexpr int kPB = 8;        // panel width of the blocked Cholesky
 
-// Cholesky of A0 + (ridge + jitter) I with the matrix resident in LDS (one
+// put(i, k, A[i][k]) for the lower triangle of the n x n matrix A (n <= 128),
+// rows spread over the workgroup's waves, eight rows' loads in flight
+template <typename Put>
+__device__ __forceinline__ void load_lower(const double *__restrict__ A, int n, Put &&put) {
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    for (int i0 = wv; i0 < n; i0 += 8 * nw) {
+        double v[8][2];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int i = i0 + u * nw;
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                v[u][h] = (i < n && lane + 64 * h <= i) ? A[(long)i * n + lane + 64 * h] : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int i = i0 + u * nw;
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                if (i < n && lane + 64 * h <= i) put(i, lane + 64 * h, v[u][h]);
+        }
+    }
+}
+
+template <int... Is, typename F>
+__device__ __forceinline__ void each_of(std::integer_sequence<int, Is...>, F &&f) {
+    (f(std::integral_constant<int, Is>{}), ...);
+}
+
+// x of the four lanes j + 16 q, q = 0 .. 3, replaced by the one of q = G: the
+// row swaps of v_permlane16_swap leave rows {0, 0, 2, 2} and {1, 1, 3, 3} of a
+// value swapped with itself, v_permlane32_swap its halves.
+template <int G>
+__device__ __forceinline__ double row_bcast(double x) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, x);
+    unsigned h[2] = {(unsigned)u, (unsigned)(u >> 32)};
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const auto a = __builtin_amdgcn_permlane16_swap(h[i], h[i], false, false);
+        const unsigned t = (G & 1) ? (unsigned)a[1] : (unsigned)a[0];
+        const auto b = __builtin_amdgcn_permlane32_swap(t, t, false, false);
+        h[i] = (G & 2) ? (unsigned)b[1] : (unsigned)b[0];
+    }
+    return __builtin_bit_cast(double, ((unsigned long long)h[1] << 32) | h[0]);
+}
+
+// Cholesky of A0 + (ridge + jitter) I with the lower triangle resident in LDS (one
 // workgroup, n <= 126); same pivots and retries as k_chol_solve.  Blocked,
 // right-looking: wave 0 factors each 8-column panel in registers (lane r
 // holds rows p0 + r and p0 + r + 64; the pivot row and the L entries of later
 // panel columns are broadcast with readlane, so the panel needs no barrier),
-// then all waves apply the panel to the trailing lower triangle with 4 x 4
-// register tiles.  Two barriers per panel.  Writes the factor's lower
-// triangle (the rest of L is left unspecified).
+// then all waves apply the panel to the trailing lower triangle, a 16 x 16 tile
+// at a time on matrix instructions (the chain over the panel's columns from 0,
+// subtracted from the tile).  Two barriers per panel.  Writes the factor's lower
+// triangle only.
+// Bound by the panels' chains of square roots and reciprocals, one CU's latency:
+// n = 126: 90 -> 55 us, n = 26: 17 -> 13 (trailing updates by 4 x 4 register
+// tiles over 32 x 32 threads, whatever was left of the triangle).
 __device__ __forceinline__ void k_chol_lds_body(
     const int bx, const int by, const int bz, const int gx, const double *__restrict__ A0,
     double *__restrict__ L, int n, double ridge, double *__restrict__ scal) {
-    __shared__ double As[kLdsN * kLdsN];
-    __shared__ double Pt[kPB][128];                  // the factored panel, transposed
+    __shared__ double As[kLdsN * (kLdsN | 1)];
+    __shared__ double Pt[kPB][128 + 16];             // the factored panel, transposed
     __shared__ double tr;
     __shared__ int bad;
-    const int tid = threadIdx.x, nt = blockDim.x;
-    const int lane = tid & 63, wv = tid >> 6;
-    const int tx = tid & 31, ty = tid >> 5;
+    const int tid = threadIdx.x, nw = blockDim.x >> 6;
+    const int lane = tid & 63, wv = tid >> 6, j = lane & 15, g = lane >> 4;
+    const int ld = n | 1;                            // odd: a column spreads over the banks
     double jit = 0.0;
     int ok = 0;
     for (int attempt = 0; attempt < 9 && !ok; ++attempt) {
@@ -599,10 +651,9 @@ __device__ __forceinline__ void k_chol_lds_body(
         } else if (attempt > 1) {
             jit *= 10.0;
         }
-        for (int e = tid; e < n * n; e += nt) {
-            const int i = e / n, j = e % n;
-            As[e] = A0[e] + ((i == j) ? ridge + jit : 0.0);
-        }
+        load_lower(A0, n, [&](int i, int k, double v) {
+            As[i * ld + k] = v + ((i == k) ? ridge + jit : 0.0);
+        });
         if (tid == 0) bad = 0;
         __syncthreads();
         for (int p0 = 0; p0 < n; p0 += kPB) {
@@ -612,73 +663,60 @@ __device__ __forceinline__ void k_chol_lds_body(
                 double a0[kPB], a1[kPB];
 #pragma unroll
                 for (int c = 0; c < kPB; ++c) {
-                    a0[c] = (c < pn && r0 < n) ? As[r0 * n + p0 + c] : 0.0;
-                    a1[c] = (c < pn && r1 < n) ? As[r1 * n + p0 + c] : 0.0;
+                    a0[c] = (c < pn && r0 < n && c <= lane) ? As[r0 * ld + p0 + c] : 0.0;
+                    a1[c] = (c < pn && r1 < n) ? As[r1 * ld + p0 + c] : 0.0;
                 }
                 bool failed = false;
 #pragma unroll
-                for (int j = 0; j < kPB; ++j) {
-                    if (j < pn && !failed) {
-                        const double piv = lane_bcast(a0[j], j);     // row p0 + j is lane j's
+                for (int q = 0; q < kPB; ++q) {
+                    if (q < pn && !failed) {
+                        const double piv = lane_bcast(a0[q], q);     // row p0 + q is lane q's
                         if (!(piv > 0.0)) {
                             failed = true;                           // the same in every lane
                         } else {
+                            // (rows above the diagonal, lanes < c of column
+                            // c, hold nothing that is read)
                             const double sq = sqrt(piv), inv = 1.0 / sq;
-                            if (lane == j) a0[j] = sq;
-                            else if (lane > j) a0[j] *= inv;
-                            a1[j] *= inv;
+                            a0[q] = (lane == q) ? sq : a0[q] * inv;
+                            a1[q] *= inv;
 #pragma unroll
-                            for (int c = j + 1; c < kPB; ++c) {
-                                if (c < pn) {
-                                    const double lcj = lane_bcast(a0[j], c);   // L[p0 + c][p0 + j]
-                                    if (lane > j) a0[c] = fma(-a0[j], lcj, a0[c]);
-                                    a1[c] = fma(-a1[j], lcj, a1[c]);
-                                }
+                            for (int c = q + 1; c < kPB; ++c) {
+                                const double lcj = lane_bcast(a0[q], c);   // L[p0 + c][p0 + q]
+                                a0[c] = fma(-a0[q], lcj, a0[c]);
+                                a1[c] = fma(-a1[q], lcj, a1[c]);
                             }
                         }
                     }
                 }
+                // (rows past the end are zero: the tiles below need no bounds)
 #pragma unroll
-                for (int c = 0; c < kPB; ++c)
-                    if (c < pn) {
-                        if (r0 < n) { As[r0 * n + p0 + c] = a0[c]; Pt[c][r0 - p0] = a0[c]; }
-                        if (r1 < n) { As[r1 * n + p0 + c] = a1[c]; Pt[c][r1 - p0] = a1[c]; }
-                    }
+                for (int c = 0; c < kPB; ++c) {
+                    if (c < pn && c <= lane && r0 < n) As[r0 * ld + p0 + c] = a0[c];
+                    if (c < pn && r1 < n) As[r1 * ld + p0 + c] = a1[c];
+                    Pt[c][lane] = (r0 < n) ? a0[c] : 0.0;
+                    Pt[c][lane + 64] = (r1 < n) ? a1[c] : 0.0;
+                    if (lane < 16) Pt[c][lane + 128] = 0.0;
+                }
                 if (failed && lane == 0) bad = 1;
             }
             __syncthreads();
             if (bad) break;                                  // read after the barrier: uniform
-            // trailing update A[i][k] -= sum_j L[i][p0 + j] L[k][p0 + j] for
-            // q0 <= k <= i: thread (ty, tx) owns rows q0 + ty + 32 a and columns
-            // q0 + tx + 32 b, read from the transposed panel (consecutive lanes,
-            // consecutive columns: no bank conflicts)
-            const int q0 = p0 + pn;
-            if (q0 + ty < n) {
-                double acc[4][4];
+            // A[i][k] -= sum_q L[i][p0 + q] L[k][p0 + q] for q0 <= k <= i: tile
+            // (ti, tj) of the triangle from q0 on, numbered row by row
+            const int q0 = p0 + pn, nt = (n - q0 + 15) / 16;
+            for (int t = wv; t < nt * (nt + 1) / 2; t += nw) {
+                int ti = 0, tj = t;
+                while (tj > ti) { tj -= ti + 1; ++ti; }
+                const int oi = pn + 16 * ti + j, oj = pn + 16 * tj + j;   // panel-relative rows
+                d4 acc = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-                for (int a = 0; a < 4; ++a)
+                for (int s4 = 0; s4 < kPB; s4 += 4)
+                    acc = mfma64(Pt[s4 + g][oi], Pt[s4 + g][oj], acc);
 #pragma unroll
-                    for (int b = 0; b < 4; ++b) acc[a][b] = 0.0;
-                const int oi = q0 - p0 + ty, ok0 = q0 - p0 + tx;   // panel-relative rows
-                for (int j = 0; j < pn; ++j) {
-                    double li[4], lk[4];
-#pragma unroll
-                    for (int a = 0; a < 4; ++a) {
-                        li[a] = (oi + 32 * a < 128) ? Pt[j][oi + 32 * a] : 0.0;
-                        lk[a] = (ok0 + 32 * a < 128) ? Pt[j][ok0 + 32 * a] : 0.0;
-                    }
-#pragma unroll
-                    for (int a = 0; a < 4; ++a)
-#pragma unroll
-                        for (int b = 0; b < 4; ++b) acc[a][b] = fma(li[a], lk[b], acc[a][b]);
+                for (int r = 0; r < 4; ++r) {
+                    const int i = q0 + 16 * ti + 4 * r + g, k = q0 + 16 * tj + j;
+                    if (i < n && k <= i) As[i * ld + k] -= acc[r];
                 }
-#pragma unroll
-                for (int a = 0; a < 4; ++a)
-#pragma unroll
-                    for (int b = 0; b < 4; ++b) {
-                        const int i = q0 + ty + 32 * a, k = q0 + tx + 32 * b;
-                        if (i < n && k <= i) As[i * n + k] -= acc[a][b];
-                    }
             }
             __syncthreads();
         }
@@ -689,151 +727,125 @@ __device__ __forceinline__ void k_chol_lds_body(
         scal[kScalJitter] = jit;
         scal[kScalSolveOK] = ok ? 1.0 : 0.0;
     }
-    for (int e = tid; e < n * n; e += nt) L[e] = As[e];
+    for (int i = wv; i < n; i += nw)
+        for (int k = lane; k <= i; k += 64) L[(long)i * n + k] = As[i * ld + k];
 }
 
-__global__ __launch_bounds__(1024) void k_chol_lds(const double *__restrict__ A0,
-                                                   double *__restrict__ L, int n, double ridge,
-                                                   double *__restrict__ scal) {
+constexpr int kCholNT = 1024;
+__global__ __launch_bounds__(kCholNT) void k_chol_lds(const double *__restrict__ A0,
+                                                      double *__restrict__ L, int n, double ridge,
+                                                      double *__restrict__ scal) {
     k_chol_lds_body(blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, A0, L, n, ridge, scal);
 }
 
-// W[:, c0:c0+CPW NT/64] from L y = b, L^T x = y (n <= 126), NT threads: L in
-// LDS (rows at an odd stride, so that a column read by a wave spreads over the
-// banks); wave w solves the CPW right-hand sides c0 + CPW w + q on its own, lane
-// l keeping rows l and l + 64 of each, and their 1 / L_pp, in registers.
-// Step i: x_i and 1 / L_ii go from the lane that owns row i to the whole wave
-// by readlane, with no barrier and no LDS access on the way, and every lane
-// updates its rows after (forward) or before (backward) row i with the L
-// elements it read from LDS during the step before.  The arithmetic is that
-// of the plain substitution, x_i = x_i (1 / L_ii), then one FMA per later
-// (earlier) row, in the same order for every row.
-template <int NT, int CPW>
+// W[:, c0 : c0 + 16] from L y = b, L^T x = y (n <= 126), one workgroup of four
+// waves: L's lower triangle in LDS, the right-hand sides in 16-row blocks, block
+// t in the accumulator of wave t % 4.  For each block in turn its wave solves the
+// 16 x 16 triangle in the accumulator's layout, and the waves then apply the
+// block's x to their other blocks on matrix instructions.  Each row receives its
+// updates in the order of the plain substitution: x_i = x_i (1 / L_ii), then one
+// FMA per later row in ascending i (forward), or per earlier row in descending i
+// (backward, the MFMA's inner index running down).
+// Bound by the chain of blocks (8 each way at n = 126): 48 -> 35 us, n = 26:
+// 15 -> 9 (a wave per right-hand side, one row at a time: a step of the chain
+// for each of n rows).
 __device__ __forceinline__ void k_trsm_lds_body(
     const int bx, const int by, const int bz, const int gx, const double *__restrict__ L, int n,
     const double *__restrict__ B, int nrhs, double *__restrict__ W,
     const double *__restrict__ scal) {
     if (scal[kScalSolveOK] != 1.0) return;
-    constexpr int LDL = kLdsN | 1;
-    __shared__ double Ls[kLdsN * LDL];
-    const int tid = threadIdx.x, nt = NT;
-    const int l = tid & 63, w = tid >> 6;
-    const int ld = n | 1;                          // row stride in LDS, at most LDL
-    // the lower triangle: all of a thread's loads are in flight before its
-    // first LDS store
-    constexpr int FILL = (kLdsN * kLdsN + NT - 1) / NT;
-    {
-        double v[FILL];
+    __shared__ double Ls[128 * (kLdsN | 1) + 16];
+    __shared__ double rd[128];                     // 1 / L_pp
+    __shared__ double xs[16][17];                  // the block just solved
+    const int tid = threadIdx.x, l = tid & 63, w = tid >> 6, j = l & 15, g = l >> 4;
+    const int ld = n | 1, nblk = (n + 15) / 16;
+    load_lower(L, n, [&](int i, int k, double v) { Ls[i * ld + k] = v; });
+    // rows past the end: zero entries of L, and zero right-hand sides
+    for (int e = n * ld + tid; e < 16 * nblk * ld + 16; e += 256) Ls[e] = 0.0;
+    const int col = 16 * bx + j;
+    const bool live = col < nrhs;
+    auto at = [&](int i, int k) { return Ls[i * ld + k]; };   // k <= i
+    d4 x[2];                                       // blocks w and w + 4
 #pragma unroll
-        for (int f = 0; f < FILL; ++f) {
-            const int e = tid + f * nt, i = e / n, k = e - i * n;
-            v[f] = (e < n * n && k <= i) ? L[e] : 0.0;
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int p = 16 * (w + 4 * q) + 4 * r + g;
+            x[q][r] = (live && p < n) ? B[(long)p * nrhs + col] : 0.0;
         }
-#pragma unroll
-        for (int f = 0; f < FILL; ++f) {
-            const int e = tid + f * nt, i = e / n, k = e - i * n;
-            if (e < n * n && k <= i) Ls[i * ld + k] = v[f];
-        }
-    }
-    const int c0 = bx * (CPW * NT / 64);
-    double x[CPW][2], rdv[2];
-    bool live[CPW];
-#pragma unroll
-    for (int a = 0; a < 2; ++a) {
-        const int p = l + 64 * a;
-        rdv[a] = (p < n) ? 1.0 / L[(long)p * n + p] : 0.0;
-    }
-#pragma unroll
-    for (int q = 0; q < CPW; ++q) {
-        const int col = c0 + CPW * w + q;
-        live[q] = col < nrhs;
-#pragma unroll
-        for (int a = 0; a < 2; ++a) {
-            const int p = l + 64 * a;
-            x[q][a] = (live[q] && p < n) ? B[(long)p * nrhs + col] : 0.0;
-        }
-    }
     __syncthreads();
-    // lane `src`'s v on every lane (src is the same for the whole wave)
-    auto bcast = [](double v, int src) {
-        const long long b = __builtin_bit_cast(long long, v);
-        const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, src);
-        const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), src);
-        return __builtin_bit_cast(double, (long long)(((unsigned long long)hi << 32) | lo));
-    };
-    // x_i from its owner, finished
-    auto pivot = [&](int i, double (&xi)[CPW]) {
-        const int ai = i >> 6, li = i & 63;
-        const double r = bcast(ai ? rdv[1] : rdv[0], li);
+    if (tid < 128) rd[tid] = (tid < n) ? 1.0 / Ls[tid * ld + tid] : 0.0;
+    __syncthreads();
+    // block t's triangle, in the accumulator's layout: row i = 4 R + G goes from
+    // its lanes to the others of its column, which update their later (earlier)
+    // rows; xs gets the solved rows
+    auto diag = [&](int t, d4 &c, auto fwd) {
+        const int b0 = 16 * t;
+        auto step = [&](auto I) {
+            constexpr int i = decltype(fwd)::value ? decltype(I)::value : 15 - decltype(I)::value;
+            constexpr int R = i >> 2, Gi = i & 3;
+            const double xi = row_bcast<Gi>(c[R]) * rd[b0 + i];
 #pragma unroll
-        for (int q = 0; q < CPW; ++q) xi[q] = bcast(ai ? x[q][1] : x[q][0], li) * r;
-    };
-    // the L elements of the next step (rows p < n only: the others lie
-    // outside the LDS rows written)
-    double lpn[2] = {0.0, 0.0};
-    auto next_l = [&](int off, int pstride) {
-#pragma unroll
-        for (int a = 0; a < 2; ++a) {
-            const int p = l + 64 * a;
-            if (p < n) lpn[a] = Ls[p * pstride + off];
-        }
-    };
-    next_l(0, ld);                                 // column 0
-    for (int i = 0; i < n; ++i) {                  // forward
-        const double lp[2] = {lpn[0], lpn[1]};
-        if (i + 1 < n) next_l(i + 1, ld);          // column i + 1
-        double xi[CPW];
-        pivot(i, xi);
-#pragma unroll
-        for (int a = 0; a < 2; ++a) {
-            const int p = l + 64 * a;
-            if (p == i) {
-#pragma unroll
-                for (int q = 0; q < CPW; ++q) x[q][a] = xi[q];
-            } else if (p > i && p < n) {
-#pragma unroll
-                for (int q = 0; q < CPW; ++q) x[q][a] = fma(-lp[a], xi[q], x[q][a]);
+            for (int r = 0; r < 4; ++r) {
+                if (decltype(fwd)::value ? r < R : r > R) continue;
+                const int p = 4 * r + g;
+                const bool upd = decltype(fwd)::value ? p > i : p < i;
+                const double lp = decltype(fwd)::value ? at(b0 + (upd ? p : i), b0 + i)
+                                                       : at(b0 + i, b0 + (upd ? p : i));
+                const double v = fma(-lp, xi, c[r]);
+                c[r] = (p == i) ? xi : upd ? v : c[r];
             }
+        };
+        each_of(std::make_integer_sequence<int, 16>{}, step);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) xs[4 * r + g][j] = c[r];
+    };
+    for (int t = 0; t < nblk; ++t) {               // forward
+        if (w == (t & 3)) {
+            if (t < 4) diag(t, x[0], std::true_type{});
+            else diag(t, x[1], std::true_type{});
         }
-    }
-    next_l((n - 1) * ld, 1);                       // row n - 1
-    for (int i = n - 1; i >= 0; --i) {             // backward with L^T
-        const double lp[2] = {lpn[0], lpn[1]};
-        if (i > 0) next_l((i - 1) * ld, 1);        // row i - 1
-        double xi[CPW];
-        pivot(i, xi);
+        __syncthreads();
 #pragma unroll
-        for (int a = 0; a < 2; ++a) {
-            const int p = l + 64 * a;
-            if (p == i) {
+        for (int q = 0; q < 2; ++q) {
+            const int u = w + 4 * q;
+            if (u > t && u < nblk)
 #pragma unroll
-                for (int q = 0; q < CPW; ++q) x[q][a] = xi[q];
-            } else if (p < i) {
-#pragma unroll
-                for (int q = 0; q < CPW; ++q) x[q][a] = fma(-lp[a], xi[q], x[q][a]);
-            }
+                for (int s4 = 0; s4 < 16; s4 += 4)
+                    x[q] = mfma64(-at(16 * u + j, 16 * t + s4 + g), xs[s4 + g][j], x[q]);
         }
+        __syncthreads();                           // xs is rewritten by the next block
     }
-#pragma unroll
-    for (int q = 0; q < CPW; ++q) {
-        const int col = c0 + CPW * w + q;
-#pragma unroll
-        for (int a = 0; a < 2; ++a) {
-            const int p = l + 64 * a;
-            if (live[q] && p < n) W[(long)p * nrhs + col] = x[q][a];
+    for (int t = nblk - 1; t >= 0; --t) {          // backward with L^T, i descending
+        if (w == (t & 3)) {
+            if (t < 4) diag(t, x[0], std::false_type{});
+            else diag(t, x[1], std::false_type{});
         }
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int u = w + 4 * q;
+            if (u < t)
+#pragma unroll
+                for (int s4 = 15; s4 > 0; s4 -= 4)
+                    x[q] = mfma64(-at(16 * t + s4 - g, 16 * u + j), xs[s4 - g][j], x[q]);
+        }
+        __syncthreads();
     }
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int p = 16 * (w + 4 * q) + 4 * r + g;
+            if (live && p < n) W[(long)p * nrhs + col] = x[q][r];
+        }
 }
 
-// one wave per SIMD and one right-hand side per wave: the substitution is
-// issue-bound, so the right-hand sides go 4 to a workgroup over more CUs
-constexpr int kTrsmNT = 256, kTrsmCPW = 1;
-__global__ __launch_bounds__(kTrsmNT) void k_trsm_lds(const double *__restrict__ L, int n,
-                                                      const double *__restrict__ B, int nrhs,
-                                                      double *__restrict__ W,
-                                                      const double *__restrict__ scal) {
-    k_trsm_lds_body<kTrsmNT, kTrsmCPW>(blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, L, n, B,
-                                       nrhs, W, scal);
+__global__ __launch_bounds__(256) void k_trsm_lds(const double *__restrict__ L, int n,
+                                                  const double *__restrict__ B, int nrhs,
+                                                  double *__restrict__ W,
+                                                  const double *__restrict__ scal) {
+    k_trsm_lds_body(blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, L, n, B, nrhs, W, scal);
 }
 
 // The new centres and what the M-step takes from them, sixteen centres to a
@@ -1061,19 +1073,19 @@ __global__ __launch_bounds__(256) void kb_sumAB(const BInst *__restrict__ tab, c
     k_sumAB_body(m.y, 0, 0, 0, I.partAB, I.nchAB, I.M1, I.D, I.A0, I.Bm, I.K, I.G, I.Gm);
 }
 
-__global__ __launch_bounds__(1024) void kb_chol_lds(const BInst *__restrict__ tab,
+__global__ __launch_bounds__(kCholNT) void kb_chol_lds(const BInst *__restrict__ tab,
                                                     const int *__restrict__ list) {
     const BInst &I = tab[list[blockIdx.x]];
     if (!I.do_m) return;
     k_chol_lds_body(0, 0, 0, 1, I.A0, I.A, I.M1, I.ridge, I.scal);
 }
 
-__global__ __launch_bounds__(1024) void kb_trsm_lds(const BInst *__restrict__ tab,
+__global__ __launch_bounds__(256) void kb_trsm_lds(const BInst *__restrict__ tab,
                                                     const int2 *__restrict__ map) {
     const int2 m = map[blockIdx.x];
     const BInst &I = tab[m.x];
     if (!I.do_m) return;
-    k_trsm_lds_body<1024, 2>(m.y, 0, 0, 0, I.A, I.M1, I.Bm, I.D, I.W, I.scal);
+    k_trsm_lds_body(m.y, 0, 0, 0, I.A, I.M1, I.Bm, I.D, I.W, I.scal);
 }
 
 __global__ __launch_bounds__(1024) void kb_chol_solve(const BInst *__restrict__ tab,
@@ -1207,13 +1219,11 @@ int dg_mstep_run(dg_ctx *c, double jitter) {
     DG_HIP(c, hipGetLastError());
     const double ridge = (c->cfg.lambda > 0.0) ? c->cfg.lambda / c->beta : 0.0;
     if (M1 <= kLdsN) {
-        hipLaunchKernelGGL(k_chol_lds, dim3(1), dim3(1024), 0, c->stream, c->A0, c->A, M1, ridge,
+        hipLaunchKernelGGL(k_chol_lds, dim3(1), dim3(kCholNT), 0, c->stream, c->A0, c->A, M1, ridge,
                            c->scal);
         DG_HIP(c, hipGetLastError());
-        constexpr int cols = kTrsmCPW * kTrsmNT / 64;     // right-hand sides per workgroup
-        hipLaunchKernelGGL(k_trsm_lds, dim3((unsigned)((D + cols - 1) / cols)),
-                           dim3(kTrsmNT), 0, c->stream,
-                           c->A, M1, c->Bm, D, c->W, c->scal);
+        hipLaunchKernelGGL(k_trsm_lds, dim3((unsigned)bk_cdiv(D, 16)), dim3(256), 0, c->stream, c->A,
+                           M1, c->Bm, D, c->W, c->scal);
     } else {
         int rc = blocked_chol_solve(c, ridge, jitter);
         if (rc) return rc;
@@ -1244,8 +1254,8 @@ int dg_batch_mstep(hipStream_t st, const BInst *tab, const int *list, int n, int
     flat(kb_partAB, BK_PART_AB, 256);
     flat(kb_sumAB, BK_SUM_AB, 256);
     if (nlds > 0) {
-        hipLaunchKernelGGL(kb_chol_lds, dim3((unsigned)nlds), dim3(1024), 0, st, tab, list);
-        flat(kb_trsm_lds, BK_TRSM_LDS, 1024);
+        hipLaunchKernelGGL(kb_chol_lds, dim3((unsigned)nlds), dim3(kCholNT), 0, st, tab, list);
+        flat(kb_trsm_lds, BK_TRSM_LDS, 256);
     }
     if (n > nlds)
         hipLaunchKernelGGL(kb_chol_solve, dim3((unsigned)(n - nlds)), dim3(1024), 0, st, tab,
