@@ -151,242 +151,6 @@ __device__ __forceinline__ void k_chol_solve_body(
     }
 }
 
-// ---- blocked Cholesky and solves for M + 1 > 126 ---------------------------
-// (A0 + (ridge + jitter) I) W = B factored and solved by 64 x 64 blocks over
-// many workgroups, one launch per step: for each diagonal block k the block
-// is factored in LDS (k_bc_potrf), the panel below it solved against it
-// (k_bc_trsm) and the trailing lower triangle updated (k_bc_syrk); then the
-// forward and backward substitutions run block by block, a triangular solve
-// of the block's rows (k_bc_fwd / k_bc_bwd) and a product that moves its
-// contribution into the remaining rows (k_bc_fwd_update / k_bc_bwd_update).
-// A non-positive pivot clears scal[kScalSolveOK]; every later kernel of the
-// sequence then returns at once, and the host retries with a jitter.
-constexpr int BC = 64;
-
-__global__ __launch_bounds__(256) void k_bc_init(const double *__restrict__ A0,
-                                                 double *__restrict__ A, int n, double ridge,
-                                                 double jit, const double *__restrict__ B,
-                                                 double *__restrict__ X, int nrhs,
-                                                 double *__restrict__ scal) {
-    const long e = (long)blockIdx.x * 256 + threadIdx.x;
-    const long nn = (long)n * n;
-    if (e < nn) A[e] = A0[e] + ((e / n == e % n) ? ridge + jit : 0.0);
-    else if (e < nn + (long)n * nrhs) X[e - nn] = B[e - nn];
-    if (e == 0) {
-        scal[kScalSolveOK] = 1.0;
-        scal[kScalJitter] = jit;
-    }
-}
-
-// factor the kb x kb diagonal block at k0 in LDS (right-looking, column by column)
-__global__ __launch_bounds__(256) void k_bc_potrf(double *__restrict__ A, int n, int k0,
-                                                  double *__restrict__ scal) {
-    __shared__ double L[BC][BC + 1];
-    __shared__ int bad;
-    if (scal[kScalSolveOK] != 1.0) return;
-    const int tid = threadIdx.x;
-    const int kb = min(BC, n - k0);
-    for (int e = tid; e < kb * kb; e += 256) L[e / kb][e % kb] = A[(long)(k0 + e / kb) * n + k0 + e % kb];
-    if (tid == 0) bad = 0;
-    __syncthreads();
-    for (int j = 0; j < kb; ++j) {
-        if (tid == 0) {
-            const double p = L[j][j];
-            if (!(p > 0.0)) bad = 1;
-            else L[j][j] = sqrt(p);
-        }
-        __syncthreads();
-        if (bad) break;
-        const double ljj = L[j][j];
-        for (int i = j + 1 + tid; i < kb; i += 256) L[i][j] /= ljj;
-        __syncthreads();
-        const int m = kb - j - 1;
-        for (int e = tid; e < m * m; e += 256) {
-            const int r = j + 1 + e / m, c = j + 1 + e % m;
-            if (c <= r) L[r][c] = fma(-L[r][j], L[c][j], L[r][c]);
-        }
-        __syncthreads();
-    }
-    if (bad) {
-        if (tid == 0) scal[kScalSolveOK] = 0.0;
-        return;
-    }
-    for (int e = tid; e < kb * kb; e += 256) {
-        const int r = e / kb, c = e % kb;
-        if (c <= r) A[(long)(k0 + r) * n + k0 + c] = L[r][c];
-    }
-}
-
-// rows i >= k0 + kb of the panel: L21 = A21 L11^-T, one row per thread
-__global__ __launch_bounds__(256) void k_bc_trsm(double *__restrict__ A, int n, int k0,
-                                                 const double *__restrict__ scal) {
-    __shared__ double L[BC][BC + 1];
-    if (scal[kScalSolveOK] != 1.0) return;
-    const int tid = threadIdx.x;
-    const int kb = min(BC, n - k0), k1 = k0 + kb;
-    for (int e = tid; e < kb * kb; e += 256) L[e / kb][e % kb] = A[(long)(k0 + e / kb) * n + k0 + e % kb];
-    __syncthreads();
-    const long i = (long)k1 + (long)blockIdx.x * 256 + tid;
-    if (i >= n) return;
-    double x[BC];
-#pragma unroll
-    for (int j = 0; j < BC; ++j) x[j] = (j < kb) ? A[i * n + k0 + j] : 0.0;
-#pragma unroll
-    for (int j = 0; j < BC; ++j) {
-        if (j < kb) {
-            double s = x[j];
-#pragma unroll
-            for (int p = 0; p < j; ++p) s = fma(-x[p], L[j][p], s);
-            x[j] = s / L[j][j];
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < BC; ++j)
-        if (j < kb) A[i * n + k0 + j] = x[j];
-}
-
-// trailing update of the lower triangle: A[i][j] -= sum_p L[i][p] L[j][p]
-// over the panel columns p, for k1 <= j <= i < n; 64 x 64 tiles (ti >= tj)
-__global__ __launch_bounds__(256) void k_bc_syrk(double *__restrict__ A, int n, int k0,
-                                                 const double *__restrict__ scal) {
-    __shared__ double Li[BC][BC + 1], Lj[BC][BC + 1];
-    if (blockIdx.y > blockIdx.x || scal[kScalSolveOK] != 1.0) return;
-    const int kb = min(BC, n - k0), k1 = k0 + kb;
-    const int i0 = k1 + blockIdx.x * BC, j0 = k1 + blockIdx.y * BC;
-    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-    for (int e = tid; e < BC * BC; e += 256) {
-        const int r = e / BC, p = e % BC;
-        Li[r][p] = (i0 + r < n && p < kb) ? A[(long)(i0 + r) * n + k0 + p] : 0.0;
-        Lj[r][p] = (j0 + r < n && p < kb) ? A[(long)(j0 + r) * n + k0 + p] : 0.0;
-    }
-    __syncthreads();
-    double acc[4][4];
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = 0.0;
-    for (int p = 0; p < kb; ++p) {
-        double av[4], bv[4];
-#pragma unroll
-        for (int a = 0; a < 4; ++a) av[a] = Li[ty + 16 * a][p];
-#pragma unroll
-        for (int b = 0; b < 4; ++b) bv[b] = Lj[tx + 16 * b][p];
-#pragma unroll
-        for (int a = 0; a < 4; ++a)
-#pragma unroll
-            for (int b = 0; b < 4; ++b) acc[a][b] = fma(av[a], bv[b], acc[a][b]);
-    }
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            const int i = i0 + ty + 16 * a, j = j0 + tx + 16 * b;
-            if (i < n && j <= i) A[(long)i * n + j] -= acc[a][b];
-        }
-}
-
-// forward substitution of block k: X[k0..k1) = L_kk^-1 X[k0..k1), one
-// right-hand side per thread
-__global__ __launch_bounds__(256) void k_bc_fwd(const double *__restrict__ A, int n, int k0,
-                                                double *__restrict__ X, int nrhs,
-                                                const double *__restrict__ scal) {
-    __shared__ double L[BC][BC + 1];
-    if (scal[kScalSolveOK] != 1.0) return;
-    const int tid = threadIdx.x;
-    const int kb = min(BC, n - k0);
-    for (int e = tid; e < kb * kb; e += 256) L[e / kb][e % kb] = A[(long)(k0 + e / kb) * n + k0 + e % kb];
-    __syncthreads();
-    const int c = blockIdx.x * 256 + tid;
-    if (c >= nrhs) return;
-    double x[BC];
-#pragma unroll
-    for (int j = 0; j < BC; ++j) {
-        if (j < kb) {
-            double s = X[(long)(k0 + j) * nrhs + c];
-#pragma unroll
-            for (int p = 0; p < j; ++p) s = fma(-L[j][p], x[p], s);
-            x[j] = s / L[j][j];
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < BC; ++j)
-        if (j < kb) X[(long)(k0 + j) * nrhs + c] = x[j];
-}
-
-// backward substitution of block k: X[k0..k1) = L_kk^-T X[k0..k1)
-__global__ __launch_bounds__(256) void k_bc_bwd(const double *__restrict__ A, int n, int k0,
-                                                double *__restrict__ X, int nrhs,
-                                                const double *__restrict__ scal) {
-    __shared__ double L[BC][BC + 1];
-    if (scal[kScalSolveOK] != 1.0) return;
-    const int tid = threadIdx.x;
-    const int kb = min(BC, n - k0);
-    for (int e = tid; e < kb * kb; e += 256) L[e / kb][e % kb] = A[(long)(k0 + e / kb) * n + k0 + e % kb];
-    __syncthreads();
-    const int c = blockIdx.x * 256 + tid;
-    if (c >= nrhs) return;
-    double x[BC];
-#pragma unroll
-    for (int jj = BC - 1; jj >= 0; --jj) {
-        if (jj < kb) {
-            double s = X[(long)(k0 + jj) * nrhs + c];
-#pragma unroll
-            for (int p = jj + 1; p < BC; ++p)
-                if (p < kb) s = fma(-L[p][jj], x[p], s);
-            x[jj] = s / L[jj][jj];
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < BC; ++j)
-        if (j < kb) X[(long)(k0 + j) * nrhs + c] = x[j];
-}
-
-// X[i] -= sum_p L[i][k0 + p] X[k0 + p] for the rows i >= k1 (forward) or
-// X[i] -= sum_p L[k0 + p][i] X[k0 + p] for the rows i < k0 (backward), in
-// 64 x 64 tiles of (rows, right-hand sides)
-template <bool FWD>
-__global__ __launch_bounds__(256) void k_bc_update(const double *__restrict__ A, int n, int k0,
-                                                   double *__restrict__ X, int nrhs,
-                                                   const double *__restrict__ scal) {
-    __shared__ double Lt[BC][BC + 1], Xs[BC][BC + 1];
-    if (scal[kScalSolveOK] != 1.0) return;
-    const int kb = min(BC, n - k0), k1 = k0 + kb;
-    const int r0 = (FWD ? k1 : 0) + blockIdx.x * BC, c0 = blockIdx.y * BC;
-    const int rend = FWD ? n : k0;
-    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-    for (int e = tid; e < BC * BC; e += 256) {
-        const int r = e / BC, p = e % BC;
-        const int i = r0 + r;
-        Lt[r][p] = (i < rend && p < kb)
-                       ? (FWD ? A[(long)i * n + k0 + p] : A[(long)(k0 + p) * n + i]) : 0.0;
-        Xs[r][p] = (r < kb && c0 + p < nrhs) ? X[(long)(k0 + r) * nrhs + c0 + p] : 0.0;
-    }
-    __syncthreads();
-    double acc[4][4];
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = 0.0;
-    for (int p = 0; p < kb; ++p) {
-        double av[4], bv[4];
-#pragma unroll
-        for (int a = 0; a < 4; ++a) av[a] = Lt[ty + 16 * a][p];
-#pragma unroll
-        for (int b = 0; b < 4; ++b) bv[b] = Xs[p][tx + 16 * b];
-#pragma unroll
-        for (int a = 0; a < 4; ++a)
-#pragma unroll
-            for (int b = 0; b < 4; ++b) acc[a][b] = fma(av[a], bv[b], acc[a][b]);
-    }
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            const int i = r0 + ty + 16 * a, c = c0 + tx + 16 * b;
-            if (i < rend && c < nrhs) X[(long)i * nrhs + c] -= acc[a][b];
-        }
-}
-
 // tr(A0) into scal[kScalJitter] (the retries' jitter scale)
 __global__ __launch_bounds__(64) void k_bc_trace(const double *__restrict__ A0, int n,
                                                  double *__restrict__ scal) {
@@ -618,6 +382,363 @@ __device__ __forceinline__ double row_bcast(double x) {
         h[i] = (G & 2) ? (unsigned)b[1] : (unsigned)b[0];
     }
     return __builtin_bit_cast(double, ((unsigned long long)h[1] << 32) | h[0]);
+}
+
+// ---- blocked Cholesky and solves for M + 1 > 126 ---------------------------
+// (A0 + (ridge + jitter) I) W = B by 64 x 64 blocks over many workgroups.  The
+// right-hand sides, transposed, are further rows below A: their blocks of the
+// factor are the forward substitution, with the same chain for every element.
+// S is that (n + nrhs) x n matrix, row-major, factored in place; Ld takes the
+// diagonal blocks' factors, transposed and filled up with the identity, 64 x 64
+// each.  One launch per block column (k_bc_step), one for the whole backward
+// substitution (k_bc_back).  A non-positive pivot clears scal[kScalSolveOK]; every
+// later kernel of the sequence then returns at once, and the host retries with a
+// jitter.
+constexpr int BC = 64;
+constexpr int kBcLd = BC + 2;    // LDS row stride: 16 rows x 2 inner indexes hit 32 banks
+
+__global__ __launch_bounds__(256) void k_bc_init(const double *__restrict__ A0,
+                                                 double *__restrict__ S, int n, double ridge,
+                                                 double jit, const double *__restrict__ B,
+                                                 int nrhs, double *__restrict__ scal) {
+    const long e = (long)blockIdx.x * 256 + threadIdx.x;
+    const long nn = (long)n * n;
+    if (e < nn) {
+        S[e] = A0[e] + ((e / n == e % n) ? ridge + jit : 0.0);
+    } else if (e < nn + (long)n * nrhs) {
+        const long c = (e - nn) / n, p = (e - nn) % n;
+        S[e] = B[p * nrhs + c];
+    }
+    if (e == 0) {
+        scal[kScalSolveOK] = 1.0;
+        scal[kScalJitter] = jit;
+    }
+}
+
+// Block column kc of the factorisation, with block column kc - 1's products:
+// workgroup (x, 0) takes 64 rows below the diagonal block through all of it,
+//   P = S[rows][kc] - L[rows][kc - 1] L[kc][kc - 1]^T,  P <- P L_kk^-T,
+// and finds L_kk for itself, from the diagonal block less its own product
+// (the same in every workgroup, none waits for another; workgroup 0 leaves it in
+// Ld); workgroup (x, 1 + y) subtracts the product from one 64 x 64 tile of the
+// columns after kc.  So a step is one launch, and the tiles run beside the panel.
+//   Wave 0 factors 16 columns at a time in registers (a row to a lane, the pivot
+// row broadcast with readlane), waves 1 .. 4 meanwhile solve their 16 rows of the
+// panel against the 16 columns before, and all five apply the 16 columns to the
+// rest of the diagonal block on matrix instructions.  The panel is held as
+// [column][row], so that a solved 16 x 16 block in an accumulator is, as it lies,
+// the operand of the products that follow.
+// Bound by the chain of 64 square roots and divisions per step.  n = 1001, 166
+// right-hand sides: 32 us a step; three launches for the factorisation and two
+// for the forward substitution per block, each a third-full chain of its own,
+// 86 + 46 + 20 and 32 + 20 us.
+constexpr int kBcNT = 320;
+__global__ __launch_bounds__(kBcNT) void k_bc_step(double *__restrict__ S, int n, int nrows, int kc,
+                                                   double *__restrict__ Ld,
+                                                   double *__restrict__ scal) {
+    __shared__ double Pk[BC][kBcLd];               // L[kc][kc - 1], or a tile's columns
+    __shared__ double Dg[BC][kBcLd];               // the diagonal block
+    __shared__ int bad;
+    if (scal[kScalSolveOK] != 1.0) return;
+    const int tid = threadIdx.x, l = tid & 63, j = l & 15, g = l >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int k0 = kc * BC, kb = min(BC, n - k0), k1 = k0 + kb, kp = k0 - BC;
+    const int i0 = k1 + blockIdx.x * BC;           // the first of this workgroup's rows
+    const bool panel = blockIdx.y == 0;
+    const int c0 = panel ? k0 : k1 + ((int)blockIdx.y - 1) * BC;
+    if (!panel && c0 > i0 + BC - 1) return;        // above the diagonal
+    const int cn = min(BC, n - c0);                // columns of this workgroup's tile
+    if (kc > 0)
+        for (int e = tid; e < BC * BC; e += kBcNT) {
+            const int r = e >> 6, p = e & 63;
+            Pk[r][p] = (r < cn) ? S[(long)(c0 + r) * n + kp + p] : 0.0;
+        }
+    const int wr = panel ? w - 1 : w;              // which 16 of the rows, if 0 .. 3
+    const bool rows = wr >= 0 && wr < 4;
+    const int ir = min(i0 + 16 * max(wr, 0) + j, nrows - 1);   // this lane's row (past the end: the last)
+    double pa[16];                                 // L[ir][kp + 4 s + g]
+#pragma unroll
+    for (int s = 0; s < 16; ++s) pa[s] = (kc > 0 && rows) ? S[(long)ir * n + kp + 4 * s + g] : 0.0;
+    if (!panel) {
+        __syncthreads();
+        if (!rows) return;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            d4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int s = 0; s < 16; ++s) acc = mfma64(pa[s], Pk[16 * t + j][4 * s + g], acc);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int i = i0 + 16 * wr + 4 * r + g, c = c0 + 16 * t + j;
+                if (i < nrows && c < n && c <= i) S[(long)i * n + c] -= acc[r];
+            }
+        }
+        return;
+    }
+    d4 x[4];                                       // P, [column 16 t + 4 r + g][row j]
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int p = 16 * t + 4 * r + g;
+            x[t][r] = (rows && p < kb) ? S[(long)ir * n + k0 + p] : 0.0;
+        }
+    for (int e = tid; e < BC * BC; e += kBcNT) {
+        const int r = e >> 6, c = e & 63;
+        Dg[r][c] = (r < kb && c <= r) ? S[(long)(k0 + r) * n + k0 + c] : (r == c) ? 1.0 : 0.0;
+    }
+    if (tid == 0) bad = 0;
+    __syncthreads();
+    if (kc > 0) {
+        for (int t = w; t < 10; t += 5) {          // the diagonal block's lower tiles
+            const int ti = (t < 1) ? 0 : (t < 3) ? 1 : (t < 6) ? 2 : 3, tj = t - ti * (ti + 1) / 2;
+            d4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int s = 0; s < 16; ++s)
+                acc = mfma64(Pk[16 * ti + j][4 * s + g], Pk[16 * tj + j][4 * s + g], acc);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int i = 16 * ti + 4 * r + g, c = 16 * tj + j;
+                if (c <= i) Dg[i][c] -= acc[r];    // (0 past the end: Pk's rows are)
+            }
+        }
+        if (rows)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                d4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                for (int s = 0; s < 16; ++s) acc = mfma64(Pk[16 * t + j][4 * s + g], pa[s], acc);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) x[t][r] -= acc[r];
+            }
+        __syncthreads();
+    }
+    // columns 16 t .. of the panel, once those of L_kk are there
+    auto solve = [&](auto T) {
+        constexpr int t = decltype(T)::value;
+        each_of(std::make_integer_sequence<int, t>{}, [&](auto U) {
+            constexpr int u = decltype(U)::value;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                x[t] = mfma64(-Dg[16 * t + j][16 * u + 4 * r + g], x[u][r], x[t]);
+        });
+        each_of(std::make_integer_sequence<int, 16>{}, [&](auto I) {
+            constexpr int i = decltype(I)::value, R = i >> 2, Gi = i & 3;
+            const double xi = row_bcast<Gi>(x[t][R]) / Dg[16 * t + i][16 * t + i];
+#pragma unroll
+            for (int r = R; r < 4; ++r) {
+                const int p = 4 * r + g;
+                const double v = fma(-xi, Dg[16 * t + max(p, i)][16 * t + i], x[t][r]);
+                x[t][r] = (p == i) ? xi : (p > i) ? v : x[t][r];
+            }
+        });
+    };
+    each_of(std::make_integer_sequence<int, 4>{}, [&](auto T) {
+        constexpr int t = decltype(T)::value;
+        if (w == 0) {
+            double a[16];
+#pragma unroll
+            for (int c = 0; c < 16; ++c) a[c] = Dg[l][16 * t + c];
+            bool failed = false;
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                const double piv = lane_bcast(a[q], 16 * t + q);
+                failed = failed || !(piv > 0.0);
+                const double sq = sqrt(piv);
+                a[q] = (l == 16 * t + q) ? sq : a[q] / sq;
+#pragma unroll
+                for (int c = q + 1; c < 16; ++c)
+                    a[c] = fma(-a[q], lane_bcast(a[q], 16 * t + c), a[c]);
+            }
+#pragma unroll
+            for (int c = 0; c < 16; ++c)
+                if (l >= 16 * t + c) Dg[l][16 * t + c] = a[c];
+            if (failed && l == 0) bad = 1;
+        } else if constexpr (t > 0) {
+            solve(std::integral_constant<int, t - 1>{});
+        }
+        __syncthreads();
+        if constexpr (t < 3) {
+            constexpr int nt = 3 - t;              // 16 x 16 tiles a side after this column
+            for (int q = w; q < nt * (nt + 1) / 2; q += 5) {
+                const int a = (q < 1) ? 0 : (q < 3) ? 1 : 2;
+                const int ti = t + 1 + a, tj = t + 1 + q - a * (a + 1) / 2;
+                d4 c;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) c[r] = Dg[16 * ti + 4 * r + g][16 * tj + j];
+#pragma unroll
+                for (int s = 0; s < 16; s += 4)
+                    c = mfma64(-Dg[16 * ti + j][16 * t + s + g], Dg[16 * tj + j][16 * t + s + g], c);
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (16 * tj + j <= 16 * ti + 4 * r + g) Dg[16 * ti + 4 * r + g][16 * tj + j] = c[r];
+            }
+            __syncthreads();
+        }
+    });
+    if (bad) {                                     // the same in every workgroup
+        if (tid == 0 && blockIdx.x == 0) scal[kScalSolveOK] = 0.0;
+        return;
+    }
+    if (blockIdx.x == 0)
+        for (int e = tid; e < BC * BC; e += kBcNT) {
+            const int c = e >> 6, r = e & 63;
+            Ld[(long)kc * BC * BC + e] = (c <= r) ? Dg[r][c] : 0.0;
+        }
+    if (w == 0) return;
+    solve(std::integral_constant<int, 3>{});
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int p = 16 * t + 4 * r + g;
+            if (p < kb && i0 + 16 * wr + j < nrows) S[(long)ir * n + k0 + p] = x[t][r];
+        }
+}
+
+// L^T W = Y for sixteen right-hand sides, Y^T in the rows of S after the n-th:
+// block by block from the last.  Wave 0 solves a block, a right-hand side to a
+// lane, while waves 1 .. 4 subtract the products of the blocks solved before it
+// from the next (16 of its rows each); the solved block's own product follows.
+// Row i of a block takes x[i + 1], x[i + 2], .. in that order, so its chain can
+// only begin when x[i + 1] is known: 2016 dependent FMAs and 64 divisions a block
+// bound the kernel.  n = 1001, 166 right-hand sides: 289 us (two launches per
+// block, 50 + 20 us each).
+__global__ __launch_bounds__(kBcNT) void k_bc_back(const double *__restrict__ S, int n, int nrhs,
+                                                   const double *__restrict__ Ld,
+                                                   double *__restrict__ W,
+                                                   const double *__restrict__ scal) {
+    __shared__ __align__(16) double Lt[2][BC][kBcLd];   // L_kk transposed: Lt[i][p] = L[p][i]
+    __shared__ double Ln[BC][kBcLd];                    // L[k][k - 1]
+    __shared__ double Sx[BC][16], Xs[BC][16];           // the block's right side, its solution
+    __shared__ double Sn[BC][16];                       // the next one's, but for the block's product
+    if (scal[kScalSolveOK] != 1.0) return;
+    const int tid = threadIdx.x, l = tid & 63, j = l & 15, g = l >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nb = (n + BC - 1) / BC;
+    const int col = min(16 * (int)blockIdx.x + j, nrhs - 1);   // past the end: the last again
+    const bool live = 16 * (int)blockIdx.x + j < nrhs;
+    const double *Yc = S + (long)(n + col) * n;
+    const int ro = 16 * (w - 1);                   // waves 1 .. 4: their rows of a block
+    auto stage = [&](int k) {                      // Ld of block k, by the threads of waves 1 .. 4
+        for (int e = tid - 64; e < BC * BC; e += 256)
+            Lt[k & 1][e >> 6][e & 63] = Ld[(long)k * BC * BC + e];
+    };
+    if (w > 0) {
+        stage(nb - 1);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int i = ro + 4 * r + g, p = (nb - 1) * BC + i;
+            Sx[i][j] = (p < n) ? Yc[p] : 0.0;
+        }
+    }
+    __syncthreads();
+    for (int k = nb - 1; k >= 0; --k) {
+        const int k0 = k * BC, kb = min(BC, n - k0);
+        if (w == 0) {
+            // L's entries of a row are read sixteen at a time, one run ahead
+            const double(*T)[kBcLd] = Lt[k & 1];
+            double x[BC], cur[16], s = Sx[BC - 1][j], dg = T[BC - 1][BC - 1];
+            each_of(std::make_integer_sequence<int, BC>{}, [&](auto I) {
+                constexpr int i = BC - 1 - decltype(I)::value, m0 = (i + 1) / 16;
+                double sn = 0.0, dn = 0.0;
+                each_of(std::make_integer_sequence<int, 4 - m0>{}, [&](auto M) {
+                    constexpr int m = m0 + decltype(M)::value;
+                    constexpr int ni = (m < 3) ? i : i - 1;           // the run after this one
+                    constexpr int nm = (m < 3) ? m + 1 : i / 16;
+                    double nxt[16];
+                    if constexpr (ni >= 0) {
+#pragma unroll
+                        for (int p = 0; p < 16; ++p) nxt[p] = (16 * nm + p > ni) ? T[ni][16 * nm + p] : 0.0;
+                        if constexpr (m == 3) {
+                            sn = Sx[ni][j];
+                            dn = T[ni][ni];
+                        }
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int p = 0; p < 16; ++p)
+                        if (16 * m + p > i) s = fma(-cur[p], x[16 * m + p], s);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if constexpr (ni >= 0)
+#pragma unroll
+                        for (int p = 0; p < 16; ++p) cur[p] = nxt[p];
+                });
+                if constexpr (i == BC - 1) {
+#pragma unroll
+                    for (int p = 0; p < 16; ++p) cur[p] = T[BC - 2][BC - 16 + p];
+                    sn = Sx[BC - 2][j];
+                    dn = T[BC - 2][BC - 2];
+                }
+                x[i] = s / dg;
+                s = sn;
+                dg = dn;
+                Xs[i][j] = x[i];                   // (the four lanes of a right-hand side alike)
+            });
+        } else if (k > 0) {
+            stage(k - 1);
+            // (opaque: the rows' offsets kept over the blocks would spill)
+            int ld = n, ldw = nrhs;
+            asm volatile("" : "+s"(ld), "+s"(ldw));
+            const int r0 = k0 - BC + ro;           // this wave's first row in block k - 1
+            d4 c;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) c[r] = Yc[r0 + 4 * r + g];
+            const double *Lr = S + r0 + j;
+            for (int q = 0; q < 16; ++q)           // (wanted after the barrier)
+                Ln[4 * q + g][ro + j] = Lr[(long)min(k0 + 4 * q + g, n - 1) * ld];
+            // half a block's rows at a time, one half ahead (only the last block has
+            // rows past the end: the last of L, zero of x)
+            double lv[8], xv[8];
+            auto load = [&](int b, int h) {
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+                    const int p = b * BC + 32 * h + 4 * q + g, pc = min(p, n - 1);
+                    lv[q] = Lr[(long)pc * ld];
+                    xv[q] = W[(long)pc * ldw + col];
+                    xv[q] = (p < n) ? xv[q] : 0.0;
+                }
+            };
+            if (nb - 1 > k) load(nb - 1, 0);
+            for (int b = nb - 1; b > k; --b) {
+                d4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    double lc[8], xc[8];
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) { lc[q] = lv[q]; xc[q] = xv[q]; }
+                    if (h == 0) load(b, 1);
+                    else if (b - 1 > k) load(b - 1, 0);
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) acc = mfma64(lc[q], xc[q], acc);
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) c[r] -= acc[r];
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) Sn[ro + 4 * r + g][j] = c[r];
+        }
+        __syncthreads();
+        if (w > 0) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int i = ro + 4 * r + g;
+                if (live && i < kb) W[(long)(k0 + i) * nrhs + col] = Xs[i][j];
+            }
+        }
+        if (w > 0 && k > 0) {
+            d4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                const int p = 4 * q + g;
+                acc = mfma64(Ln[p][ro + j], Xs[p][j], acc);   // (x is 0 past the end)
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                Sx[ro + 4 * r + g][j] = Sn[ro + 4 * r + g][j] - acc[r];
+        }
+        __syncthreads();
+    }
 }
 
 // Cholesky of A0 + (ridge + jitter) I with the lower triangle resident in LDS (one
@@ -1154,42 +1275,22 @@ int dg_centres_from_w(dg_ctx *c) {
     return DG_OK;
 }
 
-// (A0 + (ridge + jit) I) W = Bm for M + 1 > 126 by the blocked kernels;
-// clears scal[kScalSolveOK] on a non-positive pivot
+// (A0 + (ridge + jit) I) W = Bm for M + 1 > 126 by the blocked kernels, in the
+// (consumed) partials of A and B; clears scal[kScalSolveOK] on a non-positive pivot
 int blocked_chol_solve(dg_ctx *c, double ridge, double jit) {
-    const int n = c->M1, D = c->D;
+    const int n = c->M1, D = c->D, nb = (n + BC - 1) / BC;
+    double *S = c->partAB, *Ld = c->A;             // (n >= 127: n^2 > 64 (n + 63))
     const long tot = (long)n * n + (long)n * D;
     hipLaunchKernelGGL(k_bc_init, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, c->stream,
-                       c->A0, c->A, n, ridge, jit, c->Bm, c->W, D, c->scal);
-    const int nb = (n + BC - 1) / BC;
+                       c->A0, S, n, ridge, jit, c->Bm, D, c->scal);
     for (int k = 0; k < nb; ++k) {
-        const int k0 = k * BC, rest = n - k0 - BC;
-        hipLaunchKernelGGL(k_bc_potrf, dim3(1), dim3(256), 0, c->stream, c->A, n, k0, c->scal);
-        if (rest > 0) {
-            const int tb = (rest + BC - 1) / BC;
-            hipLaunchKernelGGL(k_bc_trsm, dim3((unsigned)((rest + 255) / 256)), dim3(256), 0,
-                               c->stream, c->A, n, k0, c->scal);
-            hipLaunchKernelGGL(k_bc_syrk, dim3((unsigned)tb, (unsigned)tb), dim3(256), 0, c->stream,
-                               c->A, n, k0, c->scal);
-        }
+        const int k1 = std::min(n, (k + 1) * BC);
+        const int rt = (n + D - k1 + BC - 1) / BC, ct = (k > 0) ? (n - k1 + BC - 1) / BC : 0;
+        hipLaunchKernelGGL(k_bc_step, dim3((unsigned)rt, (unsigned)(1 + ct)), dim3(kBcNT), 0,
+                           c->stream, S, n, n + D, k, Ld, c->scal);
     }
-    const unsigned rb = (unsigned)((D + BC - 1) / BC);
-    for (int k = 0; k < nb; ++k) {
-        const int k0 = k * BC, rest = n - k0 - BC;
-        hipLaunchKernelGGL(k_bc_fwd, dim3((unsigned)((D + 255) / 256)), dim3(256), 0, c->stream,
-                           c->A, n, k0, c->W, D, c->scal);
-        if (rest > 0)
-            hipLaunchKernelGGL((k_bc_update<true>), dim3((unsigned)((rest + BC - 1) / BC), rb),
-                               dim3(256), 0, c->stream, c->A, n, k0, c->W, D, c->scal);
-    }
-    for (int k = nb - 1; k >= 0; --k) {
-        const int k0 = k * BC;
-        hipLaunchKernelGGL(k_bc_bwd, dim3((unsigned)((D + 255) / 256)), dim3(256), 0, c->stream,
-                           c->A, n, k0, c->W, D, c->scal);
-        if (k0 > 0)
-            hipLaunchKernelGGL((k_bc_update<false>), dim3((unsigned)((k0 + BC - 1) / BC), rb),
-                               dim3(256), 0, c->stream, c->A, n, k0, c->W, D, c->scal);
-    }
+    hipLaunchKernelGGL(k_bc_back, dim3((unsigned)((D + 15) / 16)), dim3(kBcNT), 0, c->stream, S, n,
+                       D, Ld, c->W, c->scal);
     DG_HIP(c, hipGetLastError());
     return DG_OK;
 }

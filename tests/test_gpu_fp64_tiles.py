@@ -115,6 +115,7 @@ def test_ctemp_at_tile_edges(N, D, K):
     (40, 1, 3, 1), (60, 3, 17, 5), (200, 17, 64, 26), (150, 12, 65, 31), (300, 33, 130, 32),
     (260, 50, 127, 63), (300, 15, 500, 64), (300, 166, 260, 65), (400, 180, 600, 126),
     (300, 20, 700, 127), (300, 40, 700, 130), (400, 65, 900, 257), (300, 33, 1100, 400),
+    (300, 1, 300, 128), (300, 64, 300, 192), (350, 7, 400, 191),
 ])
 def test_mstep_at_tile_edges(N, D, K, M1):
     """One M-step at the edges of the products' and the factorisation's tiles,
