@@ -114,7 +114,7 @@ enum BKind {
     BK_MAKE_Y16, BK_BLOCK_LISTS, BK_COUNT
 };
 // tile sizes the flat grids are counted in (checked against the kernels)
-constexpr int kBRK = 64, kBRD = 16;     // k_reduce32: centres x dims per workgroup
+constexpr int kBRK = 64, kBRD = 4;      // k_reduce32: centres x rows per workgroup
 constexpr int kBCentres = 16;            // k_centres: centres per workgroup
 // One instance of a batched step, as the batched kernels read it from a
 // device table: the shape, the device buffers of its context and the
@@ -154,7 +154,7 @@ __host__ __device__ inline int bk_count(const BInst &I, int kind) {
     const auto cdiv = bk_cdiv;
     switch (kind) {
         case BK_MAKE_AK: return cdiv(I.Kp, 256);
-        case BK_REDUCE32: return cdiv(I.K, kBRK) * cdiv(I.D, kBRD);
+        case BK_REDUCE32: return cdiv(I.K, kBRK) * (I.D / kBRD + 1);   // D rows of R T, one of G
         case BK_ZERO_FIX: return I.D;
         case BK_PART_AB:
             return cdiv(I.M1, dg_ab_tile(I.M1)) * cdiv(I.M1 + I.D, dg_ab_tile(I.M1)) * I.nchAB;

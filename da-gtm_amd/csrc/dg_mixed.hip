@@ -1184,60 +1184,64 @@ __global__ __launch_bounds__(NTH) void k_item_table(const int2 *__restrict__ bra
 }
 
 // ---------------------------------------------------------------- helpers
-// RT[k][d] = sum_c partRT[c][d][k] and G[k] = sum_c partG[c][k], each in FP64
-// in chunk order.  One thread per output (lanes along the contiguous centre
-// axis); the chunk loop issues eight independent loads before it adds them,
-// in order.  A workgroup owns 64 centres x 16 dims and transposes them through
-// LDS so each FP64 row segment of RT is written as 128 contiguous bytes.
-// Workgroups of the first dim tile also sum G.
-constexpr int RK = 64, RD = 16, RU = 8;
+// RT[k][d] = sum_c partRT[c][d][k] and G[k] = sum_c partG[c][k] (row D of a
+// centre), each in FP64 in chunk order.  One thread per output (lanes along the
+// contiguous centre axis), 64 centres x 4 rows to a workgroup.  A chunk's partial
+// sums of a centre group exist only where pass 2 had blocks to visit (blocks > 0
+// in the pair's run-table entry): the workgroup lists those chunks first and
+// reads no others, sixteen loads in flight, added in order.  Small workgroups:
+// the chain over the chunks is a thread's, so the load latencies of few outputs
+// with many chunks have to spread over the chip.
+// Bound by memory where there are many outputs, by the loads' latency where
+// there are few.  N = 100000, K = 8000, D = 166: 44 -> 19 us; N = 10^6, the same:
+// 166 -> 41; N = 50000, K = 1600, D = 64: 56 -> 14.5; N = 1000, K = 400, D = 12:
+// 11.5 -> 3.7 (16-row workgroups, every chunk read, eight loads in flight).
+constexpr int RK = 64, RD = 4, RU = 16;
 
 __device__ __forceinline__ void k_reduce32_body(
     const int bx, const int by, const int bz, const int gx, const float *__restrict__ partRT,
     const float *__restrict__ partG, int NC, int K, int D, double *__restrict__ RT,
     double *__restrict__ G, const int2 *__restrict__ brange) {
     __shared__ double tile[RK][RD + 1];
+    __shared__ int lst[RK * RD], cnt[RD];
     const int t = threadIdx.x, kk = t & (RK - 1), dd = t / RK;
     const int k0 = bx * RK, d0 = by * RD;
-    const int k = k0 + kk, d = d0 + dd;
-    const long KD = (long)K * D;
-    // chunk c's partial sums of this centre group exist only where pass 2 had
-    // blocks to visit (blocks > 0 in the pair's run-table entry; no table:
-    // everywhere)
+    const int k = min(k0 + kk, K - 1), d = min(d0 + dd, D);
+    const long step = (d < D) ? (long)K * D : K;
+    const float *p = (d < D) ? partRT + (long)d * K + k : partG + k;
     const int KG = (K + CT - 1) / CT, grp = k0 / CT;
-    auto live = [&](int c) { return !brange || brange[RS * ((long)c * KG + grp)].y > 0; };
     double s = 0.0;
-    if (k < K && d < D) {
-        const float *p = partRT + (long)d * K + k;
-        int c = 0;
-        for (; c + RU <= NC; c += RU) {
+    for (int c0 = 0; c0 < NC; c0 += RK * RD) {
+        const int c = c0 + t;
+        const bool live = c < NC && brange[RS * ((long)c * KG + grp)].y > 0;
+        const unsigned long long bal = __ballot(live);
+        const int pos = __builtin_amdgcn_mbcnt_hi((unsigned)(bal >> 32),
+                                                  __builtin_amdgcn_mbcnt_lo((unsigned)bal, 0));
+        if (kk == 0) cnt[dd] = __popcll(bal);
+        __syncthreads();
+        int off = 0, m = 0;
+#pragma unroll
+        for (int w = 0; w < RD; ++w) {
+            if (w < dd) off += cnt[w];
+            m += cnt[w];
+        }
+        if (live) lst[off + pos] = c;
+        __syncthreads();
+        for (int i = 0; i < m; i += RU) {
             float v[RU];
 #pragma unroll
-            for (int u = 0; u < RU; ++u) v[u] = p[(long)(c + u) * KD];
+            for (int u = 0; u < RU; ++u) v[u] = p[lst[min(i + u, m - 1)] * step];
 #pragma unroll
-            for (int u = 0; u < RU; ++u) s += live(c + u) ? (double)v[u] : 0.0;
+            for (int u = 0; u < RU; ++u) s += (i + u < m) ? (double)v[u] : 0.0;
         }
-        for (; c < NC; ++c) s += live(c) ? (double)p[(long)c * KD] : 0.0;
+        __syncthreads();                           // before the next chunks' list
     }
     tile[kk][dd] = s;
     __syncthreads();
-    {
-        const int r = t / RD, e = t % RD;
-        if (k0 + r < K && d0 + e < D) RT[(long)(k0 + r) * D + d0 + e] = tile[r][e];
-    }
-    if (by == 0 && t < RK && k < K) {
-        // RU loads in flight, then their sums in chunk order (as for R T)
-        double g = 0.0;
-        int c = 0;
-        for (; c + RU <= NC; c += RU) {
-            float v[RU];
-#pragma unroll
-            for (int u = 0; u < RU; ++u) v[u] = partG[(long)(c + u) * K + k];
-#pragma unroll
-            for (int u = 0; u < RU; ++u) g += live(c + u) ? (double)v[u] : 0.0;
-        }
-        for (; c < NC; ++c) g += live(c) ? (double)partG[(long)c * K + k] : 0.0;
-        G[k] = g;
+    const int r = t / RD, e = t % RD;
+    if (k0 + r < K) {
+        if (d0 + e < D) RT[(long)(k0 + r) * D + d0 + e] = tile[r][e];
+        else if (d0 + e == D) G[k0 + r] = tile[r][e];
     }
 }
 
@@ -1692,12 +1696,15 @@ __global__ __launch_bounds__(NTH) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         if (item >= total) break;
         const BInst &I = find_inst<true>(tab, list, nlist, item);
         if (!I.do_e) continue;
-        // the instance's items in XCD-aware order, empty ones included (they
-        // write zero partial sums; the queue hands items out dynamically)
+        // the instance's items in XCD-aware order; a pair without blocks has
+        // no partial sums, and kb_reduce32 reads none
         const int L = item - I.item_e2, KGi = I.Kp / CT, xs = L & 7, sl = L >> 3;
-        e2_body<KS, TT, GM, RLO>((long)(sl / KGi) * 8 + xs, sl % KGi, opaque_tid(), I.T16, I.T16t, I.Np, I.Y16, I.yy32, I.K, I.Kp,
-                                 I.D, I.mscal, I.beta_f, I.it, I.pP32, I.blkThr, I.CL,
-                                 I.Kp / CT, I.partRT32, I.partG32, I.brange);
+        const long cidx = (long)(sl / KGi) * 8 + xs;
+        const int kg = sl % KGi;
+        if (I.brange[RS * (cidx * KGi + kg)].y <= 0) continue;
+        e2_body<KS, TT, GM, RLO>(cidx, kg, opaque_tid(), I.T16, I.T16t, I.Np, I.Y16, I.yy32, I.K,
+                                 I.Kp, I.D, I.mscal, I.beta_f, I.it, I.pP32, I.blkThr, I.CL, KGi,
+                                 I.partRT32, I.partG32, I.brange);
     }
 }
 
@@ -1733,7 +1740,7 @@ __global__ __launch_bounds__(RK * RD) void kb_reduce32(const BInst *__restrict__
     if (!I.do_e) return;
     const int nkx = (I.K + RK - 1) / RK;
     k_reduce32_body(m.y % nkx, m.y / nkx, 0, 0, I.partRT32, I.partG32, I.NC, I.K, I.D, I.RT,
-                    I.G, nullptr);
+                    I.G, I.brange);
 }
 
 __global__ __launch_bounds__(256) void kb_zero_fix(const BInst *__restrict__ tab,
@@ -2114,7 +2121,7 @@ int dg_estep_mixed(dg_ctx *c, int isDA, double temp) {
     DG_HIP(c, hipGetLastError());
     if (c->timing) DG_HIP(c, hipEventRecord(c->ev[2], c->stream));
     hipLaunchKernelGGL(k_reduce32,
-                       dim3((unsigned)((c->K + RK - 1) / RK), (unsigned)((c->D + RD - 1) / RD)),
+                       dim3((unsigned)((c->K + RK - 1) / RK), (unsigned)(c->D / RD + 1)),
                        dim3(RK * RD), 0, c->stream, c->partRT32, c->partG32, b->NC, c->K, c->D,
                        c->RT, c->G, b->brange);
     DG_HIP(c, hipGetLastError());
