@@ -187,6 +187,12 @@ int download_rows(dg_ctx *c, double *dst, long ldd, const double *src, long rows
     return e == hipSuccess ? DG_OK : dg_hip_check(c, e, "copy to the host");
 }
 
+// the step's kernels leave their scalars in h_scal themselves
+int sync_step(dg_ctx *c) {
+    DG_HIP(c, hipStreamSynchronize(c->stream));
+    return DG_OK;
+}
+
 int sync_scalars(dg_ctx *c) {
     DG_HIP(c, hipMemcpyAsync(c->h_scal, c->scal, kScalCount * sizeof(double),
                              hipMemcpyDeviceToHost, c->stream));
@@ -313,7 +319,8 @@ int dg_create(const dg_config *cfg, dg_ctx **out) {
         if (hipEventCreate(&ev) != hipSuccess) { dg_destroy(c); return DG_EHIP; }
     if (dalloc(c, &c->scal, kScalCount) != DG_OK ||
         hipHostMalloc((void **)&c->h_scal, kScalCount * sizeof(double), hipHostMallocDefault) !=
-            hipSuccess) {
+            hipSuccess ||
+        hipHostGetDevicePointer((void **)&c->m_scal, c->h_scal, 0) != hipSuccess) {
         dg_destroy(c);
         return DG_ENOMEM;
     }
@@ -410,7 +417,7 @@ int dg_estep(dg_ctx *c, int isDA, double temp, dg_estep_out *out) {
     else rc = dg_estep_fp64(c, isDA, temp);
     if (rc) return rc;
     if (c->timing) DG_HIP(c, hipEventRecord(c->ev[3], c->stream));
-    if ((rc = sync_scalars(c))) return rc;
+    if ((rc = sync_step(c))) return rc;
     if (c->timing) {
         float a = 0, b = 0, d = 0;
         (void)hipEventElapsedTime(&a, c->ev[0], c->ev[1]);
@@ -447,7 +454,7 @@ int dg_mstep(dg_ctx *c, double *beta_out) {
     if (c->timing) DG_HIP(c, hipEventRecord(c->ev[4], c->stream));
     if ((rc = dg_mstep_run(c, 0.0))) return rc;
     if (c->timing) DG_HIP(c, hipEventRecord(c->ev[5], c->stream));
-    if ((rc = sync_scalars(c))) return rc;
+    if ((rc = sync_step(c))) return rc;
     if (c->h_scal[kScalSolveOK] != 1.0 && c->M1 > 126) {
         // a non-positive pivot: retry with a jitter of 1e-13 tr(A) / n, growing
         // x10 per retry, at most 8 retries (the policy of the one-kernel
@@ -455,7 +462,7 @@ int dg_mstep(dg_ctx *c, double *beta_out) {
         if ((rc = dg_mstep_trace(c)) || (rc = sync_scalars(c))) return rc;
         double jit = 1e-13 * c->h_scal[kScalJitter] / c->M1;
         for (int attempt = 1; attempt <= 8; ++attempt, jit *= 10.0) {
-            if ((rc = dg_mstep_run(c, jit)) || (rc = sync_scalars(c))) return rc;
+            if ((rc = dg_mstep_run(c, jit)) || (rc = sync_step(c))) return rc;
             if (c->h_scal[kScalSolveOK] == 1.0) break;
         }
     }

@@ -546,11 +546,12 @@ __global__ __launch_bounds__(NT, 2) void k_e2_f64(
 }
 
 // RT and G from the chunk partials, summed in chunk order with eight loads in
-// flight; the last workgroup sums pass 1's partial log sums into scal instead.
+// flight; the last workgroup sums pass 1's partial log sums into scal and the host's
+// copy of it (pinned: a copy of 64 bytes after the step took 5 us) instead.
 __global__ __launch_bounds__(256) void k_reduce_parts(
     const double *__restrict__ partRT, const double *__restrict__ partG, int NC, int K, int D,
     double *__restrict__ RT, double *__restrict__ G, const double *__restrict__ partLog, long nlog,
-    double *__restrict__ scal) {
+    double *__restrict__ scal, double *__restrict__ hscal) {
     if (blockIdx.x == gridDim.x - 1) {
         __shared__ double s[3][256];
         double a[3] = {0.0, 0.0, 0.0};
@@ -564,9 +565,9 @@ __global__ __launch_bounds__(256) void k_reduce_parts(
             __syncthreads();
         }
         if (threadIdx.x == 0) {
-            scal[kScalSumLogG] = s[0][0];
-            scal[kScalSumLogH] = s[1][0];
-            scal[kScalNZero] = s[2][0];
+            scal[kScalSumLogG] = hscal[kScalSumLogG] = s[0][0];
+            scal[kScalSumLogH] = hscal[kScalSumLogH] = s[1][0];
+            scal[kScalNZero] = hscal[kScalNZero] = s[2][0];
         }
         return;
     }
@@ -1061,7 +1062,7 @@ int dg_estep_fp64(dg_ctx *c, int isDA, double temp) {
     const long nred = (long)c->K * c->D + c->K;
     hipLaunchKernelGGL(k_reduce_parts, dim3((unsigned)((nred + 255) / 256 + 1)), dim3(256), 0,
                        c->stream, c->partRT, c->partG, c->NC, c->K, c->D, c->RT, c->G,
-                       c->partLog64, dg_pass1_wgs(c->N), c->scal);
+                       c->partLog64, dg_pass1_wgs(c->N), c->scal, c->m_scal);
     DG_HIP(c, hipGetLastError());
     return DG_OK;
 }

@@ -63,6 +63,7 @@ struct dg_ctx {
     int nchAB = 1;                 // centre chunks of the A/B reduction
     double *scal = nullptr;        // device scalars (see kScal*)
     double *h_scal = nullptr;      // pinned host mirror
+    double *m_scal = nullptr;      // its device address: the last kernel of a step writes there
 
     // ---- mixed-precision state ----
     int mixed_ready = 0;

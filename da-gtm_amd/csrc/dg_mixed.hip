@@ -570,35 +570,37 @@ __global__ __launch_bounds__(NTH) __attribute__((amdgpu_waves_per_eu(KS <= 11 ? 
                                         perm, gmx, bnd, t0, smargin);
 }
 
-// scal[0..2] = sums over the pass-1 workgroup partials (fixed tree order).
-__device__ __forceinline__ void k_sum_partlog_body(
-    const int bx, const int by, const int bz, const int gx, const double *__restrict__ part,
-    long nb, double *__restrict__ scal) {
-    __shared__ double s[3][1024];
-    double a = 0.0, b = 0.0, c = 0.0;
-    for (long i = threadIdx.x; i < nb; i += 1024) {
-        a += part[3 * i]; b += part[3 * i + 1]; c += part[3 * i + 2];
-    }
-    s[0][threadIdx.x] = a; s[1][threadIdx.x] = b; s[2][threadIdx.x] = c;
+// scal[0..2] = sums over the pass-1 workgroup partials, in hscal too if there is one:
+// 1024 chains in a fixed tree, four of them to a thread.
+__device__ __forceinline__ void k_sum_partlog_body(const double *__restrict__ part, long nb,
+                                                   double *__restrict__ scal,
+                                                   double *__restrict__ hscal) {
+    __shared__ double s[3][256];
+    double a[4][3] = {};
+    for (long i = threadIdx.x; i < nb; i += 1024)
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int x = 0; x < 3; ++x)
+                a[u][x] += (i + 256 * u < nb) ? part[3 * (i + 256 * u) + x] : 0.0;
+#pragma unroll
+    for (int x = 0; x < 3; ++x)
+        s[x][threadIdx.x] = (a[0][x] + a[2][x]) + (a[1][x] + a[3][x]);
     __syncthreads();
-    for (int w = 512; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) {
-            s[0][threadIdx.x] += s[0][threadIdx.x + w];
-            s[1][threadIdx.x] += s[1][threadIdx.x + w];
-            s[2][threadIdx.x] += s[2][threadIdx.x + w];
-        }
+    for (int w = 128; w > 0; w >>= 1) {
+        if ((int)threadIdx.x < w)
+#pragma unroll
+            for (int x = 0; x < 3; ++x) s[x][threadIdx.x] += s[x][threadIdx.x + w];
         __syncthreads();
     }
     if (threadIdx.x == 0) {
-        scal[kScalSumLogG] = s[0][0];
-        scal[kScalSumLogH] = s[1][0];
-        scal[kScalNZero] = s[2][0];
+        constexpr int slot[3] = {kScalSumLogG, kScalSumLogH, kScalNZero};
+#pragma unroll
+        for (int x = 0; x < 3; ++x) {
+            scal[slot[x]] = s[x][0];
+            if (hscal) hscal[slot[x]] = s[x][0];
+        }
     }
-}
-
-__global__ __launch_bounds__(1024) void k_sum_partlog(const double *__restrict__ part, long nb,
-                                                      double *__restrict__ scal) {
-    k_sum_partlog_body(blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, part, nb, scal);
 }
 
 // Per-centre exponent term of pass 1, -beta log2(e) |y_k|^2 / 2 (the same
@@ -1155,10 +1157,19 @@ __global__ __launch_bounds__(NTH) void k_block_ranges(const float *__restrict__ 
 // Pass 2's work list, one workgroup per XCD x: the (chunk, group) pairs of
 // chunks c = x, x + 8, ... (chunk after chunk, groups in order) whose block
 // range is not empty, at itab[x + 8 i] (i = 0, 1, ...), and their number
-// icnt[x].  Ballots and per-wave counts keep the order.
+// icnt[x].  Ballots and per-wave counts keep the order.  A ninth workgroup sums
+// pass 1's partial log sums (a launch of its own took 4 us).
 __global__ __launch_bounds__(NTH) void k_item_table(const int2 *__restrict__ brange, int NC,
                                                      int KG, int *__restrict__ itab,
-                                                     int *__restrict__ icnt) {
+                                                     int *__restrict__ icnt,
+                                                     const double *__restrict__ partLog, long nlog,
+                                                     double *__restrict__ scal,
+                                                     double *__restrict__ hscal) {
+    static_assert(NTH == 256, "k_sum_partlog_body's workgroup");
+    if (blockIdx.x == 8) {
+        k_sum_partlog_body(partLog, nlog, scal, hscal);
+        return;
+    }
     __shared__ int s_w[NTH / 64];
     const int x = blockIdx.x;
     const int nch = (NC - x + 7) / 8;              // this XCD's chunks
@@ -1573,8 +1584,8 @@ void launch_mixed(dg_ctx *c, MixedBufs *b, float beta, float it, int two, int is
     constexpr int DR = 32 * ((16 * KS + 31) / 32);
     hipLaunchKernelGGL(k_block_ranges, dim3((unsigned)(KG * b->NC)), dim3(NTH), 0, c->stream,
                        b->bnd, b->Np, chunk, KG, skip_below(DR > c->D), b->brange);
-    hipLaunchKernelGGL(k_item_table, dim3(8), dim3(NTH), 0, c->stream, b->brange, b->NC, KG,
-                       b->itab, b->icnt);
+    hipLaunchKernelGGL(k_item_table, dim3(9), dim3(NTH), 0, c->stream, b->brange, b->NC, KG,
+                       b->itab, b->icnt, b->partLog, b->Np / PT, c->scal, c->m_scal);
     if (DR > c->D) launch_e2<KS, TT, true>(c, b, beta, it, chunk, KG);
     else launch_e2<KS, TT, false>(c, b, beta, it, chunk, KG);
 }
@@ -1726,11 +1737,11 @@ __global__ __launch_bounds__(256) void kb_make_ak(const BInst *__restrict__ tab,
     k_make_ak_body(m.y, 0, 0, 0, I.yy32, I.K, I.Kp, I.beta_f, I.aK32);
 }
 
-__global__ __launch_bounds__(1024) void kb_sum_partlog(const BInst *__restrict__ tab,
+__global__ __launch_bounds__(256) void kb_sum_partlog(const BInst *__restrict__ tab,
                                                        const int *__restrict__ list) {
     const BInst &I = tab[list[blockIdx.x]];
     if (!I.do_e) return;
-    k_sum_partlog_body(0, 0, 0, 1, I.partLog, I.Np / PT, I.scal);
+    k_sum_partlog_body(I.partLog, I.Np / PT, I.scal, nullptr);
 }
 
 __global__ __launch_bounds__(RK * RD) void kb_reduce32(const BInst *__restrict__ tab,
@@ -2125,9 +2136,6 @@ int dg_estep_mixed(dg_ctx *c, int isDA, double temp) {
                        dim3(RK * RD), 0, c->stream, c->partRT32, c->partG32, b->NC, c->K, c->D,
                        c->RT, c->G, b->brange);
     DG_HIP(c, hipGetLastError());
-    hipLaunchKernelGGL(k_sum_partlog, dim3(1), dim3(1024), 0, c->stream, b->partLog, b->Np / PT,
-                       c->scal);
-    DG_HIP(c, hipGetLastError());
     hipLaunchKernelGGL(k_zero_fix, dim3((unsigned)c->D), dim3(256), 0, c->stream, c->scal, c->T64,
                        c->ldt, c->pm, c->N, c->K, c->D, c->RT, c->G);
     DG_HIP(c, hipGetLastError());
@@ -2184,7 +2192,7 @@ int dg_batch_estep(hipStream_t st, const BInst *tab, const int *list, int n, con
         rc = (k.TT == 1) ? launch_class<1>(k, ss, tab, list, counters, false, cus)
                          : launch_class<2>(k, ss, tab, list, counters, false, cus);
         if (rc) return rc;
-        hipLaunchKernelGGL(kb_sum_partlog, dim3(un), dim3(1024), 0, ss, tab, l);
+        hipLaunchKernelGGL(kb_sum_partlog, dim3(un), dim3(256), 0, ss, tab, l);
         hipLaunchKernelGGL(kb_block_ranges, dim3((unsigned)k.wg_lists), dim3(NTH), 0, ss, tab,
                            k.map_lists);
         rc = (k.TT == 1) ? launch_class<1>(k, ss, tab, list, counters, true, cus)

@@ -1158,10 +1158,14 @@ __device__ __forceinline__ void k_beta_final_body(const double *__restrict__ par
     }
 }
 
+// (hscal: the host's copy of the M-step's scalars, in pinned memory)
 __global__ __launch_bounds__(256) void k_beta_final(const double *__restrict__ part, int n,
-                                                    const double *__restrict__ amax,
-                                                    double *__restrict__ scal) {
+                                                    const double *__restrict__ amax, double *scal,
+                                                    double *__restrict__ hscal) {
     k_beta_final_body(part, n, amax, scal);
+    __syncthreads();
+    const int i = kScalBetaSum + (int)threadIdx.x;
+    if (i <= kScalYMax) hscal[i] = scal[i];
 }
 
 // ---------------------------------------------------------------- batched
@@ -1336,7 +1340,8 @@ int dg_mstep_run(dg_ctx *c, double jitter) {
     hipLaunchKernelGGL(k_centres, dim3((unsigned)nb), dim3(256), 0, c->stream, c->FI, c->W, K, M1, D,
                        c->ldt, c->G, c->RT, c->Y64, c->yy, c->partAB, amax);
     DG_HIP(c, hipGetLastError());
-    hipLaunchKernelGGL(k_beta_final, dim3(1), dim3(256), 0, c->stream, c->partAB, nb, amax, c->scal);
+    hipLaunchKernelGGL(k_beta_final, dim3(1), dim3(256), 0, c->stream, c->partAB, nb, amax, c->scal,
+                       c->m_scal);
     DG_HIP(c, hipGetLastError());
     return DG_OK;
 }
