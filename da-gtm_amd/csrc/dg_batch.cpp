@@ -246,7 +246,7 @@ int dg_batch_run_mixed(std::vector<dg_ctx *> &ctx, const dg_anneal_params *param
     }
     for (int kind : {BK_PART_AB, BK_SUM_AB, BK_CENTRES})
         whole(b.h_list + n, n, kind);
-    whole(b.h_list + n, b.nlds, BK_TRSM_LDS);
+    whole(b.h_list + n, b.nlds, BK_SOLVE_LDS);
     DG_HIP(nullptr, hipMalloc((void **)&b.d_map, sizeof(int2) * std::max<size_t>(1, hmap.size())));
     DG_HIP(nullptr, hipMemcpy(b.d_map, hmap.data(), sizeof(int2) * hmap.size(),
                               hipMemcpyHostToDevice));

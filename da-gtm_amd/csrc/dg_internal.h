@@ -111,7 +111,7 @@ enum {
 // each instance with exactly its own workgroup count (bk_count): a device map
 // per launch gives workgroup g its (table index, workgroup within instance).
 enum BKind {
-    BK_MAKE_AK, BK_REDUCE32, BK_ZERO_FIX, BK_PART_AB, BK_SUM_AB, BK_TRSM_LDS, BK_CENTRES,
+    BK_MAKE_AK, BK_REDUCE32, BK_ZERO_FIX, BK_PART_AB, BK_SUM_AB, BK_SOLVE_LDS, BK_CENTRES,
     BK_MAKE_Y16, BK_BLOCK_LISTS, BK_COUNT
 };
 // tile sizes the flat grids are counted in (checked against the kernels)
@@ -160,7 +160,7 @@ __host__ __device__ inline int bk_count(const BInst &I, int kind) {
         case BK_PART_AB:
             return cdiv(I.M1, dg_ab_tile(I.M1)) * cdiv(I.M1 + I.D, dg_ab_tile(I.M1)) * I.nchAB;
         case BK_SUM_AB: return cdiv((long)I.M1 * I.M1 + (long)I.M1 * I.D, 256) + cdiv(I.K, 256);
-        case BK_TRSM_LDS: return cdiv(I.D, 16);
+        case BK_SOLVE_LDS: return cdiv(I.D, 16);
         case BK_CENTRES: return cdiv(I.K, kBCentres);
         case BK_MAKE_Y16: return cdiv(I.Kp, 4);
         case BK_BLOCK_LISTS: return (I.Kp / 128) * I.NC;

@@ -741,28 +741,53 @@ __global__ __launch_bounds__(kBcNT) void k_bc_back(const double *__restrict__ S,
     }
 }
 
-// Cholesky of A0 + (ridge + jitter) I with the lower triangle resident in LDS (one
-// workgroup, n <= 126); same pivots and retries as k_chol_solve.  Blocked,
-// right-looking: wave 0 factors each 8-column panel in registers (lane r
-// holds rows p0 + r and p0 + r + 64; the pivot row and the L entries of later
-// panel columns are broadcast with readlane, so the panel needs no barrier),
+// W[:, c0 : c0 + 16] from (A0 + (ridge + jitter) I) W = B for n <= 126, the lower
+// triangle resident in LDS; same pivots and retries as k_chol_solve.  Every
+// workgroup factors the matrix for itself (they run side by side, and the factor
+// need not go through memory to a second kernel).
+//   Factor: blocked, right-looking.  Wave 0 takes each 8-column panel in registers
+// (lane r holds rows p0 + r and p0 + r + 64; the pivot row and the L entries of
+// later panel columns are broadcast with readlane, so the panel needs no barrier),
 // then all waves apply the panel to the trailing lower triangle, a 16 x 16 tile
 // at a time on matrix instructions (the chain over the panel's columns from 0,
-// subtracted from the tile).  Two barriers per panel.  Writes the factor's lower
-// triangle only.
-// Bound by the panels' chains of square roots and reciprocals, one CU's latency:
-// n = 126: 90 -> 55 us, n = 26: 17 -> 13 (trailing updates by 4 x 4 register
-// tiles over 32 x 32 threads, whatever was left of the triangle).
-__device__ __forceinline__ void k_chol_lds_body(
-    const int bx, const int by, const int bz, const int gx, const double *__restrict__ A0,
-    double *__restrict__ L, int n, double ridge, double *__restrict__ scal) {
-    __shared__ double As[kLdsN * (kLdsN | 1)];
+// subtracted from the tile).  Two barriers per panel.
+//   Solve: the right-hand sides in 16-row blocks, block t in the accumulator of
+// wave t.  For each block in turn its wave solves the 16 x 16 triangle in the
+// accumulator's layout, and the waves then apply the block's x to their blocks on
+// matrix instructions.  Each row receives its updates in the order of the plain
+// substitution: x_i = x_i (1 / L_ii), then one FMA per later row in ascending i
+// (forward), or per earlier row in descending i (backward, the MFMA's inner index
+// running down).
+// Bound by the chains of square roots, reciprocals and blocks, one CU's latency.
+// n = 126: 72 us, n = 65: 40, n = 26: 18.6; as two kernels, 55 + 35, 27 + 22
+// and 13 + 9 and the gap between them, and 90 + 48, 45 + 27 and 17 + 15 with 4 x 4
+// register tiles of FMAs and a wave per right-hand side.
+constexpr int kCholNT = 1024;
+__device__ __forceinline__ void k_solve_lds_body(
+    const int bx, const double *__restrict__ A0, int n, double ridge, const double *__restrict__ B,
+    int nrhs, double *__restrict__ W, double *__restrict__ scal) {
+    __shared__ double As[128 * (kLdsN | 1) + 16];
     __shared__ double Pt[kPB][128 + 16];             // the factored panel, transposed
     __shared__ double tr;
     __shared__ int bad;
+    __shared__ double rd[128];                       // 1 / L_pp
+    __shared__ double xs[16][17];                    // the block just solved
     const int tid = threadIdx.x, nw = blockDim.x >> 6;
-    const int lane = tid & 63, wv = tid >> 6, j = lane & 15, g = lane >> 4;
+    const int lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int j = lane & 15, g = lane >> 4;
     const int ld = n | 1;                            // odd: a column spreads over the banks
+    const int nblk = (n + 15) / 16;
+    const int col = 16 * bx + j;
+    const bool live = col < nrhs;
+    d4 x = {0.0, 0.0, 0.0, 0.0};                     // block wv
+    if (wv < nblk)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int p = 16 * wv + 4 * r + g;
+            x[r] = (live && p < n) ? B[(long)p * nrhs + col] : 0.0;
+        }
+    // rows past the end: zero entries of L, and zero right-hand sides
+    for (int e = n * ld + tid; e < 16 * nblk * ld + 16; e += blockDim.x) As[e] = 0.0;
     double jit = 0.0;
     int ok = 0;
     for (int attempt = 0; attempt < 9 && !ok; ++attempt) {
@@ -844,59 +869,14 @@ __device__ __forceinline__ void k_chol_lds_body(
         ok = !bad;
         __syncthreads();                                     // before the next attempt resets bad
     }
-    if (tid == 0) {
+    if (tid == 0 && bx == 0) {
         scal[kScalJitter] = jit;
         scal[kScalSolveOK] = ok ? 1.0 : 0.0;
     }
-    for (int i = wv; i < n; i += nw)
-        for (int k = lane; k <= i; k += 64) L[(long)i * n + k] = As[i * ld + k];
-}
-
-constexpr int kCholNT = 1024;
-__global__ __launch_bounds__(kCholNT) void k_chol_lds(const double *__restrict__ A0,
-                                                      double *__restrict__ L, int n, double ridge,
-                                                      double *__restrict__ scal) {
-    k_chol_lds_body(blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, A0, L, n, ridge, scal);
-}
-
-// W[:, c0 : c0 + 16] from L y = b, L^T x = y (n <= 126), one workgroup of four
-// waves: L's lower triangle in LDS, the right-hand sides in 16-row blocks, block
-// t in the accumulator of wave t % 4.  For each block in turn its wave solves the
-// 16 x 16 triangle in the accumulator's layout, and the waves then apply the
-// block's x to their other blocks on matrix instructions.  Each row receives its
-// updates in the order of the plain substitution: x_i = x_i (1 / L_ii), then one
-// FMA per later row in ascending i (forward), or per earlier row in descending i
-// (backward, the MFMA's inner index running down).
-// Bound by the chain of blocks (8 each way at n = 126): 48 -> 35 us, n = 26:
-// 15 -> 9 (a wave per right-hand side, one row at a time: a step of the chain
-// for each of n rows).
-__device__ __forceinline__ void k_trsm_lds_body(
-    const int bx, const int by, const int bz, const int gx, const double *__restrict__ L, int n,
-    const double *__restrict__ B, int nrhs, double *__restrict__ W,
-    const double *__restrict__ scal) {
-    if (scal[kScalSolveOK] != 1.0) return;
-    __shared__ double Ls[128 * (kLdsN | 1) + 16];
-    __shared__ double rd[128];                     // 1 / L_pp
-    __shared__ double xs[16][17];                  // the block just solved
-    const int tid = threadIdx.x, l = tid & 63, w = tid >> 6, j = l & 15, g = l >> 4;
-    const int ld = n | 1, nblk = (n + 15) / 16;
-    load_lower(L, n, [&](int i, int k, double v) { Ls[i * ld + k] = v; });
-    // rows past the end: zero entries of L, and zero right-hand sides
-    for (int e = n * ld + tid; e < 16 * nblk * ld + 16; e += 256) Ls[e] = 0.0;
-    const int col = 16 * bx + j;
-    const bool live = col < nrhs;
-    auto at = [&](int i, int k) { return Ls[i * ld + k]; };   // k <= i
-    d4 x[2];                                       // blocks w and w + 4
-#pragma unroll
-    for (int q = 0; q < 2; ++q)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int p = 16 * (w + 4 * q) + 4 * r + g;
-            x[q][r] = (live && p < n) ? B[(long)p * nrhs + col] : 0.0;
-        }
+    if (!ok) return;
+    if (tid < 128) rd[tid] = (tid < n) ? 1.0 / As[tid * ld + tid] : 0.0;
     __syncthreads();
-    if (tid < 128) rd[tid] = (tid < n) ? 1.0 / Ls[tid * ld + tid] : 0.0;
-    __syncthreads();
+    auto at = [&](int i, int k) { return As[i * ld + k]; };   // k <= i
     // block t's triangle, in the accumulator's layout: row i = 4 R + G goes from
     // its lanes to the others of its column, which update their later (earlier)
     // rows; xs gets the solved rows
@@ -921,52 +901,36 @@ __device__ __forceinline__ void k_trsm_lds_body(
 #pragma unroll
         for (int r = 0; r < 4; ++r) xs[4 * r + g][j] = c[r];
     };
-    for (int t = 0; t < nblk; ++t) {               // forward
-        if (w == (t & 3)) {
-            if (t < 4) diag(t, x[0], std::true_type{});
-            else diag(t, x[1], std::true_type{});
-        }
+    for (int t = 0; t < nblk; ++t) {                 // forward
+        if (wv == t) diag(t, x, std::true_type{});
         __syncthreads();
+        if (wv > t && wv < nblk)
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const int u = w + 4 * q;
-            if (u > t && u < nblk)
-#pragma unroll
-                for (int s4 = 0; s4 < 16; s4 += 4)
-                    x[q] = mfma64(-at(16 * u + j, 16 * t + s4 + g), xs[s4 + g][j], x[q]);
-        }
-        __syncthreads();                           // xs is rewritten by the next block
+            for (int s4 = 0; s4 < 16; s4 += 4)
+                x = mfma64(-at(16 * wv + j, 16 * t + s4 + g), xs[s4 + g][j], x);
+        __syncthreads();                             // xs is rewritten by the next block
     }
-    for (int t = nblk - 1; t >= 0; --t) {          // backward with L^T, i descending
-        if (w == (t & 3)) {
-            if (t < 4) diag(t, x[0], std::false_type{});
-            else diag(t, x[1], std::false_type{});
-        }
+    for (int t = nblk - 1; t >= 0; --t) {            // backward with L^T, i descending
+        if (wv == t) diag(t, x, std::false_type{});
         __syncthreads();
+        if (wv < t)
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const int u = w + 4 * q;
-            if (u < t)
-#pragma unroll
-                for (int s4 = 15; s4 > 0; s4 -= 4)
-                    x[q] = mfma64(-at(16 * t + s4 - g, 16 * u + j), xs[s4 - g][j], x[q]);
-        }
+            for (int s4 = 15; s4 > 0; s4 -= 4)
+                x = mfma64(-at(16 * t + s4 - g, 16 * wv + j), xs[s4 - g][j], x);
         __syncthreads();
     }
 #pragma unroll
-    for (int q = 0; q < 2; ++q)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int p = 16 * (w + 4 * q) + 4 * r + g;
-            if (live && p < n) W[(long)p * nrhs + col] = x[q][r];
-        }
+    for (int r = 0; r < 4; ++r) {
+        const int p = 16 * wv + 4 * r + g;
+        if (live && p < n) W[(long)p * nrhs + col] = x[r];
+    }
 }
 
-__global__ __launch_bounds__(256) void k_trsm_lds(const double *__restrict__ L, int n,
-                                                  const double *__restrict__ B, int nrhs,
-                                                  double *__restrict__ W,
-                                                  const double *__restrict__ scal) {
-    k_trsm_lds_body(blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, L, n, B, nrhs, W, scal);
+__global__ __launch_bounds__(kCholNT) void k_solve_lds(const double *__restrict__ A0, int n,
+                                                       double ridge, const double *__restrict__ B,
+                                                       int nrhs, double *__restrict__ W,
+                                                       double *__restrict__ scal) {
+    k_solve_lds_body(blockIdx.x, A0, n, ridge, B, nrhs, W, scal);
 }
 
 // The new centres and what the M-step takes from them, sixteen centres to a
@@ -1198,19 +1162,12 @@ __global__ __launch_bounds__(256) void kb_sumAB(const BInst *__restrict__ tab, c
     k_sumAB_body(m.y, 0, 0, 0, I.partAB, I.nchAB, I.M1, I.D, I.A0, I.Bm, I.K, I.G, I.Gm);
 }
 
-__global__ __launch_bounds__(kCholNT) void kb_chol_lds(const BInst *__restrict__ tab,
-                                                    const int *__restrict__ list) {
-    const BInst &I = tab[list[blockIdx.x]];
-    if (!I.do_m) return;
-    k_chol_lds_body(0, 0, 0, 1, I.A0, I.A, I.M1, I.ridge, I.scal);
-}
-
-__global__ __launch_bounds__(256) void kb_trsm_lds(const BInst *__restrict__ tab,
-                                                    const int2 *__restrict__ map) {
+__global__ __launch_bounds__(kCholNT) void kb_solve_lds(const BInst *__restrict__ tab,
+                                                        const int2 *__restrict__ map) {
     const int2 m = map[blockIdx.x];
     const BInst &I = tab[m.x];
     if (!I.do_m) return;
-    k_trsm_lds_body(m.y, 0, 0, 0, I.A, I.M1, I.Bm, I.D, I.W, I.scal);
+    k_solve_lds_body(m.y, I.A0, I.M1, I.ridge, I.Bm, I.D, I.W, I.scal);
 }
 
 __global__ __launch_bounds__(1024) void kb_chol_solve(const BInst *__restrict__ tab,
@@ -1324,11 +1281,8 @@ int dg_mstep_run(dg_ctx *c, double jitter) {
     DG_HIP(c, hipGetLastError());
     const double ridge = (c->cfg.lambda > 0.0) ? c->cfg.lambda / c->beta : 0.0;
     if (M1 <= kLdsN) {
-        hipLaunchKernelGGL(k_chol_lds, dim3(1), dim3(kCholNT), 0, c->stream, c->A0, c->A, M1, ridge,
-                           c->scal);
-        DG_HIP(c, hipGetLastError());
-        hipLaunchKernelGGL(k_trsm_lds, dim3((unsigned)bk_cdiv(D, 16)), dim3(256), 0, c->stream, c->A,
-                           M1, c->Bm, D, c->W, c->scal);
+        hipLaunchKernelGGL(k_solve_lds, dim3((unsigned)bk_cdiv(D, 16)), dim3(kCholNT), 0, c->stream,
+                           c->A0, M1, ridge, c->Bm, D, c->W, c->scal);
     } else {
         int rc = blocked_chol_solve(c, ridge, jitter);
         if (rc) return rc;
@@ -1348,7 +1302,7 @@ int dg_mstep_run(dg_ctx *c, double jitter) {
 
 // M-step of the instances in list (n of them; nlds with M + 1 <= 126 first in
 // list, the others after), on one stream; gr holds the flat grids over that
-// list (the LDS triangular solves over its first nlds entries).  Each
+// list (the solves in LDS over its first nlds entries).  Each
 // instance's steps are those of dg_mstep_run.
 int dg_batch_mstep(hipStream_t st, const BInst *tab, const int *list, int n, int nlds,
                    const BGrids &gr) {
@@ -1359,10 +1313,7 @@ int dg_batch_mstep(hipStream_t st, const BInst *tab, const int *list, int n, int
     };
     flat(kb_partAB, BK_PART_AB, 256);
     flat(kb_sumAB, BK_SUM_AB, 256);
-    if (nlds > 0) {
-        hipLaunchKernelGGL(kb_chol_lds, dim3((unsigned)nlds), dim3(kCholNT), 0, st, tab, list);
-        flat(kb_trsm_lds, BK_TRSM_LDS, 256);
-    }
+    if (nlds > 0) flat(kb_solve_lds, BK_SOLVE_LDS, kCholNT);
     if (n > nlds)
         hipLaunchKernelGGL(kb_chol_solve, dim3((unsigned)(n - nlds)), dim3(1024), 0, st, tab,
                            list + nlds);
