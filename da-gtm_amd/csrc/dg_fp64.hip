@@ -856,6 +856,39 @@ __global__ void k_sum_chunks(const double *__restrict__ part, int nc, long len,
     out[i] = s;
 }
 
+// x summed over the wave, the same bits in every lane: rotations within rows of
+// sixteen, then the rows (row_ror and the row swaps cost a few cycles where a
+// shuffle through LDS takes over a hundred).
+template <int ROR>
+__device__ __forceinline__ double add_rotated(double x) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, x);
+    const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)u, 0x120 + ROR, 0xf, 0xf, false);
+    const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(u >> 32), 0x120 + ROR, 0xf, 0xf, false);
+    return x + __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+__device__ __forceinline__ double wave_sum(double x) {
+    x = add_rotated<8>(x);
+    x = add_rotated<4>(x);
+    x = add_rotated<2>(x);
+    x = add_rotated<1>(x);
+    // (each half of a swapped pair is a row's sum: their sum is order-free)
+    auto swapped = [](double y, bool rows32) {
+        const unsigned long long u = __builtin_bit_cast(unsigned long long, y);
+        unsigned a[2], b[2];
+        for (int h = 0; h < 2; ++h) {
+            const unsigned t = h ? (unsigned)(u >> 32) : (unsigned)u;
+            const auto r = rows32 ? __builtin_amdgcn_permlane32_swap(t, t, false, false)
+                                  : __builtin_amdgcn_permlane16_swap(t, t, false, false);
+            a[h] = r[0];
+            b[h] = r[1];
+        }
+        return __builtin_bit_cast(double, ((unsigned long long)a[1] << 32) | a[0]) +
+               __builtin_bit_cast(double, ((unsigned long long)b[1] << 32) | b[0]);
+    };
+    x = swapped(x, false);
+    return swapped(x, true);
+}
+
 // The eigenvalue of one centre's S that the critical temperature takes.  Workgroup
 // (kb, part): of A = sc (2 S1) or sc (2 S1 - 2 S2), n x n, the largest eigenvalue
 // below sc limit, and 0 in the place of those at or above it (comm.c:2149-2161):
@@ -864,7 +897,8 @@ __global__ void k_sum_chunks(const double *__restrict__ part, int nc, long len,
 // Matrix Computations, 4th ed., 8.3.1), and the one eigenvalue wanted is found by
 // Sturm counts (8.4.1) at 64 points of the interval at a time, one per lane.
 // Bound by the chain of reflections (two reductions and a matrix-vector product
-// each).  800 matrices of n = 32 in 180 us, 1216 of n = 166 in 6.1 ms; on 16 host
+// each).  800 matrices of n = 32 in 125 us (178 with shuffled sums, rows loaded one
+// at a time and updated one after the other), 1216 of n = 166 in 5.4 ms (6.1); on 16 host
 // threads, with S to copy there first, the search took 2.7 ms longer at n = 32
 // and 0.2 s at n = 166.
 __global__ __launch_bounds__(256) void k_ctemp_eig(const double *__restrict__ S, int n,
@@ -882,20 +916,28 @@ __global__ __launch_bounds__(256) void k_ctemp_eig(const double *__restrict__ S,
     const double *S1 = S + kb * 2 * n * n, *S2 = S1 + (long)n * n;
     auto at = [&](int i, int j) -> double & { return A[i * (i + 1) / 2 + j]; };   // j <= i
     auto sum = [&](double x) {                     // over the workgroup, in every thread
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
+        x = wave_sum(x);
+        if (nt == 64) return x;
         __syncthreads();                           // the last sum's readers are done
         if (l == 0) red[w] = x;
         __syncthreads();
-        double s = red[0];
-        for (int q = 1; q < nt / 64; ++q) s += red[q];
-        return s;
+        return (red[0] + red[1]) + (red[2] + red[3]);
     };
-    for (int i = w; i < n; i += nt / 64)
-        for (int j = l; j <= i; j += 64) {
-            const double a = 2.0 * S1[(long)i * n + j];
-            at(i, j) = (sub ? a - 2.0 * S2[(long)i * n + j] : a) * sc;
+    for (int e0 = tid; e0 < n * n; e0 += 8 * nt) {  // (eight elements' loads in flight)
+        double a[8], b[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int e = min(e0 + u * nt, n * n - 1);
+            a[u] = S1[e];
+            b[u] = sub ? S2[e] : 0.0;
         }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int e = e0 + u * nt, i = e / n, j = e - i * n;
+            const double x = 2.0 * a[u];
+            if (i < n && j <= i) at(i, j) = (sub ? x - 2.0 * b[u] : x) * sc;
+        }
+    }
     __syncthreads();
     for (int k = 0; k + 2 < n; ++k) {
         // the reflection that annihilates A[k + 2 .., k]: v = x - alpha e1
@@ -914,27 +956,56 @@ __global__ __launch_bounds__(256) void k_ctemp_eig(const double *__restrict__ S,
         }
         for (int i = k + 1 + tid; i < n; i += nt) v[i] = (i == k + 1) ? v0 : at(i, k);
         __syncthreads();
-        // p = 2 A v / vv, then p -= (v.p / vv) v, and A -= v p^T + p v^T
-        double vp = 0.0, pi = 0.0;
-        const int i = k + 1 + tid;                 // n <= 192 rows: one to a thread (or none)
-        for (int i0 = i; i0 < n; i0 += nt) {
-            double q[4] = {0.0, 0.0, 0.0, 0.0};    // (four chains in flight)
-            auto elem = [&](int j) { return j <= i0 ? at(i0, j) : at(j, i0); };
+        // p = 2 A v / vv, then p -= (v.p / vv) v, and A -= v p^T + p v^T; a row of the
+        // product to a thread (n <= nt): a column's elements, T(i) + j of row i, are
+        // in different banks
+        const int i = k + 1 + tid;
+        double vi = 0.0, pi = 0.0;
+        if (i < n) {
+            double q[4] = {0.0, 0.0, 0.0, 0.0};    // (four chains, eight reads in flight)
+            auto elem = [&](int j) { return A[j <= i ? i * (i + 1) / 2 + j : j * (j + 1) / 2 + i]; };
             int j = k + 1;
-            for (; j + 4 <= n; j += 4)
+            for (; j + 8 <= n; j += 8) {
+                double x[8], y[8];
 #pragma unroll
-                for (int u = 0; u < 4; ++u) q[u] = fma(elem(j + u), v[j + u], q[u]);
+                for (int u = 0; u < 8; ++u) { x[u] = elem(j + u); y[u] = v[j + u]; }
+#pragma unroll
+                for (int u = 0; u < 8; ++u) q[u & 3] = fma(x[u], y[u], q[u & 3]);
+            }
             for (; j < n; ++j) q[0] = fma(elem(j), v[j], q[0]);
             pi = 2.0 * ((q[0] + q[1]) + (q[2] + q[3])) / vv;
-            p[i0] = pi;
-            vp = fma(v[i0], pi, vp);
+            vi = v[i];
         }
-        const double c = sum(vp) / vv;
-        for (int i0 = i; i0 < n; i0 += nt) p[i0] -= c * v[i0];
+        const double c = sum(vi * pi) / vv;
+        pi -= c * vi;
+        if (i < n) p[i] = pi;
         __syncthreads();
-        for (int r = k + 1 + w; r < n; r += nt / 64) {
-            const double vr = v[r], pr = p[r];
-            for (int j = k + 1 + l; j <= r; j += 64) at(r, j) -= vr * p[j] + pr * v[j];
+        // the update: a row to a lane where one wave has them all (n = 32: 125 us, 154
+        // with lanes along the rows, one row after the other; n = 64: 359 and 473),
+        // else lanes along the rows (n = 166: 5.4 ms, and 6.4)
+        if (nt == 64) {
+            if (i < n) {
+                double *row = A + i * (i + 1) / 2;
+                int j = k + 1;
+                for (; j + 8 <= n && __any(j <= i); j += 8) {
+                    double x[8], y[8], z[8];
+    #pragma unroll
+                    for (int u = 0; u < 8; ++u) {
+                        x[u] = row[min(j + u, i)];
+                        y[u] = p[j + u];
+                        z[u] = v[j + u];
+                    }
+    #pragma unroll
+                    for (int u = 0; u < 8; ++u)
+                        if (j + u <= i) row[j + u] = x[u] - (vi * y[u] + pi * z[u]);
+                }
+                for (; j <= i; ++j) row[j] -= vi * p[j] + pi * v[j];
+            }
+        } else {
+            for (int r = k + 1 + w; r < n; r += nt / 64) {
+                const double vr = v[r], pr = p[r];
+                for (int j = k + 1 + l; j <= r; j += 64) at(r, j) -= vr * p[j] + pr * v[j];
+            }
         }
         __syncthreads();
     }
