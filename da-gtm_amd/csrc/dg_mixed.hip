@@ -1364,24 +1364,57 @@ __device__ __forceinline__ double pow2_scale(double amax) {
 
 // Split T (N x D, stride ldt) into FP16 terms: T16[t][n][d], d < ld16, with
 // rows n >= N and columns d >= D zero; tt32[n] = |t'|^2 of the split value.
-// Row n holds input row perm[n] (row n when perm is null).
-__global__ void k_make_t16(const double *__restrict__ T64, int ldt, long N, long Np, int D,
-                           int ld16, int TT, double scale, const int *__restrict__ perm,
-                           _Float16 *__restrict__ T16, float *__restrict__ tt32) {
-    const long n = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= Np) return;
-    const long src = (n < N && perm) ? (long)perm[n] : n;      // input row of point n
-    double ss = 0.0;
-    for (int d = 0; d < ld16; ++d) {
-        const double v = (n < N && d < D) ? T64[src * ldt + d] * scale : 0.0;
-        const _Float16 hi = (_Float16)(float)v;
-        const _Float16 lo = (TT == 2) ? (_Float16)(float)(v - (double)(float)hi) : (_Float16)0.0f;
-        T16[n * ld16 + d] = hi;
-        if (TT == 2) T16[(Np + n) * ld16 + d] = lo;
-        const double rep = ((double)(float)hi + (double)(float)lo) / scale;
-        ss = fma(rep, rep, ss);
+// Row n holds input row perm[n] (row n when perm is null).  A thread per row, whose
+// norm is a chain in d; the rows come through LDS sixteen columns at a time (whole
+// cache lines) and leave as 32-byte runs.  Bound by memory: N = 10^6, D = 166:
+// 4.7 -> 0.56 ms, N = 16000: 47 -> 27 us (rows straight from and to memory, an element
+// at a time).
+constexpr int kT16Rows = 64;
+__global__ __launch_bounds__(kT16Rows) void k_make_t16(
+    const double *__restrict__ T64, int ldt, long N, long Np, int D, int ld16, int TT, double scale,
+    const int *__restrict__ perm, _Float16 *__restrict__ T16, float *__restrict__ tt32) {
+    typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+    __shared__ double buf[kT16Rows][17];
+    __shared__ long rows[kT16Rows];
+    const int tid = threadIdx.x, c = tid & 15;
+    const long n0 = (long)blockIdx.x * kT16Rows, n = n0 + tid;
+    rows[tid] = (n < N && perm) ? (long)perm[n] : n;          // input row of point n
+    __syncthreads();
+    const double inv = 1.0 / scale;                // (a power of two)
+    double ss = 0.0, v[16];
+    auto load = [&](int d0) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int r = 4 * i + (tid >> 4);
+            v[i] = (n0 + r < N && d0 + c < D) ? T64[rows[r] * ldt + d0 + c] : 0.0;
+        }
+    };
+    load(0);
+    for (int d0 = 0; d0 < ld16; d0 += 16) {
+        __syncthreads();                           // the last columns are read
+#pragma unroll
+        for (int i = 0; i < 16; ++i) buf[4 * i + (tid >> 4)][c] = v[i] * scale;
+        __syncthreads();
+        if (d0 + 16 < ld16) load(d0 + 16);
+        h8 hi[2], lo[2];
+#pragma unroll
+        for (int d = 0; d < 16; ++d) {
+            const double x = buf[tid][d];
+            const _Float16 h = (_Float16)(float)x;
+            const _Float16 e = (TT == 2) ? (_Float16)(float)(x - (double)(float)h) : (_Float16)0.0f;
+            hi[d >> 3][d & 7] = h;
+            lo[d >> 3][d & 7] = e;
+            const double rep = ((double)(float)h + (double)(float)e) * inv;
+            ss = fma(rep, rep, ss);
+        }
+        if (n >= Np) continue;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            *(h8 *)(T16 + n * ld16 + d0 + 8 * i) = hi[i];
+            if (TT == 2) *(h8 *)(T16 + (Np + n) * ld16 + d0 + 8 * i) = lo[i];
+        }
     }
-    tt32[n] = (float)ss;
+    if (n < Np) tt32[n] = (float)ss;
 }
 
 // Transposed data, chunk-major: for point n in chunk c = n / CL (offset
@@ -1457,27 +1490,36 @@ __global__ __launch_bounds__(256) void k_make_y16(const double *__restrict__ Y64
 // Nearest centre of each point from the first FP16 terms (an ordering key,
 // not a result): key[n] = argmax_k (t'_n . y'_k - s |y'_k|^2 / 2), s the
 // product of the two power-of-two operand scales (mscal[0] for Y, mscal[1]
-// for T), first k on ties.  One thread per point with its row in registers as
-// FP16 pairs (v_dot2_f32_f16); the centres pass through LDS 32 at a time.
+// for T), first k on ties.  A lane holds two points' rows in registers as FP16
+// pairs (v_dot2_f32_f16), so that each LDS read of a centre serves both: read for
+// one point they take twice the dot products' time.  The centres pass through LDS
+// 32 at a time, a quarter of them to each of the four waves, which have the same
+// 128 points, four centres' chains in flight.
+// Bound by the dot products' issue.  N = 100000, K = 8000, D = 166: 6.8 -> 4.1 ms;
+// N = 16000, K = 400: 357 -> 96 us (a point per thread, one chain).
+constexpr int kNearPts = 128;        // points per workgroup
 template <int KS>
-__global__ __launch_bounds__(256) void k_nearest(const _Float16 *__restrict__ T16, long N,
-                                                 const _Float16 *__restrict__ Y16,
-                                                 const float *__restrict__ yy32, int K,
-                                                 const double *__restrict__ mscal,
-                                                 int *__restrict__ key) {
+__global__ __launch_bounds__(256, 2) void k_nearest(const _Float16 *__restrict__ T16, long N,
+                                                    const _Float16 *__restrict__ Y16,
+                                                    const float *__restrict__ yy32, int K,
+                                                    const double *__restrict__ mscal,
+                                                    int *__restrict__ key) {
     constexpr int ld = 16 * KS, NPR = ld / 2, CTL = 32;
-    __shared__ h2 ys[CTL][NPR];
+    __shared__ __attribute__((aligned(16))) h2 ys[CTL][NPR];
     __shared__ float ysq[CTL];
-    const long n = (long)blockIdx.x * 256 + threadIdx.x;
-    h2 t[NPR];
+    __shared__ float bv[4][kNearPts];
+    __shared__ int bi[4][kNearPts];
+    const int l = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const long n0 = (long)blockIdx.x * kNearPts + l;
+    h2 t[2][NPR];
 #pragma unroll
-    for (int p = 0; p < NPR; ++p) {
-        const h2 z = {(_Float16)0.0f, (_Float16)0.0f};
-        t[p] = (n < N) ? *(const h2 *)(T16 + n * ld + 2 * p) : z;
-    }
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int p = 0; p < NPR; ++p)
+            t[q][p] = *(const h2 *)(T16 + min(n0 + 64 * q, N - 1) * ld + 2 * p);
     const float s = (float)(0.5 * mscal[0] * mscal[1]);
-    float best = -INFINITY;
-    int bk = 0;
+    float best[2] = {-INFINITY, -INFINITY};
+    int bk[2] = {0, 0};
     for (int k0 = 0; k0 < K; k0 += CTL) {
         __syncthreads();
         for (int e = threadIdx.x; e < CTL * NPR; e += 256) {
@@ -1487,15 +1529,39 @@ __global__ __launch_bounds__(256) void k_nearest(const _Float16 *__restrict__ T1
         }
         if (threadIdx.x < CTL) ysq[threadIdx.x] = (k0 + (int)threadIdx.x < K) ? s * yy32[k0 + threadIdx.x] : INFINITY;
         __syncthreads();
-        for (int r = 0; r < CTL; ++r) {
-            float acc = 0.f;
+#pragma unroll 1
+        for (int r = 8 * w; r < 8 * w + 8; r += 4) {
+            float acc[4][2] = {};
 #pragma unroll
-            for (int p = 0; p < NPR; ++p) acc = __builtin_amdgcn_fdot2(t[p], ys[r][p], acc, false);
-            const float v = acc - ysq[r];
-            if (v > best) { best = v; bk = k0 + r; }
+            for (int p = 0; p < NPR; ++p)
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+#pragma unroll
+                    for (int q = 0; q < 2; ++q)
+                        acc[u][q] = __builtin_amdgcn_fdot2(t[q][p], ys[r + u][p], acc[u][q], false);
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    const float v = acc[u][q] - ysq[r + u];
+                    if (v > best[q]) { best[q] = v; bk[q] = k0 + r + u; }
+                }
         }
     }
-    if (n < N) key[n] = bk;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) { bv[w][l + 64 * q] = best[q]; bi[w][l + 64 * q] = bk[q]; }
+    __syncthreads();
+    const long n = (long)blockIdx.x * kNearPts + threadIdx.x;
+    if (threadIdx.x >= kNearPts || n >= N) return;
+    float b = bv[0][threadIdx.x];
+    int k = bi[0][threadIdx.x];
+#pragma unroll
+    for (int x = 1; x < 4; ++x) {                  // the first k of the largest
+        const float v = bv[x][threadIdx.x];
+        const int i = bi[x][threadIdx.x];
+        if (v > b || (v == b && i < k)) { b = v; k = i; }
+    }
+    key[n] = k;
 }
 
 // Supported numbers of 16-wide d steps (D is padded up to the next one).
@@ -1943,9 +2009,9 @@ int dg_mixed_pass2_blocks(dg_ctx *c, long *visited, long *total) {
 int build_t16(dg_ctx *c, MixedBufs *b) {
     const int ld16 = c->ldh;
     const int DR = 32 * ((ld16 + 31) / 32);
-    hipLaunchKernelGGL(k_make_t16, dim3((unsigned)((b->Np + 255) / 256)), dim3(256), 0, c->stream,
-                       c->T64, c->ldt, c->N, b->Np, c->D, ld16, b->TT, (double)c->t_scale,
-                       c->perm, (_Float16 *)c->T16, c->tt32);
+    hipLaunchKernelGGL(k_make_t16, dim3((unsigned)((b->Np + kT16Rows - 1) / kT16Rows)),
+                       dim3(kT16Rows), 0, c->stream, c->T64, c->ldt, c->N, b->Np, c->D, ld16, b->TT,
+                       (double)c->t_scale, c->perm, (_Float16 *)c->T16, c->tt32);
     DG_HIP(c, hipGetLastError());
     hipLaunchKernelGGL(k_transpose16,
                        dim3((unsigned)((b->Np + 63) / 64), (unsigned)((DR + 63) / 64),
@@ -2049,7 +2115,7 @@ int dg_mixed_order(dg_ctx *c) {
     int *dkey = nullptr;
     int rc;
     if ((rc = dalloc(c, &dkey, (size_t)N))) return rc;
-    const unsigned grid = (unsigned)((N + 255) / 256);
+    const unsigned grid = (unsigned)((N + kNearPts - 1) / kNearPts);
     auto go = [&](auto ks) {
         constexpr int KS = decltype(ks)::value;
         hipLaunchKernelGGL((k_nearest<KS>), dim3(grid), dim3(256), 0, c->stream,
