@@ -158,7 +158,8 @@ __host__ __device__ inline int bk_count(const BInst &I, int kind) {
         case BK_REDUCE32: return cdiv(I.K, kBRK) * (I.D / kBRD + 1);   // D rows of R T, one of G
         case BK_ZERO_FIX: return I.D;
         case BK_PART_AB:
-            return cdiv(I.M1, dg_ab_tile(I.M1)) * cdiv(I.M1 + I.D, dg_ab_tile(I.M1)) * I.nchAB;
+            return cdiv(I.M1, dg_ab_tile(I.M1)) *
+                   (cdiv(I.M1, dg_ab_tile(I.M1)) + cdiv(I.D, dg_ab_tile(I.M1))) * I.nchAB;
         case BK_SUM_AB: return cdiv((long)I.M1 * I.M1 + (long)I.M1 * I.D, 256) + cdiv(I.K, 256);
         case BK_SOLVE_LDS: return cdiv(I.D, 16);
         case BK_CENTRES: return cdiv(I.K, kBCentres);

@@ -171,48 +171,44 @@ __device__ __forceinline__ d4 mfma64(double a, double b, d4 c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
-// A tile of [A | B] holds nothing that is read: all of it above A's diagonal
-// (the factorisation takes the lower triangle).
-__device__ __forceinline__ bool upper_tile(int ti, int tj, int M1) {
-    return tj > ti && (tj + 1) * dg_ab_tile(M1) <= M1;
-}
+// Blocks (bi, bj) of half a tile's edge above A's diagonal: the factorisation takes
+// the lower triangle, and nothing computes or reads them.
+__device__ __forceinline__ bool upper_block(int bi, int bj) { return bj > bi; }
 
 // Split-K partials of [A | B] = FI^T [diag(G) FI | RT], an M1 x (M1 + D)
-// product over the centres: workgroup (bx, by, c) computes one output tile
-// over centres [c kc, min(K, (c + 1) kc)); part is nch x M1 x (M1 + D).  A wave
-// takes a quarter of it (16 RB x 16 RB) straight from global memory, where a row
-// of FI or RT is a run of whole cache lines; 4 U centres are multiplied while the
-// next ones are on their way.  dg_ab_tile chooses 64 x 64 tiles (RB = 2), which
+// product over the centres: workgroup (bx, by, c) computes one output tile (A's
+// tile columns first, then B's) over centres [c kc, min(K, (c + 1) kc)); part is
+// nch x M1 x (M1 + D).  A wave takes a quarter of it (16 RB x 16 RB), if that has
+// anything below the diagonal, straight from global memory, where a row of FI or RT
+// is a run of whole cache lines; 4 U centres are multiplied while the next ones are
+// on their way.  dg_ab_tile chooses 64 x 64 tiles (RB = 2), which
 // spread a small M1 over the chip, or for M1 > 256 128 x 128 (RB = 4), whose
 // operands take half as much of L2's rate: at M1 = 1001 it bound the small ones.
-// FP64 pipe: K = 32768, M1 = 1001, D = 166: 3043 -> 1410 us (64 x 64: 2100);
-// K = 8000, M1 = 126: 41 -> 28 us (4 x 4 register tiles of FMAs from LDS, and
-// A's upper half computed too).
+// K = 32768, M1 = 1001, D = 166: 3043 -> 1261 us (64 x 64 tiles: 2100; with B's
+// columns in A's last tile and whole diagonal tiles, 1385); K = 8000, M1 = 126: 41 ->
+// 27 us (4 x 4 register tiles of FMAs from LDS, and A's upper half computed too).
 template <int RB>
 __device__ __forceinline__ void k_partAB_body(
     const int bx, const int by, const int bz, const int gx, const double *__restrict__ FI,
     const double *__restrict__ G, const double *__restrict__ RT, int K, int M1, int D, int kc,
     double *__restrict__ part) {
-    if (upper_tile(bx, by, M1)) return;
-    const int NCOL = M1 + D;
+    const int NCOL = M1 + D, nA = bk_cdiv(M1, 32 * RB);
+    const bool isB = by >= nA;
     const int c = bz;
     const int k0 = c * kc, k1 = (k0 + kc < K) ? k0 + kc : K;
     const int l = threadIdx.x & 63, w = threadIdx.x >> 6, j = l & 15, g = l >> 4;
-    const int i0 = 16 * RB * (2 * bx + (w & 1)), j0 = 16 * RB * (2 * by + (w >> 1));
+    const int bi = 2 * bx + (w & 1), bj = 2 * (isB ? by - nA : by) + (w >> 1);
+    const int i0 = 16 * RB * bi, j0 = 16 * RB * bj, ncol = isB ? D : M1;
     const long E = (long)M1 * NCOL;
-    if (i0 >= M1 || j0 >= NCOL) return;
+    if (i0 >= M1 || j0 >= ncol || (!isB && upper_block(bi, bj))) return;
     // per lane: its columns of A's operand and of B's at centre k0 + g (past the
     // end: the last ones again, whose results are not stored), moved on by adds
-    const double *pa[RB], *pb[RB], *pg = G + k0 + g;
-    long sb[RB];
-    bool wg[RB];
+    const double *pa[RB], *pb[RB], *pg = G + k0 + g, *R = isB ? RT : FI;
+    const long sb = 4L * ncol;
 #pragma unroll
     for (int x = 0; x < RB; ++x) {
         pa[x] = FI + (long)(k0 + g) * M1 + min(i0 + 16 * x + j, M1 - 1);
-        const int col = min(j0 + 16 * x + j, NCOL - 1);
-        wg[x] = col < M1;
-        sb[x] = 4 * (wg[x] ? M1 : D);
-        pb[x] = wg[x] ? FI + (long)(k0 + g) * M1 + col : RT + (long)(k0 + g) * D + (col - M1);
+        pb[x] = R + (long)(k0 + g) * ncol + min(j0 + 16 * x + j, ncol - 1);
     }
     constexpr int U = RB == 2 ? 4 : 2;
     double ra[U][RB], rb[U][RB], rg[U];
@@ -227,7 +223,7 @@ __device__ __forceinline__ void k_partAB_body(
                 ra[u][x] = in ? *pa[x] : 0.0;
                 rb[u][x] = in ? *pb[x] : 0.0;
                 pa[x] += 4L * M1;
-                pb[x] += sb[x];
+                pb[x] += sb;
             }
         }
     };
@@ -248,7 +244,7 @@ __device__ __forceinline__ void k_partAB_body(
 #pragma unroll
             for (int x = 0; x < RB; ++x) {
                 av[u][x] = ra[u][x];
-                bv[u][x] = wg[x] ? rg[u] * rb[u][x] : rb[u][x];
+                bv[u][x] = isB ? rb[u][x] : rg[u] * rb[u][x];
             }
         next(kb + 4 * U);
 #pragma unroll
@@ -265,7 +261,8 @@ __device__ __forceinline__ void k_partAB_body(
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int i = i0 + 16 * x + 4 * r + g, jj = j0 + 16 * y + j;
-                if (i < M1 && jj < NCOL) part[(long)c * E + (long)i * NCOL + jj] = acc[x][y][r];
+                if (i < M1 && jj < ncol)
+                    part[(long)c * E + (long)i * NCOL + (isB ? M1 : 0) + jj] = acc[x][y][r];
             }
 }
 
@@ -277,12 +274,12 @@ __global__ __launch_bounds__(256, 2) void k_partAB(const double *__restrict__ FI
                                                    const double *__restrict__ RT, int K, int M1,
                                                    int D, int kc, int nch,
                                                    double *__restrict__ part) {
-    const int nx = (M1 + 32 * RB - 1) / (32 * RB), ny = (M1 + D + 32 * RB - 1) / (32 * RB);
+    const int nx = bk_cdiv(M1, 32 * RB), ny = nx + bk_cdiv(D, 32 * RB);
     const int i = blockIdx.x >> 3, tile = i % (nx * ny), c = i / (nx * ny) * 8 + (blockIdx.x & 7);
     if (c < nch) k_partAB_body<RB>(tile % nx, tile / nx, c, 0, FI, G, RT, K, M1, D, kc, part);
 }
 
-// A0 / B from the chunk partials, summed in chunk order (A0 without the tiles
+// A0 / B from the chunk partials, summed in chunk order (A0 without the blocks
 // that k_partAB leaves out); the workgroups after those copy G to Gm, which the
 // critical-temperature search reads (vggsub of dagtm.cxx:1715, still set when
 // the next E-step converges).
@@ -301,7 +298,8 @@ __device__ __forceinline__ void k_sumAB_body(
     }
     if (e >= E) return;
     const int i = (int)(e / NCOL), j = (int)(e % NCOL);
-    if (j < M1 && upper_tile(i / dg_ab_tile(M1), j / dg_ab_tile(M1), M1)) return;
+    const int half = dg_ab_tile(M1) / 2;
+    if (j < M1 && upper_block(i / half, j / half)) return;
     // eight loads in flight, then their sums in chunk order
     double s = 0.0;
     int c = 0;
@@ -1148,7 +1146,7 @@ __global__ __launch_bounds__(256, 2) void kb_partAB(const BInst *__restrict__ ta
     const int2 m = map[blockIdx.x];
     const BInst &I = tab[m.x];
     if (!I.do_m) return;
-    const int t = dg_ab_tile(I.M1), nx = bk_cdiv(I.M1, t), ny = bk_cdiv(I.M1 + I.D, t);
+    const int t = dg_ab_tile(I.M1), nx = bk_cdiv(I.M1, t), ny = nx + bk_cdiv(I.D, t);
     const int kc = (I.K + I.nchAB - 1) / I.nchAB;
     const int x = m.y % nx, y = (m.y / nx) % ny, z = m.y / (nx * ny);
     if (t == 64) k_partAB_body<2>(x, y, z, 0, I.FI, I.G, I.RT, I.K, I.M1, I.D, kc, I.partAB);
@@ -1268,7 +1266,8 @@ int dg_mstep_run(dg_ctx *c, double jitter) {
     const int nch = c->nchAB;
     const int kc = (K + nch - 1) / nch;
     const int t = dg_ab_tile(M1);
-    const dim3 abgrid((unsigned)(8 * bk_cdiv(M1, t) * bk_cdiv(M1 + D, t) * bk_cdiv(nch, 8)));
+    const int nx = bk_cdiv(M1, t);
+    const dim3 abgrid((unsigned)(8 * nx * (nx + bk_cdiv(D, t)) * bk_cdiv(nch, 8)));
     if (t == 64)
         hipLaunchKernelGGL(k_partAB<2>, abgrid, dim3(256), 0, c->stream, c->FI, c->G, c->RT, K, M1, D,
                            kc, nch, c->partAB);
