@@ -147,8 +147,12 @@ struct BInst {
 
 __host__ __device__ inline int bk_cdiv(long a, long b) { return (int)((a + b - 1) / b); }
 
-// edge of k_partAB's output tiles
-__host__ __device__ inline int dg_ab_tile(int M1) { return M1 > 256 ? 128 : 64; }
+// k_partAB's output blocks: their edge, and how many there are
+__host__ __device__ inline int dg_ab_edge(int M1) { return M1 > 256 ? 64 : 32; }
+__host__ __device__ inline int dg_ab_blocks(int M1, int D) {
+    const int e = dg_ab_edge(M1), nA = bk_cdiv(M1, e);
+    return nA * (nA + 1) / 2 + nA * bk_cdiv(D, e);
+}
 
 // workgroups of instance I in the flat grid of a kind
 __host__ __device__ inline int bk_count(const BInst &I, int kind) {
@@ -157,9 +161,7 @@ __host__ __device__ inline int bk_count(const BInst &I, int kind) {
         case BK_MAKE_AK: return cdiv(I.Kp, 256);
         case BK_REDUCE32: return cdiv(I.K, kBRK) * (I.D / kBRD + 1);   // D rows of R T, one of G
         case BK_ZERO_FIX: return I.D;
-        case BK_PART_AB:
-            return cdiv(I.M1, dg_ab_tile(I.M1)) *
-                   (cdiv(I.M1, dg_ab_tile(I.M1)) + cdiv(I.D, dg_ab_tile(I.M1))) * I.nchAB;
+        case BK_PART_AB: return cdiv(dg_ab_blocks(I.M1, I.D), 4) * I.nchAB;
         case BK_SUM_AB: return cdiv((long)I.M1 * I.M1 + (long)I.M1 * I.D, 256) + cdiv(I.K, 256);
         case BK_SOLVE_LDS: return cdiv(I.D, 16);
         case BK_CENTRES: return cdiv(I.K, kBCentres);

@@ -171,36 +171,39 @@ __device__ __forceinline__ d4 mfma64(double a, double b, d4 c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
-// Blocks (bi, bj) of half a tile's edge above A's diagonal: the factorisation takes
-// the lower triangle, and nothing computes or reads them.
-__device__ __forceinline__ bool upper_block(int bi, int bj) { return bj > bi; }
-
 // Split-K partials of [A | B] = FI^T [diag(G) FI | RT], an M1 x (M1 + D)
-// product over the centres: workgroup (bx, by, c) computes one output tile (A's
-// tile columns first, then B's) over centres [c kc, min(K, (c + 1) kc)); part is
-// nch x M1 x (M1 + D).  A wave takes a quarter of it (16 RB x 16 RB), if that has
-// anything below the diagonal, straight from global memory, where a row of FI or RT
-// is a run of whole cache lines; 4 U centres are multiplied while the next ones are
-// on their way.  dg_ab_tile chooses 64 x 64 tiles (RB = 2), which
-// spread a small M1 over the chip, or for M1 > 256 128 x 128 (RB = 4), whose
-// operands take half as much of L2's rate: at M1 = 1001 it bound the small ones.
-// K = 32768, M1 = 1001, D = 166: 3043 -> 1261 us (64 x 64 tiles: 2100; with B's
-// columns in A's last tile and whole diagonal tiles, 1385); K = 8000, M1 = 126: 41 ->
-// 27 us (4 x 4 register tiles of FMAs from LDS, and A's upper half computed too).
+// product over the centres, part being nch x M1 x (M1 + D).  A wave computes one
+// 16 RB x 16 RB block, number b of the dg_ab_blocks(M1, D) (A's lower triangle row by
+// row: the factorisation takes no more; then B's), over centres [c kc, min(K,
+// (c + 1) kc)), straight from global memory, where a row of FI or RT is a run of
+// whole cache lines; 4 U centres are multiplied while the next ones are on their
+// way.  dg_ab_edge chooses 32 x 32 blocks (RB = 2), which spread a small M1 over the
+// chip, or for M1 > 256 64 x 64 (RB = 4), whose operands take half as much of L2's
+// rate: at M1 = 1001 it bound the small ones.
+// FP64 pipe.  K = 32768, M1 = 1001, D = 166: 3043 -> 1014 us (32 x 32 blocks: 2100;
+// four blocks of a 128 x 128 tile to a workgroup, some of them above the diagonal or
+// past the end, 1261: a wave runs for 150 us, and the last round left CUs idle for a
+// fifth of the time); K = 8000, M1 = 126: 41 -> 27 us (4 x 4 register tiles of FMAs
+// from LDS, and A's upper half computed too).
 template <int RB>
 __device__ __forceinline__ void k_partAB_body(
-    const int bx, const int by, const int bz, const int gx, const double *__restrict__ FI,
-    const double *__restrict__ G, const double *__restrict__ RT, int K, int M1, int D, int kc,
-    double *__restrict__ part) {
-    const int NCOL = M1 + D, nA = bk_cdiv(M1, 32 * RB);
-    const bool isB = by >= nA;
-    const int c = bz;
+    const int b, const int c, const double *__restrict__ FI, const double *__restrict__ G,
+    const double *__restrict__ RT, int K, int M1, int D, int kc, double *__restrict__ part) {
+    const int NCOL = M1 + D, nA = bk_cdiv(M1, 16 * RB), tri = nA * (nA + 1) / 2;
+    const bool isB = b >= tri;
+    int bi = 0, bj = b;
+    if (isB) {
+        const int nB = bk_cdiv(D, 16 * RB);
+        bi = (b - tri) / nB;
+        bj = (b - tri) % nB;
+    } else {
+        while (bj > bi) bj -= ++bi;
+    }
+    if (bi >= nA) return;
     const int k0 = c * kc, k1 = (k0 + kc < K) ? k0 + kc : K;
-    const int l = threadIdx.x & 63, w = threadIdx.x >> 6, j = l & 15, g = l >> 4;
-    const int bi = 2 * bx + (w & 1), bj = 2 * (isB ? by - nA : by) + (w >> 1);
+    const int l = threadIdx.x & 63, j = l & 15, g = l >> 4;
     const int i0 = 16 * RB * bi, j0 = 16 * RB * bj, ncol = isB ? D : M1;
     const long E = (long)M1 * NCOL;
-    if (i0 >= M1 || j0 >= ncol || (!isB && upper_block(bi, bj))) return;
     // per lane: its columns of A's operand and of B's at centre k0 + g (past the
     // end: the last ones again, whose results are not stored), moved on by adds
     const double *pa[RB], *pb[RB], *pg = G + k0 + g, *R = isB ? RT : FI;
@@ -266,17 +269,20 @@ __device__ __forceinline__ void k_partAB_body(
             }
 }
 
-// The hardware hands workgroup i to XCD i mod 8: all tiles of a chunk go to one
+// The hardware hands workgroup i to XCD i mod 8: all blocks of a chunk go to one
 // XCD, whose L2 then holds the chunk's rows (4.7 MB at M1 = 1001, kc = 512).
-template <int RB>
-__global__ __launch_bounds__(256, 2) void k_partAB(const double *__restrict__ FI,
-                                                   const double *__restrict__ G,
-                                                   const double *__restrict__ RT, int K, int M1,
-                                                   int D, int kc, int nch,
-                                                   double *__restrict__ part) {
-    const int nx = bk_cdiv(M1, 32 * RB), ny = nx + bk_cdiv(D, 32 * RB);
-    const int i = blockIdx.x >> 3, tile = i % (nx * ny), c = i / (nx * ny) * 8 + (blockIdx.x & 7);
-    if (c < nch) k_partAB_body<RB>(tile % nx, tile / nx, c, 0, FI, G, RT, K, M1, D, kc, part);
+// W waves to a workgroup: two where blocks are few (M1 = 65: 7.7 us, four 9.4), four
+// of the large ones, which share lines in L1 (M1 = 1001: 1011 us; one 1021).
+template <int RB, int W>
+__global__ __launch_bounds__(64 * W, 2) void k_partAB(const double *__restrict__ FI,
+                                                      const double *__restrict__ G,
+                                                      const double *__restrict__ RT, int K, int M1,
+                                                      int D, int kc, int nch,
+                                                      double *__restrict__ part) {
+    const int nw = bk_cdiv(dg_ab_blocks(M1, D), W), i = blockIdx.x >> 3;
+    const int c = i / nw * 8 + (blockIdx.x & 7);
+    const int b = i % nw * W + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    if (c < nch) k_partAB_body<RB>(b, c, FI, G, RT, K, M1, D, kc, part);
 }
 
 // A0 / B from the chunk partials, summed in chunk order (A0 without the blocks
@@ -298,8 +304,8 @@ __device__ __forceinline__ void k_sumAB_body(
     }
     if (e >= E) return;
     const int i = (int)(e / NCOL), j = (int)(e % NCOL);
-    const int half = dg_ab_tile(M1) / 2;
-    if (j < M1 && upper_block(i / half, j / half)) return;
+    const int edge = dg_ab_edge(M1);
+    if (j < M1 && j / edge > i / edge) return;     // (above A's lower blocks)
     // eight loads in flight, then their sums in chunk order
     double s = 0.0;
     int c = 0;
@@ -1146,11 +1152,10 @@ __global__ __launch_bounds__(256, 2) void kb_partAB(const BInst *__restrict__ ta
     const int2 m = map[blockIdx.x];
     const BInst &I = tab[m.x];
     if (!I.do_m) return;
-    const int t = dg_ab_tile(I.M1), nx = bk_cdiv(I.M1, t), ny = nx + bk_cdiv(I.D, t);
-    const int kc = (I.K + I.nchAB - 1) / I.nchAB;
-    const int x = m.y % nx, y = (m.y / nx) % ny, z = m.y / (nx * ny);
-    if (t == 64) k_partAB_body<2>(x, y, z, 0, I.FI, I.G, I.RT, I.K, I.M1, I.D, kc, I.partAB);
-    else k_partAB_body<4>(x, y, z, 0, I.FI, I.G, I.RT, I.K, I.M1, I.D, kc, I.partAB);
+    const int kc = (I.K + I.nchAB - 1) / I.nchAB, nw = bk_cdiv(dg_ab_blocks(I.M1, I.D), 4);
+    const int b = m.y % nw * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), c = m.y / nw;
+    if (dg_ab_edge(I.M1) == 32) k_partAB_body<2>(b, c, I.FI, I.G, I.RT, I.K, I.M1, I.D, kc, I.partAB);
+    else k_partAB_body<4>(b, c, I.FI, I.G, I.RT, I.K, I.M1, I.D, kc, I.partAB);
 }
 
 __global__ __launch_bounds__(256) void kb_sumAB(const BInst *__restrict__ tab, const int2 *__restrict__ map) {
@@ -1265,15 +1270,14 @@ int dg_mstep_run(dg_ctx *c, double jitter) {
     const long E = (long)M1 * M1 + (long)M1 * D;
     const int nch = c->nchAB;
     const int kc = (K + nch - 1) / nch;
-    const int t = dg_ab_tile(M1);
-    const int nx = bk_cdiv(M1, t);
-    const dim3 abgrid((unsigned)(8 * nx * (nx + bk_cdiv(D, t)) * bk_cdiv(nch, 8)));
-    if (t == 64)
-        hipLaunchKernelGGL(k_partAB<2>, abgrid, dim3(256), 0, c->stream, c->FI, c->G, c->RT, K, M1, D,
-                           kc, nch, c->partAB);
-    else
-        hipLaunchKernelGGL(k_partAB<4>, abgrid, dim3(256), 0, c->stream, c->FI, c->G, c->RT, K, M1, D,
-                           kc, nch, c->partAB);
+    const int nblk = dg_ab_blocks(M1, D);
+    auto ab = [&](auto kernel, int w) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(8 * bk_cdiv(nblk, w) * bk_cdiv(nch, 8))),
+                           dim3(64 * w), 0, c->stream, c->FI, c->G, c->RT, K, M1, D, kc, nch,
+                           c->partAB);
+    };
+    if (dg_ab_edge(M1) == 32) ab(k_partAB<2, 2>, 2);
+    else ab(k_partAB<4, 4>, 4);
     DG_HIP(c, hipGetLastError());
     hipLaunchKernelGGL(k_sumAB, dim3((unsigned)(bk_cdiv(E, 256) + bk_cdiv(K, 256))), dim3(256), 0,
                        c->stream, c->partAB, nch, M1, D, c->A0, c->Bm, K, c->G, c->Gm);
