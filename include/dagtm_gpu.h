@@ -204,8 +204,8 @@ int dg_anneal_ctl(const dg_anneal_params *p, dg_hda_state *hda, const dg_anneal_
  *             (vggsub, dagtm.cxx:1715 and 1922)
  *   ctemp_k   K outputs, may be NULL
  * R is the responsibility matrix of the last dg_estep (which must be at the
- * current state), computed in FP64 in both precisions.  Cost O(K N D^2) on
- * the device plus 2K symmetric D x D eigenvalue problems on the host. */
+ * current state), computed in FP64 in both precisions.  Cost O(K N D^2) and
+ * 2K symmetric D x D eigenvalue problems, all on the device. */
 int dg_next_ctemp(dg_ctx *ctx, double temp, double eps, const double *gg,
                   double *ctemp_max, double *ctemp_k);
 
