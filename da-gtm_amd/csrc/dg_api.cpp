@@ -630,16 +630,16 @@ static int next_ctemp_impl(dg_ctx *c, double temp, double eps, const double *gg,
         DG_HIP(c, hipStreamSynchronize(c->stream));
     }
     // per centre: eig(H) of mpicomm.c:599-626 with H = [[2S1 - S2, -S2], [-S2, 2S1 - S2]]
-    // is eig(2 S1) together with eig(2 S1 - 2 S2) (H is block-symmetric).  A
-    // centre of hardly any weight has its matrices scaled up (mpicomm.c:617-628).
-    const double GG_MIN = 1e-250;
+    // is eig(2 S1) together with eig(2 S1 - 2 S2) (H is block-symmetric).  The
+    // kernel scales each matrix by its size (mpicomm.c:617-628 does below a weight
+    // of 1e-250).
     const DgCtempPlan p = dg_ctemp_plan(c);
     std::vector<double> lim((size_t)2 * K), val((size_t)2 * K);
     for (int k0 = 0; k0 < K; k0 += p.KB) {
         const int kb = std::min(p.KB, K - k0);
         for (int i = 0; i < kb; ++i) {
             lim[(size_t)2 * k0 + i] = (temp - eps) * g[k0 + i] * 2.0 / c->beta;
-            lim[(size_t)2 * k0 + kb + i] = g[k0 + i] == 0.0 ? 0.0 : g[k0 + i] < GG_MIN ? 1.0 / GG_MIN : 1.0;
+            lim[(size_t)2 * k0 + kb + i] = g[k0 + i] == 0.0 ? 0.0 : 1.0;
         }
     }
     DevBuf buf;

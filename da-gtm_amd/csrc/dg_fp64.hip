@@ -890,10 +890,11 @@ __device__ __forceinline__ double wave_sum(double x) {
 }
 
 // The eigenvalue of one centre's S that the critical temperature takes.  Workgroup
-// (kb, part): of A = sc (2 S1) or sc (2 S1 - 2 S2), n x n, the largest eigenvalue
-// below sc limit, and 0 in the place of those at or above it (comm.c:2149-2161):
-// val[2 kb + part] = their maximum / sc.  A's lower triangle is packed in LDS,
-// reduced to tridiagonal form by Householder reflections (Golub & Van Loan,
+// (kb, part): of A = 2 S1 or 2 S1 - 2 S2, n x n, the largest eigenvalue below
+// limit, and 0 in the place of those at or above it (comm.c:2149-2161):
+// val[2 kb + part] = their maximum.  A's lower triangle is packed in LDS, scaled by
+// a power of two to a largest entry in [1, 2) (a centre's weight, and so its S, may
+// be any double down to the smallest, and the sums below square the entries), reduced to tridiagonal form by Householder reflections (Golub & Van Loan,
 // Matrix Computations, 4th ed., 8.3.1), and the one eigenvalue wanted is found by
 // Sturm counts (8.4.1) at 64 points of the interval at a time, one per lane.
 // Bound by the chain of reflections (two reductions and a matrix-vector product
@@ -903,15 +904,14 @@ __device__ __forceinline__ double wave_sum(double x) {
 // and 0.2 s at n = 166.
 __global__ __launch_bounds__(256) void k_ctemp_eig(const double *__restrict__ S, int n,
                                                    const double *__restrict__ limit,
-                                                   const double *__restrict__ scale,
+                                                   const double *__restrict__ asked,
                                                    double *__restrict__ val) {
     extern __shared__ double A[];                  // n (n + 1) / 2, then v, p, d, e of n each
     __shared__ double red[4];
     const int tid = threadIdx.x, nt = blockDim.x, l = tid & 63, w = tid >> 6;
     const long kb = blockIdx.x;
     const int sub = blockIdx.y;
-    const double sc = scale[kb], lim = limit[kb] * sc;
-    if (sc == 0.0) return;                         // a centre without weight: not asked for
+    if (asked[kb] == 0.0) return;                  // a centre without weight
     double *v = A + n * (n + 1) / 2, *p = v + n, *d = p + n, *e = d + n;
     const double *S1 = S + kb * 2 * n * n, *S2 = S1 + (long)n * n;
     auto at = [&](int i, int j) -> double & { return A[i * (i + 1) / 2 + j]; };   // j <= i
@@ -923,6 +923,7 @@ __global__ __launch_bounds__(256) void k_ctemp_eig(const double *__restrict__ S,
         __syncthreads();
         return (red[0] + red[1]) + (red[2] + red[3]);
     };
+    double top = 0.0;                              // the largest |entry| (NaN left out)
     for (int e0 = tid; e0 < n * n; e0 += 8 * nt) {  // (eight elements' loads in flight)
         double a[8], b[8];
 #pragma unroll
@@ -934,10 +935,21 @@ __global__ __launch_bounds__(256) void k_ctemp_eig(const double *__restrict__ S,
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
             const int e = e0 + u * nt, i = e / n, j = e - i * n;
-            const double x = 2.0 * a[u];
-            if (i < n && j <= i) at(i, j) = (sub ? x - 2.0 * b[u] : x) * sc;
+            const double x = sub ? 2.0 * a[u] - 2.0 * b[u] : 2.0 * a[u];
+            if (i < n && j <= i) {
+                at(i, j) = x;
+                top = fmax(top, fabs(x));
+            }
         }
     }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) top = fmax(top, __shfl_xor(top, o));
+    if (l == 0) red[w] = top;
+    __syncthreads();
+    for (int x = 0; x < nt / 64; ++x) top = fmax(top, red[x]);
+    const int ex = (top > 0.0 && top < INFINITY) ? ilogb(top) : 0;   // 2^ex <= top < 2^(ex + 1)
+    const double lim = ldexp(limit[kb], -ex);
+    for (int x = tid; x < n * (n + 1) / 2; x += nt) A[x] = ldexp(A[x], -ex);
     __syncthreads();
     for (int k = 0; k + 2 < n; ++k) {
         // the reflection that annihilates A[k + 2 .., k]: v = x - alpha e1
@@ -1071,7 +1083,7 @@ __global__ __launch_bounds__(256) void k_ctemp_eig(const double *__restrict__ S,
             best = fmax(best, 0.5 * (a + b));
         }
     }
-    if (l == 0) val[2 * kb + sub] = best / sc;
+    if (l == 0) val[2 * kb + sub] = ldexp(best, ex);
 }
 
 }  // namespace

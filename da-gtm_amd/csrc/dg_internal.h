@@ -235,8 +235,9 @@ int dg_resp_dense_fp64(dg_ctx *ctx, double *dR, long ldR);
 int dg_map_fp64(dg_ctx *ctx, const double *dX, int L, double *dM);
 // The critical temperatures' eigenvalues for centres k0 .. k0 + KB - 1, from the FP64
 // normalisers: dVal[2 k + part] for part 0 (2 S1) and 1 (2 S1 - 2 S2).  dLimit
-// holds, for each batch, its KB limits and then its KB scales at 2 k0; buf the
-// batch's R, moment partials and, with several chunks, their sums.
+// holds, for each batch at 2 k0, its KB limits and then KB flags (0: a centre
+// without weight, left out); buf the batch's R, moment partials and, with several
+// chunks, their sums.
 struct DgCtempPlan {
     int KB, nc, pairs;        // centres per batch, N chunks, tile pairs of a moment
     size_t r_len, s_len;      // doubles of R and of one set of S1, S2
