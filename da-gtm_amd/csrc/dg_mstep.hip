@@ -395,16 +395,18 @@ __device__ __forceinline__ double row_bcast(double x) {
 // S is that (n + nrhs) x n matrix, row-major, factored in place; Ld takes the
 // diagonal blocks' factors, transposed and filled up with the identity, 64 x 64
 // each.  One launch per block column (k_bc_step), one for the whole backward
-// substitution (k_bc_back).  A non-positive pivot clears scal[kScalSolveOK]; every
-// later kernel of the sequence then returns at once, and the host retries with a
-// jitter.
+// substitution (k_bc_back).  failed[kc] is 1 where a pivot before block column kc was
+// not positive: launch kc reads failed[kc] and writes failed[kc + 1], so that no
+// workgroup reads what another one of its launch writes.  After a failure the
+// kernels of the sequence return at once, and the host retries with a jitter.
 constexpr int BC = 64;
 constexpr int kBcLd = BC + 2;    // LDS row stride: 16 rows x 2 inner indexes hit 32 banks
 
 __global__ __launch_bounds__(256) void k_bc_init(const double *__restrict__ A0,
                                                  double *__restrict__ S, int n, double ridge,
                                                  double jit, const double *__restrict__ B,
-                                                 int nrhs, double *__restrict__ scal) {
+                                                 int nrhs, double *__restrict__ failed,
+                                                 double *__restrict__ scal) {
     const long e = (long)blockIdx.x * 256 + threadIdx.x;
     const long nn = (long)n * n;
     if (e < nn) {
@@ -414,7 +416,7 @@ __global__ __launch_bounds__(256) void k_bc_init(const double *__restrict__ A0,
         S[e] = B[p * nrhs + c];
     }
     if (e == 0) {
-        scal[kScalSolveOK] = 1.0;
+        failed[0] = 0.0;
         scal[kScalJitter] = jit;
     }
 }
@@ -439,12 +441,15 @@ __global__ __launch_bounds__(256) void k_bc_init(const double *__restrict__ A0,
 constexpr int kBcNT = 320;
 __global__ __launch_bounds__(kBcNT) void k_bc_step(double *__restrict__ S, int n, int nrows, int kc,
                                                    double *__restrict__ Ld,
-                                                   double *__restrict__ scal) {
+                                                   double *__restrict__ failed) {
     __shared__ double Pk[BC][kBcLd];               // L[kc][kc - 1], or a tile's columns
     __shared__ double Dg[BC][kBcLd];               // the diagonal block
     __shared__ int bad;
-    if (scal[kScalSolveOK] != 1.0) return;
     const int tid = threadIdx.x, l = tid & 63, j = l & 15, g = l >> 4;
+    if (failed[kc] != 0.0) {
+        if (tid == 0 && blockIdx.x == 0 && blockIdx.y == 0) failed[kc + 1] = 1.0;
+        return;
+    }
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int k0 = kc * BC, kb = min(BC, n - k0), k1 = k0 + kb, kp = k0 - BC;
     const int i0 = k1 + blockIdx.x * BC;           // the first of this workgroup's rows
@@ -580,10 +585,8 @@ __global__ __launch_bounds__(kBcNT) void k_bc_step(double *__restrict__ S, int n
             __syncthreads();
         }
     });
-    if (bad) {                                     // the same in every workgroup
-        if (tid == 0 && blockIdx.x == 0) scal[kScalSolveOK] = 0.0;
-        return;
-    }
+    if (tid == 0 && blockIdx.x == 0) failed[kc + 1] = bad ? 1.0 : 0.0;
+    if (bad) return;                               // the same in every workgroup
     if (blockIdx.x == 0)
         for (int e = tid; e < BC * BC; e += kBcNT) {
             const int c = e >> 6, r = e & 63;
@@ -611,15 +614,18 @@ __global__ __launch_bounds__(kBcNT) void k_bc_step(double *__restrict__ S, int n
 __global__ __launch_bounds__(kBcNT) void k_bc_back(const double *__restrict__ S, int n, int nrhs,
                                                    const double *__restrict__ Ld,
                                                    double *__restrict__ W,
-                                                   const double *__restrict__ scal) {
+                                                   const double *__restrict__ failed,
+                                                   double *__restrict__ scal) {
     __shared__ __align__(16) double Lt[2][BC][kBcLd];   // L_kk transposed: Lt[i][p] = L[p][i]
     __shared__ double Ln[BC][kBcLd];                    // L[k][k - 1]
     __shared__ double Sx[BC][16], Xs[BC][16];           // the block's right side, its solution
     __shared__ double Sn[BC][16];                       // the next one's, but for the block's product
-    if (scal[kScalSolveOK] != 1.0) return;
     const int tid = threadIdx.x, l = tid & 63, j = l & 15, g = l >> 4;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nb = (n + BC - 1) / BC;
+    const bool ok = failed[nb] == 0.0;
+    if (tid == 0 && blockIdx.x == 0) scal[kScalSolveOK] = ok ? 1.0 : 0.0;
+    if (!ok) return;
     const int col = min(16 * (int)blockIdx.x + j, nrhs - 1);   // past the end: the last again
     const bool live = 16 * (int)blockIdx.x + j < nrhs;
     const double *Yc = S + (long)(n + col) * n;
@@ -1240,21 +1246,22 @@ int dg_centres_from_w(dg_ctx *c) {
 }
 
 // (A0 + (ridge + jit) I) W = Bm for M + 1 > 126 by the blocked kernels, in the
-// (consumed) partials of A and B; clears scal[kScalSolveOK] on a non-positive pivot
+// (consumed) partials of A and B; scal[kScalSolveOK] is 0 after a non-positive pivot
 int blocked_chol_solve(dg_ctx *c, double ridge, double jit) {
     const int n = c->M1, D = c->D, nb = (n + BC - 1) / BC;
-    double *S = c->partAB, *Ld = c->A;             // (n >= 127: n^2 > 64 (n + 63))
+    // (n >= 127: n^2 > 64 (n + 63) + nb, the diagonal blocks and nb + 1 flags)
+    double *S = c->partAB, *Ld = c->A, *failed = Ld + (size_t)nb * BC * BC;
     const long tot = (long)n * n + (long)n * D;
     hipLaunchKernelGGL(k_bc_init, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, c->stream,
-                       c->A0, S, n, ridge, jit, c->Bm, D, c->scal);
+                       c->A0, S, n, ridge, jit, c->Bm, D, failed, c->scal);
     for (int k = 0; k < nb; ++k) {
         const int k1 = std::min(n, (k + 1) * BC);
         const int rt = (n + D - k1 + BC - 1) / BC, ct = (k > 0) ? (n - k1 + BC - 1) / BC : 0;
         hipLaunchKernelGGL(k_bc_step, dim3((unsigned)rt, (unsigned)(1 + ct)), dim3(kBcNT), 0,
-                           c->stream, S, n, n + D, k, Ld, c->scal);
+                           c->stream, S, n, n + D, k, Ld, failed);
     }
     hipLaunchKernelGGL(k_bc_back, dim3((unsigned)((D + 15) / 16)), dim3(kBcNT), 0, c->stream, S, n,
-                       D, Ld, c->W, c->scal);
+                       D, Ld, c->W, failed, c->scal);
     DG_HIP(c, hipGetLastError());
     return DG_OK;
 }
