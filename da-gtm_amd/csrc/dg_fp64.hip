@@ -26,6 +26,7 @@
 // falling back to R = 1/K (h = K; g = K in EM mode only).
 #include <algorithm>
 #include <cmath>
+#include <limits>
 #include <type_traits>
 
 #include "dg_internal.h"
@@ -1088,6 +1089,13 @@ __global__ __launch_bounds__(256) void k_ctemp_eig(const double *__restrict__ S,
 
 }  // namespace
 
+// 1 / temp.  For an infinite temperature the smallest positive number: the same
+// share for every centre whose exponent is finite, none for the others, where 0
+// times their -inf would be NaN.
+static double inv_temp(bool isDA, double temp) {
+    return isDA ? std::max(1.0 / temp, std::numeric_limits<double>::denorm_min()) : 1.0;
+}
+
 // Pass 1 splits a point tile's slices over four workgroups up to 64 x 16 points
 // per CU: below that, whole point tiles are too few to spread evenly (N = 10^5,
 // D = 166, K = 8000: 6.4 ms split, 7.2 whole; N = 260000, K = 1000: 2.17 and
@@ -1099,7 +1107,7 @@ long dg_pass1_wgs(long N) { return N < kSplitPoints ? (N + NT - 1) / NT : (N + P
 
 int dg_pass1_fp64(dg_ctx *c, int isDA, double temp) {
     const double nbh = -c->beta / 2.0;
-    const double it = isDA ? 1.0 / temp : 1.0;
+    const double it = inv_temp(isDA, temp);
     const PointOut po{c->pm, c->pl, c->logg, c->logh, it, log((double)c->K),
                       (isDA && it != 1.0) ? 1 : 0, isDA};
     const unsigned tiles = (unsigned)((c->N + P1 - 1) / P1);
@@ -1121,7 +1129,7 @@ int dg_pass1_fp64(dg_ctx *c, int isDA, double temp) {
 
 int dg_pass2_fp64(dg_ctx *c, int isDA, double temp) {
     const double nbh = -c->beta / 2.0;
-    const double it = isDA ? 1.0 / temp : 1.0;
+    const double it = inv_temp(isDA, temp);
     const long tiles = (c->N + TP - 1) / TP;
     const long chunk = ((tiles + c->NC - 1) / c->NC) * TP;
     const dim3 grid((unsigned)((c->K + 63) / 64), (unsigned)c->NC);
@@ -1165,7 +1173,7 @@ static Ranges centre_ranges(long N, int K) {
 size_t dg_map_part(long N, int K) { return (size_t)5 * N * centre_ranges(N, K).count; }
 
 int dg_resp_dense_fp64(dg_ctx *c, double *dR, long ldR) {
-    const double it = c->last_isDA ? 1.0 / c->last_temp : 1.0;
+    const double it = inv_temp(c->last_isDA, c->last_temp);
     const Ranges r = centre_ranges(c->N, c->K);
     hipLaunchKernelGGL(k_resp_dense, dim3((unsigned)((c->N + P1 - 1) / P1), (unsigned)r.count),
                        dim3(NT), 0, c->stream, c->T64, c->tt, c->N, c->Y64, c->yy, c->K, c->D,
@@ -1176,7 +1184,7 @@ int dg_resp_dense_fp64(dg_ctx *c, double *dR, long ldR) {
 
 int dg_ctemp_fp64(dg_ctx *c, int k0, int KB, const DgCtempPlan &p, const double *dLimit,
                   double *buf, double *dVal) {
-    const double it = c->last_isDA ? 1.0 / c->last_temp : 1.0;
+    const double it = inv_temp(c->last_isDA, c->last_temp);
     const int D = c->D;
     double *R = buf, *part = buf + p.r_len, *S = p.nc > 1 ? part + p.s_len * p.nc : part;
     // R of these centres, then their moments, then the eigenvalues
@@ -1225,7 +1233,7 @@ DgCtempPlan dg_ctemp_plan(const dg_ctx *c) {
 }
 
 int dg_map_fp64(dg_ctx *c, const double *dX, int L, double *dM) {
-    const double it = c->last_isDA ? 1.0 / c->last_temp : 1.0;
+    const double it = inv_temp(c->last_isDA, c->last_temp);
     const Ranges r = centre_ranges(c->N, c->K);
     hipLaunchKernelGGL(k_map_f64, dim3((unsigned)((c->N + P1 - 1) / P1), (unsigned)r.count), dim3(NT),
                        0, c->stream, c->T64, c->tt, c->N, c->Y64, c->yy, c->K, c->D, c->ldt,
