@@ -662,8 +662,9 @@ __global__ __launch_bounds__(NT, 2) void k_map_f64(
             m = top;
         }
         const double ms = (m == -INFINITY) ? 0.0 : m;
-        // (the sum is at least 1, and all that is left out of it below 2^-66)
-        if (__any((top - ms) * it > -60.0)) {
+        // (below this every p is exactly 0; a higher bound would drop a small p whose
+        // coordinate is large)
+        if (__any((top - ms) * it > kExpUnderflowX)) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const double v = exp((x[r] - ms) * it);
