@@ -14,6 +14,7 @@
 #include <cstdlib>
 #include <functional>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <new>
 #include <string>
@@ -785,9 +786,18 @@ int dg_map(dg_ctx *c, const double *X, int L, long ldX, double *M, long ldM) {
         if ((rc = dg_estep(c, c->last_isDA, c->last_temp, &eo))) return rc;
     }
     c->fp64_due = c->mixed();
+    // a centre's coordinates may be a few doubles of a much longer row
+    std::unique_ptr<double[]> packed;
+    if (ldX != L) {
+        packed.reset(new (std::nothrow) double[(size_t)c->K * L]);
+        if (!packed) return dg_fail(c, DG_ENOMEM, "host allocation");
+        for (int k = 0; k < c->K; ++k)
+            std::memcpy(&packed[(size_t)k * L], X + (size_t)k * ldX, (size_t)L * sizeof(double));
+        X = packed.get();
+    }
     // the coordinates and the projection behind the projection's sums
     double *dX = c->partRT + dg_map_part(c->N, c->K), *dM = dX + (size_t)c->K * L;
-    if ((rc = upload_rows(c, dX, L, X, ldX, c->K, L)) || (rc = dg_map_fp64(c, dX, L, dM))) return rc;
+    if ((rc = upload_rows(c, dX, L, X, L, c->K, L)) || (rc = dg_map_fp64(c, dX, L, dM))) return rc;
     return download_rows(c, M, ldM, dM, c->N, L);
 }
 
