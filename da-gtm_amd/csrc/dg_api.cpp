@@ -413,7 +413,7 @@ int dg_estep(dg_ctx *c, int isDA, double temp, dg_estep_out *out) {
     if (isDA && !(temp > 0.0)) return dg_fail(c, DG_EINVAL, "dg_estep: temp must be > 0");
     int rc;
     if ((rc = select_device(c))) return rc;
-    c->fp64_due = false;
+    c->fp64_due = c->fp64_norm = false;
     if (c->mixed()) rc = dg_estep_mixed(c, isDA, temp);
     else rc = dg_estep_fp64(c, isDA, temp);
     if (rc) return rc;
@@ -440,11 +440,23 @@ int dg_estep(dg_ctx *c, int isDA, double temp, dg_estep_out *out) {
 
 // The FP64 outputs of a mixed context (dg_map, dg_next_ctemp, dg_resp_dense)
 // leave G and R T in FP64 for what reads them next, as the rest of their state:
-// computed here, when something does.
+// computed here, when something does, from the normalisers where one of them made
+// those.
 static int due_stats(dg_ctx *c) {
     if (!c->fp64_due) return DG_OK;
+    const int rc = c->fp64_norm ? dg_stats_fp64(c, c->last_isDA, c->last_temp)
+                                : dg_estep_fp64(c, c->last_isDA, c->last_temp);
+    if (rc) return rc;
     c->fp64_due = false;
-    return dg_estep_fp64(c, c->last_isDA, c->last_temp);
+    c->fp64_norm = c->mixed();
+    return DG_OK;
+}
+
+// the FP64 normalisers of a mixed context's E-step
+static int fp64_normalisers(dg_ctx *c) {
+    const int rc = dg_pass1_fp64(c, c->last_isDA, c->last_temp);
+    c->fp64_norm = rc == DG_OK;
+    return rc;
 }
 
 int dg_mstep(dg_ctx *c, double *beta_out) {
@@ -620,7 +632,7 @@ static int next_ctemp_impl(dg_ctx *c, double temp, double eps, const double *gg,
     if ((rc = select_device(c))) return rc;
     // R in FP64: the mixed path refreshes the FP64 per-point normalisers
     c->fp64_due = c->mixed();
-    if (c->mixed() && (rc = dg_pass1_fp64(c, c->last_isDA, c->last_temp))) return rc;
+    if (c->mixed() && (rc = fp64_normalisers(c))) return rc;
     const int K = c->K;
     std::vector<double> g(K), ck(K);
     if (gg) {
@@ -839,7 +851,7 @@ int dg_resp_dense(dg_ctx *c, double *R, long ldR) {
     int rc;
     if ((rc = select_device(c))) return rc;
     c->fp64_due = c->mixed();
-    if (c->mixed() && (rc = dg_pass1_fp64(c, c->last_isDA, c->last_temp))) return rc;
+    if (c->mixed() && (rc = fp64_normalisers(c))) return rc;
     DevBuf own;
     double *dR = c->partRT;
     if ((size_t)c->K * c->N > c->partRT_len) {

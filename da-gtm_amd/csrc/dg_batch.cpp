@@ -311,7 +311,7 @@ int dg_batch_run_mixed(std::vector<dg_ctx *> &ctx, const dg_anneal_params *param
             const double nfree =
                 isDA ? batch_quality(c->N, c->K, c->D, c->beta, s[kScalSumLogH], temp) : -llh;
             c->have_estep = true;
-            c->fp64_due = false;
+            c->fp64_due = c->fp64_norm = false;
             c->last_isDA = isDA != 0;
             c->last_temp = isDA ? temp : 1.0;
             mach[i].estep_done(llh, nfree);

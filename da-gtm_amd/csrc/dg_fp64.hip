@@ -1128,7 +1128,7 @@ int dg_pass1_fp64(dg_ctx *c, int isDA, double temp) {
     return DG_OK;
 }
 
-int dg_pass2_fp64(dg_ctx *c, int isDA, double temp) {
+static int dg_pass2_fp64(dg_ctx *c, int isDA, double temp) {
     const double nbh = -c->beta / 2.0;
     const double it = inv_temp(isDA, temp);
     const long tiles = (c->N + TP - 1) / TP;
@@ -1144,11 +1144,8 @@ int dg_pass2_fp64(dg_ctx *c, int isDA, double temp) {
     return DG_OK;
 }
 
-int dg_estep_fp64(dg_ctx *c, int isDA, double temp) {
+int dg_stats_fp64(dg_ctx *c, int isDA, double temp) {
     int rc;
-    if (c->timing) DG_HIP(c, hipEventRecord(c->ev[0], c->stream));
-    if ((rc = dg_pass1_fp64(c, isDA, temp))) return rc;
-    if (c->timing) DG_HIP(c, hipEventRecord(c->ev[1], c->stream));
     if ((rc = dg_pass2_fp64(c, isDA, temp))) return rc;
     if (c->timing) DG_HIP(c, hipEventRecord(c->ev[2], c->stream));
     const long nred = (long)c->K * c->D + c->K;
@@ -1157,6 +1154,14 @@ int dg_estep_fp64(dg_ctx *c, int isDA, double temp) {
                        c->partLog64, dg_pass1_wgs(c->N), c->scal, c->m_scal);
     DG_HIP(c, hipGetLastError());
     return DG_OK;
+}
+
+int dg_estep_fp64(dg_ctx *c, int isDA, double temp) {
+    int rc;
+    if (c->timing) DG_HIP(c, hipEventRecord(c->ev[0], c->stream));
+    if ((rc = dg_pass1_fp64(c, isDA, temp))) return rc;
+    if (c->timing) DG_HIP(c, hipEventRecord(c->ev[1], c->stream));
+    return dg_stats_fp64(c, isDA, temp);
 }
 
 // k_resp_dense and k_map_f64 split the centre tiles into ranges until there are

@@ -29,6 +29,7 @@ struct dg_ctx {
     bool have_estep = false;       // G/RT/pm/pl valid for the current Y
     bool fp64_due = false;         // mixed: an FP64 output was made from this E-step, so the
                                    // next reader of G and R T gets them from an FP64 E-step
+    bool fp64_norm = false;        // mixed: pm, pl and partLog64 are FP64 pass 1's for this E-step
     bool have_w = false;           // W holds the last M-step's (or a caller's) weights
     bool last_isDA = true;
     double last_temp = 1.0;
@@ -231,6 +232,7 @@ size_t dg_pass1_part(long N);     // doubles of partRT that pass 1 needs for its
 size_t dg_map_part(long N, int K);   // doubles of partRT that dg_map_fp64 needs
 int dg_estep_fp64(dg_ctx *ctx, int isDA, double temp);
 int dg_pass1_fp64(dg_ctx *ctx, int isDA, double temp);   // its first half: pm, pl, log g, log h
+int dg_stats_fp64(dg_ctx *ctx, int isDA, double temp);   // its second: G, R T, the log sums
 int dg_resp_dense_fp64(dg_ctx *ctx, double *dR, long ldR);
 int dg_map_fp64(dg_ctx *ctx, const double *dX, int L, double *dM);
 // The critical temperatures' eigenvalues for centres k0 .. k0 + KB - 1, from the FP64
