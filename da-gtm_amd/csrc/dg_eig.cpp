@@ -1,8 +1,9 @@
 // Eigenvalues of a real symmetric matrix (host code): Householder reduction to
 // tridiagonal form followed by the implicit QL iteration with Wilkinson shifts
 // (Golub & Van Loan, Matrix Computations, 4th ed., sections 8.3.1 and 8.3.5).
-// Used for the small D x D problems of the critical-temperature search; plain
-// C++ with no device code, so the tests can build it on its own.
+// Not part of the library, which finds the critical temperatures' eigenvalues on
+// the device (k_ctemp_eig): the same reduction in plain C++, for a host without a
+// device.  tests/test_ctemp.py builds it by itself and holds it against LAPACK.
 #include <algorithm>
 #include <cmath>
 #include <limits>

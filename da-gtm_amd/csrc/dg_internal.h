@@ -249,9 +249,6 @@ DgCtempPlan dg_ctemp_plan(const dg_ctx *ctx);
 int dg_ctemp_fp64(dg_ctx *ctx, int k0, int KB, const DgCtempPlan &p, const double *dLimit,
                   double *buf, double *dVal);
 
-// ---- host eigenvalues (dg_eig.cpp): the plain statement that the tests hold against LAPACK ----
-extern "C" int dg_sym_eigvals(int n, const double *A, long lda, double *w);
-
 // ---- mixed kernels (dg_mixed.hip) ----
 int dg_mixed_prepare_t(dg_ctx *ctx);
 // Built-in pass-2 chunk count for the context's shape; *lo / *hi (may be

@@ -608,7 +608,7 @@ __device__ __forceinline__ void k_sum_partlog_body(const double *__restrict__ pa
 // tile in AKS floats: the tile's 32 values, their largest (pass 1's screen),
 // three -inf pads.
 __device__ __forceinline__ void k_make_ak_body(
-    const int bx, const int by, const int bz, const int gx, const float *__restrict__ yy32,
+    const int bx, const float *__restrict__ yy32,
     int K, int Kp, float beta, float *__restrict__ aK32) {
     const int k = bx * blockDim.x + threadIdx.x;
     const float cb = -0.5f * beta * kLog2e;
@@ -625,7 +625,7 @@ __device__ __forceinline__ void k_make_ak_body(
 
 __global__ void k_make_ak(const float *__restrict__ yy32, int K, int Kp, float beta,
                           float *__restrict__ aK32) {
-    k_make_ak_body(blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, yy32, K, Kp, beta, aK32);
+    k_make_ak_body(blockIdx.x, yy32, K, Kp, beta, aK32);
 }
 
 // ---------------------------------------------------------------- pass 2
@@ -1210,7 +1210,7 @@ __global__ __launch_bounds__(NTH) void k_item_table(const int2 *__restrict__ bra
 constexpr int RK = 64, RD = 4, RU = 16;
 
 __device__ __forceinline__ void k_reduce32_body(
-    const int bx, const int by, const int bz, const int gx, const float *__restrict__ partRT,
+    const int bx, const int by, const float *__restrict__ partRT,
     const float *__restrict__ partG, int NC, int K, int D, double *__restrict__ RT,
     double *__restrict__ G, const int2 *__restrict__ brange) {
     __shared__ double tile[RK][RD + 1];
@@ -1261,14 +1261,14 @@ __global__ __launch_bounds__(RK * RD) void k_reduce32(const float *__restrict__ 
                                                       int K, int D, double *__restrict__ RT,
                                                       double *__restrict__ G,
                                                       const int2 *__restrict__ brange) {
-    k_reduce32_body(blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, partRT, partG, NC, K, D, RT, G,
+    k_reduce32_body(blockIdx.x, blockIdx.y, partRT, partG, NC, K, D, RT, G,
                     brange);
 }
 
 // Zero-column fall-back R = 1/K for the points pass 2 skipped: RT[k] +=
 // (1/K) sum_{n in Z} t_n, G[k] += |Z| / K.  Exits at once when |Z| = 0.
 __device__ __forceinline__ void k_zero_fix_body(
-    const int bx, const int by, const int bz, const int gx, const double *__restrict__ scal,
+    const int bx, const double *__restrict__ scal,
     const double *__restrict__ T64, int ldt, const double *__restrict__ pm, long N, int K,
     int D, double *__restrict__ RT, double *__restrict__ G) {
     const double nz = scal[kScalNZero];
@@ -1296,20 +1296,19 @@ __global__ __launch_bounds__(256) void k_zero_fix(const double *__restrict__ sca
                                                   const double *__restrict__ pm, long N, int K,
                                                   int D, double *__restrict__ RT,
                                                   double *__restrict__ G) {
-    k_zero_fix_body(blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, scal, T64, ldt, pm, N, K, D, RT,
-                    G);
+    k_zero_fix_body(blockIdx.x, scal, T64, ldt, pm, N, K, D, RT, G);
 }
 
 // Workgroup partials of max |x| and of the count of values not exact in
 // FP16 over rows x D (stride ld): part[2 b], part[2 b + 1].
 constexpr int kAmaxWG = 256;
-__device__ __forceinline__ void k_absmax_part_body(
-    const int bx, const int by, const int bz, const int gx, const double *__restrict__ X,
-    long rows, int ld, int D, double *__restrict__ part) {
+__global__ __launch_bounds__(256) void k_absmax_part(const double *__restrict__ X, long rows,
+                                                     int ld, int D, double *__restrict__ part) {
+    const int bx = blockIdx.x;
     __shared__ double smax[256], scnt[256];
     double mx = 0.0, cnt = 0.0;
     const long total = rows * D;
-    for (long e = (long)bx * 256 + threadIdx.x; e < total; e += (long)gx * 256) {
+    for (long e = (long)bx * 256 + threadIdx.x; e < total; e += (long)gridDim.x * 256) {
         const double v = X[(e / D) * ld + (e % D)];
         mx = fmax(mx, fabs(v));
         const _Float16 hv = (_Float16)(float)v;
@@ -1327,14 +1326,8 @@ __device__ __forceinline__ void k_absmax_part_body(
     if (threadIdx.x == 0) { part[2 * bx] = smax[0]; part[2 * bx + 1] = scnt[0]; }
 }
 
-__global__ __launch_bounds__(256) void k_absmax_part(const double *__restrict__ X, long rows,
-                                                     int ld, int D, double *__restrict__ part) {
-    k_absmax_part_body(blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, X, rows, ld, D, part);
-}
-
-__device__ __forceinline__ void k_absmax_final_body(
-    const int bx, const int by, const int bz, const int gx, const double *__restrict__ part,
-    int n, double *__restrict__ out) {
+__global__ __launch_bounds__(256) void k_absmax_final(const double *__restrict__ part, int n,
+                                                      double *__restrict__ out) {
     __shared__ double smax[256], scnt[256];
     double mx = 0.0, cnt = 0.0;
     for (int i = threadIdx.x; i < n; i += 256) { mx = fmax(mx, part[2 * i]); cnt += part[2 * i + 1]; }
@@ -1348,11 +1341,6 @@ __device__ __forceinline__ void k_absmax_final_body(
         __syncthreads();
     }
     if (threadIdx.x == 0) { out[0] = smax[0]; out[1] = scnt[0]; }
-}
-
-__global__ __launch_bounds__(256) void k_absmax_final(const double *__restrict__ part, int n,
-                                                      double *__restrict__ out) {
-    k_absmax_final_body(blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, part, n, out);
 }
 
 // Power-of-two scale putting max |x| at or below 2^14.
@@ -1454,7 +1442,7 @@ __global__ void k_transpose16(const _Float16 *__restrict__ T16, long N, long Np,
 // scale chosen from scal_in[0] = max |Y|: Y16[t][k][d], rows k >= K zero;
 // yy32[k] = |y'|^2 of the split value; mscal[0] = the scale.
 __device__ __forceinline__ void k_make_y16_body(
-    const int bx, const int by, const int bz, const int gx, const double *__restrict__ Y64,
+    const int bx, const double *__restrict__ Y64,
     int ldt, int K, int Kp, int D, int ld16, const double *__restrict__ amax,
     _Float16 *__restrict__ Y16, float *__restrict__ yy32, double *__restrict__ mscal) {
     // one wave per centre row; lanes step over d, the norm is a wave sum
@@ -1483,7 +1471,7 @@ __global__ __launch_bounds__(256) void k_make_y16(const double *__restrict__ Y64
                                                   _Float16 *__restrict__ Y16,
                                                   float *__restrict__ yy32,
                                                   double *__restrict__ mscal) {
-    k_make_y16_body(blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, Y64, ldt, K, Kp, D, ld16, amax,
+    k_make_y16_body(blockIdx.x, Y64, ldt, K, Kp, D, ld16, amax,
                     Y16, yy32, mscal);
 }
 
@@ -1800,7 +1788,7 @@ __global__ __launch_bounds__(256) void kb_make_ak(const BInst *__restrict__ tab,
     const int2 m = map[blockIdx.x];
     const BInst &I = tab[m.x];
     if (!I.do_e) return;
-    k_make_ak_body(m.y, 0, 0, 0, I.yy32, I.K, I.Kp, I.beta_f, I.aK32);
+    k_make_ak_body(m.y, I.yy32, I.K, I.Kp, I.beta_f, I.aK32);
 }
 
 __global__ __launch_bounds__(256) void kb_sum_partlog(const BInst *__restrict__ tab,
@@ -1816,7 +1804,7 @@ __global__ __launch_bounds__(RK * RD) void kb_reduce32(const BInst *__restrict__
     const BInst &I = tab[m.x];
     if (!I.do_e) return;
     const int nkx = (I.K + RK - 1) / RK;
-    k_reduce32_body(m.y % nkx, m.y / nkx, 0, 0, I.partRT32, I.partG32, I.NC, I.K, I.D, I.RT,
+    k_reduce32_body(m.y % nkx, m.y / nkx, I.partRT32, I.partG32, I.NC, I.K, I.D, I.RT,
                     I.G, I.brange);
 }
 
@@ -1825,7 +1813,7 @@ __global__ __launch_bounds__(256) void kb_zero_fix(const BInst *__restrict__ tab
     const int2 m = map[blockIdx.x];
     const BInst &I = tab[m.x];
     if (!I.do_e) return;
-    k_zero_fix_body(m.y, 0, 0, 0, I.scal, I.T64, I.ldt, I.pm, I.N, I.K, I.D, I.RT, I.G);
+    k_zero_fix_body(m.y, I.scal, I.T64, I.ldt, I.pm, I.N, I.K, I.D, I.RT, I.G);
 }
 
 __global__ __launch_bounds__(NTH) void kb_block_ranges(const BInst *__restrict__ tab,
@@ -1841,7 +1829,7 @@ __global__ __launch_bounds__(256) void kb_make_y16(const BInst *__restrict__ tab
     const int2 m = map[blockIdx.x];
     const BInst &I = tab[m.x];
     if (!I.do_m) return;
-    k_make_y16_body(m.y, 0, 0, 0, I.Y64, I.ldt, I.K, I.Kp, I.D, I.ldh, I.scal + kScalYMax, I.Y16,
+    k_make_y16_body(m.y, I.Y64, I.ldt, I.K, I.Kp, I.D, I.ldh, I.scal + kScalYMax, I.Y16,
                     I.yy32, I.mscal);
 }
 

@@ -18,10 +18,9 @@
 namespace {
 
 // out[r] = sum_d X[r][d]^2, sequential in d (the ddot loops of comm.c:604-618)
-__device__ __forceinline__ void k_rownorm_body(
-    const int bx, const int by, const int bz, const int gx, const double *__restrict__ X,
-    long rows, int ld, int D, double *__restrict__ out) {
-    const long r = (long)bx * blockDim.x + threadIdx.x;
+__global__ void k_rownorm(const double *__restrict__ X, long rows, int ld, int D,
+                          double *__restrict__ out) {
+    const long r = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= rows) return;
     // eight loads in flight, then their FMAs in order
     double s = 0.0;
@@ -38,11 +37,6 @@ __device__ __forceinline__ void k_rownorm_body(
         s = fma(v, v, s);
     }
     out[r] = s;
-}
-
-__global__ void k_rownorm(const double *__restrict__ X, long rows, int ld, int D,
-                          double *__restrict__ out) {
-    k_rownorm_body(blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, X, rows, ld, D, out);
 }
 
 // Deterministic block-tree sum of a vector into scal[slot].  Single workgroup, FP64.
@@ -82,9 +76,8 @@ __device__ void block_trace(const double *__restrict__ A0, int n, double *out) {
 // growing x10 per retry, at most 8 retries.  scal[kScalSolveOK] = 1 on
 // success, scal[kScalJitter] = the jitter used.
 __device__ __forceinline__ void k_chol_solve_body(
-    const int bx, const int by, const int bz, const int gx, const double *__restrict__ A0,
-    double *__restrict__ A, int n, double ridge, const double *__restrict__ B, int nrhs,
-    double *__restrict__ Wout, double *__restrict__ scal) {
+    const double *__restrict__ A0, double *__restrict__ A, int n, double ridge,
+    const double *__restrict__ B, int nrhs, double *__restrict__ Wout, double *__restrict__ scal) {
     __shared__ int fail;
     __shared__ double tr;
     const int tid = threadIdx.x, nt = blockDim.x;
@@ -290,7 +283,7 @@ __global__ __launch_bounds__(64 * W, 2) void k_partAB(const double *__restrict__
 // critical-temperature search reads (vggsub of dagtm.cxx:1715, still set when
 // the next E-step converges).
 __device__ __forceinline__ void k_sumAB_body(
-    const int bx, const int by, const int bz, const int gx, const double *__restrict__ part,
+    const int bx, const double *__restrict__ part,
     int nch, int M1, int D, double *__restrict__ A0, double *__restrict__ B, int K,
     const double *__restrict__ G, double *__restrict__ Gm) {
     const int NCOL = M1 + D;
@@ -326,7 +319,7 @@ __global__ __launch_bounds__(256) void k_sumAB(const double *__restrict__ part, 
                                                double *__restrict__ B, int K,
                                                const double *__restrict__ G,
                                                double *__restrict__ Gm) {
-    k_sumAB_body(blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, part, nch, M1, D, A0, B, K, G, Gm);
+    k_sumAB_body(blockIdx.x, part, nch, M1, D, A0, B, K, G, Gm);
 }
 
 constexpr int kLdsN = 126;   // largest M+1 whose factor fits in LDS
@@ -752,7 +745,7 @@ __global__ __launch_bounds__(kBcNT) void k_bc_back(const double *__restrict__ S,
 }
 
 // W[:, c0 : c0 + 16] from (A0 + (ridge + jitter) I) W = B for n <= 126, the lower
-// triangle resident in LDS; same pivots and retries as k_chol_solve.  Every
+// triangle resident in LDS; same pivots and retries as k_chol_solve_body.  Every
 // workgroup factors the matrix for itself (they run side by side, and the factor
 // need not go through memory to a second kernel).
 //   Factor: blocked, right-looking.  Wave 0 takes each 8-column panel in registers
@@ -1168,7 +1161,7 @@ __global__ __launch_bounds__(256) void kb_sumAB(const BInst *__restrict__ tab, c
     const int2 m = map[blockIdx.x];
     const BInst &I = tab[m.x];
     if (!I.do_m) return;
-    k_sumAB_body(m.y, 0, 0, 0, I.partAB, I.nchAB, I.M1, I.D, I.A0, I.Bm, I.K, I.G, I.Gm);
+    k_sumAB_body(m.y, I.partAB, I.nchAB, I.M1, I.D, I.A0, I.Bm, I.K, I.G, I.Gm);
 }
 
 __global__ __launch_bounds__(kCholNT) void kb_solve_lds(const BInst *__restrict__ tab,
@@ -1183,7 +1176,7 @@ __global__ __launch_bounds__(1024) void kb_chol_solve(const BInst *__restrict__ 
                                                       const int *__restrict__ list) {
     const BInst &I = tab[list[blockIdx.x]];
     if (!I.do_m) return;
-    k_chol_solve_body(0, 0, 0, 1, I.A0, I.A, I.M1, I.ridge, I.Bm, I.D, I.W, I.scal);
+    k_chol_solve_body(I.A0, I.A, I.M1, I.ridge, I.Bm, I.D, I.W, I.scal);
 }
 
 __global__ __launch_bounds__(256, 2) void kb_centres(const BInst *__restrict__ tab,
