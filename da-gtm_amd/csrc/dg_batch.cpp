@@ -18,7 +18,8 @@
 // graphs never change.  Between the phases the host runs each instance's
 // control (dgc::AnnealMachine) on its scalars.  Every batched kernel computes
 // for an instance exactly what its single-instance launch computes, so each
-// instance's results equal its own dg_anneal run bit for bit.
+// instance's results equal its own dg_anneal run bit for bit (for M + 1 > 126 but
+// for the rounding of the solve, which one workgroup does here).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

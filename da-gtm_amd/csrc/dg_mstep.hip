@@ -1140,7 +1140,8 @@ __global__ __launch_bounds__(256) void k_beta_final(const double *__restrict__ p
 // list the table indices of the instances in this launch, and one grid
 // dimension selects list[slot].  Each instance keeps its own grid extents;
 // workgroups past them return before any barrier.  Every instance computes
-// exactly what its own single-instance launch computes.
+// exactly what its own single-instance launch computes, but for kb_chol_solve
+// (M + 1 > 126), whose chains differ from those of the blocked kernels.
 
 static_assert(CW == kBCentres, "flat-grid tile sizes");
 

@@ -222,8 +222,11 @@ int dg_next_ctemp(dg_ctx *ctx, double temp, double eps, const double *gg,
  * table.  workers = -1 runs the same launches without graph capture.  With
  * workers >= 1 (and in FP64) a pool of host threads takes the items from a
  * shared queue in order of decreasing K*N*D and runs their annealing loops on
- * their own streams.  Results do not depend on the mode, the worker count or
- * the order: each item's result equals its own dg_anneal run bit for bit.
+ * their own streams.  Results do not depend on the worker count or the order:
+ * each item's result equals its own dg_anneal run bit for bit.  The exception
+ * is the batched modes (0 and -1) with M + 1 > 126: they solve for W in one
+ * workgroup per instance, dg_mstep by blocks, so that W differs by the
+ * rounding of the solve (and a run of many steps may converge a step apart).
  * The reference runs one instance per process; this has no counterpart
  * there. */
 typedef struct {
