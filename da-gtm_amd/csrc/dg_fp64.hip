@@ -743,7 +743,7 @@ bool with_db(int db, F &&f) {
 // its column.  The waves' sums are added in order, and the chunk's partial goes
 // to part[((chunk * KB + kb) * 2 + s) * D * D + a * D + b].
 // Bound by the FP64 pipe: 4 flops for each entry, point and centre.  N = 5003,
-// D = 32, K = 400: 158 us with R (4 x 4 tiles of FMAs from LDS and one thread per
+// D = 32, K = 400: 143 us, and 14 for R (4 x 4 tiles of FMAs from LDS and one thread per
 // point for its R: 1107 us).  D = 166: 69 % of the pipe's rate.
 // diag: the pair's columns are its rows, and its upper tiles are not wanted.
 template <int RB, bool diag>
@@ -1215,7 +1215,7 @@ int dg_ctemp_fp64(dg_ctx *c, int k0, int KB, const DgCtempPlan &p, const double 
                            c->stream, part, p.nc, len, S);
         DG_HIP(c, hipGetLastError());
     }
-    // (a wave is enough for 64 rows; 145 KB of LDS at D = 192)
+    // (a wave is enough for 64 rows; 154368 bytes of LDS at D = 192)
     const size_t lds = ((size_t)D * (D + 1) / 2 + 4 * D) * sizeof(double);
     hipLaunchKernelGGL(k_ctemp_eig, dim3((unsigned)KB, 2), dim3(D <= 64 ? 64 : 256), lds, c->stream, S,
                        D, dLimit + 2 * (long)k0, dLimit + 2 * (long)k0 + KB, dVal + 2 * (long)k0);

@@ -44,7 +44,7 @@ struct dg_ctx {
     double *Y64 = nullptr;         // K x ldt
     double *yy = nullptr;          // K      |y_k|^2
     double *W = nullptr;           // M1 x D
-    double *A = nullptr;           // M1 x M1 (lower triangle holds the factor after a solve)
+    double *A = nullptr;           // M1 x M1, M1 > 126 only: scratch of the solve
     double *A0 = nullptr;          // M1 x M1 unfactored copy
     double *Bm = nullptr;          // M1 x D
     double *G = nullptr;           // K

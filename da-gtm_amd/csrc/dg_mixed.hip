@@ -1204,9 +1204,11 @@ __global__ __launch_bounds__(NTH) void k_item_table(const int2 *__restrict__ bra
 // the chain over the chunks is a thread's, so the load latencies of few outputs
 // with many chunks have to spread over the chip.
 // Bound by memory where there are many outputs, by the loads' latency where
-// there are few.  N = 100000, K = 8000, D = 166: 44 -> 19 us; N = 10^6, the same:
-// 166 -> 41; N = 50000, K = 1600, D = 64: 56 -> 14.5; N = 1000, K = 400, D = 12:
-// 11.5 -> 3.7 (16-row workgroups, every chunk read, eight loads in flight).
+// there are few; its time goes with the live chunks.  N = 100000, K = 8000, D = 166:
+// 44 -> 19 us; N = 10^6, the same: 166 -> 43 at a state under way, 156 -> 104 on
+// average (94 to 147) over the first steps of a run; N = 50000, K = 1600, D = 64: 56 -> 14.5;
+// N = 1000, K = 400, D = 12: 11.5 -> 3.7 (16-row workgroups, every chunk read, eight
+// loads in flight).
 constexpr int RK = 64, RD = 4, RU = 16;
 
 __device__ __forceinline__ void k_reduce32_body(

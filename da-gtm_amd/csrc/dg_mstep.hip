@@ -1199,7 +1199,7 @@ __global__ __launch_bounds__(256) void kb_beta_final(const BInst *__restrict__ t
 
 }  // namespace
 
-// dst[r * ld + d] = src[r * D + d] for d < D, 0 for D <= d < ld.
+// dst[r * ld + d] = src[r * lds + d] for d < D, 0 for D <= d < ld.
 __global__ __launch_bounds__(256) void k_pad_rows(const double *__restrict__ src, long rows,
                                                   int D, long lds, int ld,
                                                   double *__restrict__ dst) {

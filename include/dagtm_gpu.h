@@ -250,7 +250,9 @@ int dg_batch_anneal(const dg_config *cfg, int workers, const dg_batch_item *item
 /* MAP projection M = R^T X (N x L, ldM >= L) with the responsibilities at
  * the current model state and the last E-step's temperature (an E-step is
  * run first when an M-step has moved the model since).  Computed in FP64
- * in both precisions.  Replaces dagtm.cxx:2347-2355; unlike the reference
+ * in both precisions; a dg_mstep or dg_get_stats after it (or after dg_next_ctemp
+ * or dg_resp_dense) and before the next dg_estep takes G and R T in FP64 too,
+ * and computes them then.  Replaces dagtm.cxx:2347-2355; unlike the reference
  * after a maxloop exit (which reuses R o dist, Q4), R here is always the
  * responsibility matrix. */
 int dg_map(dg_ctx *ctx, const double *X, int L, long ldX, double *M,
